@@ -1,0 +1,148 @@
+// Host side of the block-scaled MFMA matmul (f32 activations, from batched
+// decode to prefill sizes): activation preparation, the matmul kernel, then
+// (where K is split) the partial-sum reduction.
+#include <hip/hip_runtime_api.h>
+
+#include <algorithm>
+#include <cstdint>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+
+#include "bs_args.h"
+#include "rlxq.h"
+#include "rlxq_internal.hpp"
+
+namespace rlxq {
+
+namespace {
+size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
+// Bytes of one weight row per 256-element unit.
+int64_t bs_seg_bytes(int scheme) {
+  switch (scheme) {
+    case RLXQ_GGUF_Q4_1: return 160;
+    case RLXQ_GGUF_Q4_0: case RLXQ_GGUF_Q4_K: return 144;
+    case RLXQ_GGUF_Q8_0: return 272;
+    case RLXQ_GGUF_Q5_K: return 176;
+    case RLXQ_MLX_AFFINE4: return 128;
+    case RLXQ_MLX_AFFINE8: return 256;
+    default: return 0;
+  }
+}
+}  // namespace
+
+bool bs_scheme(int scheme) {
+  return bs_seg_bytes(scheme) > 0;
+}
+
+int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
+                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, const char* gemm_name) {
+  const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
+  const int64_t nu = (k + 255) / 256;   // 256-element units
+  // 64-row tiles past 32 rows (197 rows of Q4_K, 4096->24576: 131 us in four
+  // of them, 151 in seven 32-row ones; 64 rows of Q4_1: 51 and 55); 128
+  // columns.  RLXQ_BS="RT,splits" (tuning) sets the 32-row tiles per
+  // workgroup (1 or 2) and, unless 0, the K splits.
+  const int64_t r32 = (m + 31) / 32;
+  int RT = gemm_name || m > 32 ? 2 : 1;
+  int64_t want = 0;
+  if (const char* e = std::getenv("RLXQ_BS")) {
+    int a1, a2;
+    if (std::sscanf(e, "%d,%d", &a1, &a2) == 2 && (a1 == 1 || a1 == 2)) RT = gemm_name ? 2 : a1, want = a2;
+  }
+  if (gemm_name)
+    if (const char* e = std::getenv("RLXQ_GEMM_SPLITS")) want = std::max(1, std::atoi(e));
+  const int64_t tiles_m = (m + 32 * RT - 1) / (32 * RT), tiles_n = (n + 127) / 128;
+  const int64_t rtiles = tiles_m * RT;
+  int64_t splits = 1;
+  if (want > 0) splits = std::min<int64_t>(want, nu);
+  else   // K splits until two workgroups per CU are there, of at least two units, at most 24 MiB of partial sums
+    while (tiles_m * tiles_n * splits < 2 * cus && nu / (splits * 2) >= 2 && splits < 32 &&
+           splits * 2 * m * n * 4 <= ((int64_t)24 << 20))
+      splits *= 2;
+  const int64_t uslice = (nu + splits - 1) / splits;
+  splits = (nu + uslice - 1) / uslice;
+  if (tiles_m * tiles_n * splits > 0x7fffffff || rtiles > 0x3ffffff)
+    return fail(ctx, RLXQ_E_SHAPE, "dequant_matmul: block-scaled grid");
+
+  const int nh = 2;
+  const size_t x_bytes = round256((size_t)(16 * nu * rtiles * nh) * 1024), s_bytes = round256((size_t)rtiles * 128);
+  const size_t sum_bytes = round256((size_t)(nu * rtiles) * 1024);
+  const size_t part_bytes = splits > 1 ? round256((size_t)(splits * m * n) * 4) : 0;
+  void* ws = nullptr;
+  int rc;
+  // (what counts against the no-allocation limit: the f16 hi and lo rows)
+  const size_t need = x_bytes + s_bytes + sum_bytes + part_bytes, core = (size_t)(r32 * 32 * k) * 4;
+  if ((rc = workspace(ctx, need, &ws, stream, need > core ? need - core : 0))) return rc;
+  char* wsb = static_cast<char*>(ws);
+
+  rlxq_bs_prep_args p;
+  std::memset(&p, 0, sizeof p);
+  p.x = x;
+  p.x16 = reinterpret_cast<uint8_t*>(wsb);
+  p.inv_s = reinterpret_cast<float*>(wsb + x_bytes);
+  p.ssum = reinterpret_cast<uint32_t*>(wsb + x_bytes + s_bytes);
+  p.M = m;
+  p.K = k;
+  p.rtiles = (int32_t)rtiles;
+  p.nh = nh;
+  p.kb8 = (int32_t)(8 * nu);
+  p.order = scheme == RLXQ_GGUF_Q5_K ? 1 : sk_order(scheme);
+  p.x_bf16 = x_dtype == RLXQ_BF16;
+  p.rdiv = 1;
+  hipFunction_t fn;
+  if ((rc = get_fn(ctx, "rlxq_bs_prep", &fn))) return rc;
+  void* pargs[] = {&p};
+  if ((rc = launch(ctx, fn, dim3((unsigned)(32 * rtiles)), dim3(512), 0, stream, pargs, "rlxq_bs_prep"))) return rc;
+
+  rlxq_bs_args a;
+  std::memset(&a, 0, sizeof a);
+  a.x16 = p.x16;
+  a.inv_s = p.inv_s;
+  a.ssum = p.ssum;
+  a.w = static_cast<const uint8_t*>(w);
+  a.scales = sb.scales;
+  a.biases = sb.biases;
+  a.part = splits > 1 ? reinterpret_cast<float*>(wsb + x_bytes + s_bytes + sum_bytes) : nullptr;
+  a.y = y;
+  a.M = m;
+  a.N = n;
+  a.K = k;
+  a.rb = rb;
+  a.y_ld = n;
+  a.group = sb.group;
+  a.rtiles = (int32_t)rtiles;
+  a.uslice = (int32_t)uslice;
+  a.splits = (int32_t)splits;
+  a.tiles_n = (int32_t)tiles_n;
+  a.tiles_m = (int32_t)tiles_m;
+  a.y_bf16 = y_dtype == RLXQ_BF16;
+  a.sb_bf16 = sb.sb_bf16;
+  char name[64];
+  if (gemm_name) std::snprintf(name, sizeof name, "%s", gemm_name);
+  else std::snprintf(name, sizeof name, "rlxq_skinnyns_%s_bs_rt%d", scheme_name(scheme), RT);
+  if ((rc = get_fn(ctx, name, &fn))) return rc;
+  void* args[] = {&a};
+  // three activation slots (two 32-element blocks each), the waves' weight
+  // regions (rows an odd number of 16-byte pieces apart)
+  const int64_t seg = bs_seg_bytes(scheme), lrow = (seg / 16) % 2 ? seg : seg + 16;
+  const size_t lds = (size_t)(3 * RT * nh) * 4096 + (size_t)(128 * lrow);
+  if ((rc = launch(ctx, fn, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(256), lds, stream, args, name)))
+    return rc;
+  if (splits > 1) {
+    rlxq_skinny_args r;
+    std::memset(&r, 0, sizeof r);
+    r.part = a.part;
+    r.y = y;
+    r.M = m;
+    r.N = n;
+    r.y_ld = n;
+    r.splits = (int32_t)splits;
+    r.y_bf16 = a.y_bf16;
+    rc = splits_reduce(ctx, r, stream);
+    if (!rc) ctx->last_kernel = name;
+  }
+  return rc;
+}
+
+}  // namespace rlxq

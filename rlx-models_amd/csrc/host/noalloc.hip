@@ -25,7 +25,7 @@
 
 namespace {
 
-static __device__ __align__(256) unsigned char scratch[RLXQ_NOALLOC_SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[RLXQ_NOALLOC_SCRATCH_BYTES + rlxq::kNoallocSlack];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;

@@ -244,6 +244,14 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   splits = (k + kslice - 1) / kslice;
   char name[64];
   std::snprintf(name, sizeof name, "rlxq_gemm_%s_t%d%s", scheme_name(scheme), tile, vs.c_str());
+  if (split && bs_scheme(scheme)) {
+    SkinnySb sb;
+    sb.scales = scales;
+    sb.biases = biases;
+    sb.group = is_mlx(scheme) ? group : 32;
+    sb.sb_bf16 = sb_code(sb_dtype);
+    return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, name);
+  }
   hipFunction_t fn;
   int rc;
   if ((rc = get_fn(ctx, name, &fn))) return rc;
@@ -369,6 +377,9 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
       sb.biases = biases;
       sb.group = is_mlx(scheme) ? group : 32;
       sb.sb_bf16 = sb_code(sb_dtype);
+      if (!xbf && m > 16 && bs_scheme(scheme) && !std::getenv("RLXQ_SKINNY_XR") && !std::getenv("RLXQ_SKINNY_NS") &&
+          !std::getenv("RLXQ_SKINNY_XL"))
+        return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, nullptr);
       return skinny_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb);
     }
   }

@@ -47,6 +47,9 @@ RLXQ_EMBED(rlxq_co_moe3, "moe3.co")
 RLXQ_EMBED(rlxq_co_moe4, "moe4.co")
 RLXQ_EMBED(rlxq_co_int8, "int8.co")
 RLXQ_EMBED(rlxq_co_skinny, "skinny.co")
+RLXQ_EMBED(rlxq_co_bsgemm0, "bsgemm0.co")
+RLXQ_EMBED(rlxq_co_bsgemm1, "bsgemm1.co")
+RLXQ_EMBED(rlxq_co_bsgemm2, "bsgemm2.co")
 
 namespace {
 
@@ -72,6 +75,9 @@ const Image kImages[] = {
     {rlxq_co_moe4_begin, rlxq_co_moe4_end, "moe4"},
     {rlxq_co_int8_begin, rlxq_co_int8_end, "int8"},
     {rlxq_co_skinny_begin, rlxq_co_skinny_end, "skinny"},
+    {rlxq_co_bsgemm0_begin, rlxq_co_bsgemm0_end, "bsgemm0"},
+    {rlxq_co_bsgemm1_begin, rlxq_co_bsgemm1_end, "bsgemm1"},
+    {rlxq_co_bsgemm2_begin, rlxq_co_bsgemm2_end, "bsgemm2"},
 };
 
 std::string hip_msg(hipError_t e) { return std::string(hipGetErrorName(e)) + ": " + hipGetErrorString(e); }
@@ -146,9 +152,9 @@ int launch(rlxq_ctx* ctx, hipFunction_t fn, dim3 grid, dim3 block, size_t lds, v
   return RLXQ_OK;
 }
 
-int workspace(rlxq_ctx* ctx, size_t bytes, void** out, void* stream) {
+int workspace(rlxq_ctx* ctx, size_t bytes, void** out, void* stream, size_t slack) {
   if (ctx->fixed_active) {
-    if (bytes > ctx->fixed_bytes)
+    if (bytes > ctx->fixed_bytes + std::min(slack, kNoallocSlack))
       return fail(ctx, RLXQ_E_SCRATCH,
                   "this call needs " + std::to_string(bytes) + " B of scratch; the no-allocation entry point holds " +
                       std::to_string(ctx->fixed_bytes) + " B");

@@ -87,9 +87,17 @@ int blocks_per_cu(rlxq_ctx* ctx, const std::string& name, hipFunction_t fn, int 
 int launch(rlxq_ctx* ctx, hipFunction_t fn, dim3 grid, dim3 block, size_t lds, void* stream,
            void** args, const char* what);
 
+// Bytes the no-allocation array holds past RLXQ_NOALLOC_SCRATCH_BYTES: block
+// sums, padding rows and split-K partial sums of the block-scaled matmul,
+// which do not count against the published limit (24 MiB of partial sums and,
+// at the limit's 64 MiB of activations, at most 3 of block sums and 22 of
+// padding).
+constexpr size_t kNoallocSlack = (size_t)52 << 20;
+
 // Ensures at least `bytes` of context scratch for `stream`; returns its
-// device pointer.
-int workspace(rlxq_ctx* ctx, size_t bytes, void** out, void* stream);
+// device pointer.  `slack` of them do not count against the no-allocation
+// entry point's limit.
+int workspace(rlxq_ctx* ctx, size_t bytes, void** out, void* stream, size_t slack = 0);
 // Frees the stream's retired buffers whose completion event has passed
 // (reclaim), or all of them (free, after the stream has been synchronised).
 void reclaim_retired(rlxq_ctx::Scratch& w);
@@ -148,6 +156,11 @@ int prep_x16(rlxq_ctx* ctx, const void* x, int x_dtype, int64_t m, int64_t k, in
 int sk_post_exp(int scheme);
 int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
                     int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb = SkinnySb());
+// Block-scaled MFMA matmul (f32 activations): its formats, and the call.
+// gemm_name: kernel name for prefill sizes (more than 256 rows), else NULL.
+bool bs_scheme(int scheme);
+int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
+                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, const char* gemm_name);
 int i8b_dispatch(rlxq_ctx* ctx, int group, const void* x, int x_dtype, const void* w, const void* scales,
                  const void* zp, int sb_dtype, int64_t m, int64_t k, int64_t n, void* y, int y_dtype,
                  void* stream);

@@ -1,0 +1,107 @@
+"""The block-scaled MFMA matmul (f32 activations, more than 16 rows) against
+the float64 oracle: edges of its row, column and K tiles, K that is not whole
+256-element units, K splits, and rows of very different size.
+
+Bound per output: the activations' hi + lo split keeps each element to 2^-22,
+and each of the K / 32 block results is rounded a few times in f32 on its way
+into the sum, so |error| <= (2^-21 + (K / 32 + 8) 2^-23) sum_k |x_k| 3 W_k,
+W_k the largest weight of k's block of 32 (scale * code and the min / bias
+are each at most three times that in the synthetic rows)."""
+import numpy as np
+import pytest
+
+from conftest import announce
+
+pytestmark = pytest.mark.gpu
+
+Q8_0, Q4_0, Q4_1, MLX4, MLX8, Q4_K, Q5_K = 1, 2, 3, 4, 5, 7, 10
+NAMES = {Q8_0: "q8_0", Q4_0: "q4_0", Q4_1: "q4_1", MLX4: "mlx4", MLX8: "mlx8", Q4_K: "q4_k", Q5_K: "q5_k"}
+
+
+def _t(a):
+    import torch
+
+    return torch.from_numpy(np.ascontiguousarray(a)).cuda()
+
+
+def _case(orc, scheme, rng, n, k):
+    """(packed, scales, biases, group, dequantized float64 weights)"""
+    if scheme in (MLX4, MLX8):
+        bits, group = (4, 64) if scheme == MLX4 else (8, 32)
+        codes = rng.integers(0, 1 << bits, (n, k)).astype(np.uint32)
+        wq = orc.mlx_pack(codes, bits)
+        sc = rng.uniform(0.01, 0.1, (n, k // group)).astype(np.float32)
+        bi = rng.uniform(-0.5, 0.1, (n, k // group)).astype(np.float32)
+        wd = codes * np.repeat(sc.astype(np.float64), group, 1) + np.repeat(bi.astype(np.float64), group, 1)
+        return _t(wq.view(np.uint8)), _t(sc), _t(bi), group, wd
+    packed = orc.synth(scheme, rng, n, k)
+    return _t(packed), None, None, 32, orc.dequantize(scheme, packed, k).astype(np.float64).reshape(n, k)
+
+
+def _check(ctx, orc, scheme, m, k, n, y_dtype=None):
+    import torch
+
+    rng = np.random.default_rng(m * 7 + k + n * 3 + scheme)
+    w, sc, bi, group, wd = _case(orc, scheme, rng, n, k)
+    x = rng.standard_normal((m, k)).astype(np.float32)
+    x[0] *= 1e-6
+    x[m // 2] *= 3e4
+    x[m - 1, ::3] = 0.0
+    y = ctx.dequant_matmul(_t(x), w, scheme, n, group=group, scales=sc, biases=bi, y_dtype=y_dtype)
+    kern = ctx.last_kernel
+    torch.cuda.synchronize()
+    want = x.astype(np.float64) @ wd.T
+    wmax = np.repeat(np.abs(wd).reshape(n, k // 32, 32).max(2), 32, 1)
+    lim = (2.0 ** -21 + (k / 32 + 8) * 2.0 ** -23) * (np.abs(x).astype(np.float64) @ (3 * wmax).T)
+    got = y.double().cpu().numpy()
+    if y_dtype is not None:
+        lim = lim + np.abs(want) * 2.0 ** -8   # one rounding to bf16
+    assert np.all(np.abs(got - want) <= lim), (kern, float(np.max(np.abs(got - want) / lim)))
+    return kern
+
+
+@pytest.mark.parametrize("scheme", list(NAMES), ids=lambda s: NAMES[s])
+@pytest.mark.parametrize("mkn", [(17, 256, 1), (32, 512, 127), (33, 1792, 129), (64, 1024, 128), (65, 768, 300),
+                                 (200, 2304, 130), (256, 4096, 64)], ids=str)
+def test_batched(ctx, orc, scheme, mkn):
+    announce(f"block-scaled {NAMES[scheme]} {mkn}")
+    kern = _check(ctx, orc, scheme, *mkn)
+    assert kern.startswith(f"rlxq_skinnyns_{NAMES[scheme]}_bs_rt"), kern
+
+
+@pytest.mark.parametrize("scheme,mkn", [(Q4_1, (300, 64 * 13, 301)), (Q4_0, (257, 64 * 5, 130)), (Q8_0, (259, 64 * 7, 33)),
+                                        (MLX4, (258, 64 * 9, 65)), (Q4_1, (18, 384, 5)), (MLX8, (20, 128, 40)),
+                                        (Q4_K, (513, 2560, 385)), (Q5_K, (321, 256, 256))], ids=str)
+@pytest.mark.parametrize("ydt", ["f32", "bf16"])
+def test_partial_units_and_prefill(ctx, orc, scheme, mkn, ydt):
+    import torch
+
+    announce(f"block-scaled {NAMES[scheme]} {mkn} y={ydt}")
+    if ydt == "bf16" and mkn[0] < 64:
+        pytest.skip("bf16 output takes this kernel from 64 rows")
+    _check(ctx, orc, scheme, *mkn, y_dtype=torch.bfloat16 if ydt == "bf16" else None)
+
+
+@pytest.mark.parametrize("cfg", ["1,1", "1,3", "2,1", "2,5", "2,32"])
+def test_row_tiles_and_splits(ctx, orc, monkeypatch, cfg):
+    monkeypatch.setenv("RLXQ_BS", cfg)
+    for scheme, mkn in ((Q4_1, (70, 1792, 200)), (Q4_K, (40, 2816, 129))):
+        announce(f"block-scaled {cfg} {NAMES[scheme]} {mkn}")
+        kern = _check(ctx, orc, scheme, *mkn)
+        assert kern == f"rlxq_skinnyns_{NAMES[scheme]}_bs_rt{cfg[0]}", kern
+
+
+def test_noalloc_is_the_same(ctx, orc):
+    """The no-allocation entry point runs the same kernel on its own array."""
+    import torch
+
+    rng = np.random.default_rng(4)
+    for (m, k, n) in ((64, 4096, 2048), (300, 2048, 1024)):
+        announce(f"block-scaled noalloc {(m, k, n)}")
+        w = _t(orc.synth_q4_1(rng, n, k))
+        x = _t(rng.standard_normal((m, k)).astype(np.float32))
+        want = ctx.dequant_matmul(x, w, Q4_1, n)
+        y = torch.full((m, n), float("nan"), device="cuda")
+        ctx.dequant_matmul_noalloc(x, w, Q4_1, n, y=y)
+        torch.cuda.synchronize()
+        assert torch.equal(y, want)
