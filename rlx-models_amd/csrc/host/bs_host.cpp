@@ -26,6 +26,7 @@ int64_t bs_seg_bytes(int scheme) {
     case RLXQ_GGUF_Q5_K: return 176;
     case RLXQ_MLX_AFFINE4: return 128;
     case RLXQ_MLX_AFFINE8: return 256;
+    case RLXQ_GGUF_Q6_K: return 240;   // (210 bytes from the dword they start in, and padding)
     default: return 0;
   }
 }

@@ -4,26 +4,33 @@
 // types (F32 x and y, crates/rlx-models-core/src/standard_decoder.rs:727-738,
 // 12421-12433).
 //
-// A weight block is scale * (code [* small integer]) + min: the codes are
-// integers that f16 holds exactly, so they go to the matrix cores as they are
-// and the block's scale is applied in f32 to the block's 16 x 16 MFMA result:
-//   T = mfma(x hi, codes, 0); T = mfma(x lo, codes, T); acc += scale * T
-// for each 32-element block, one f32 scale per lane (lane j of a result
-// holds column j).  Against carrying every weight as two f16 operands (hi and
-// lo) that is two MFMAs per block for f32 activations instead of three or
-// four, and no conversion of weights beyond picking the code bits out: an
-// f16 whose bits are the code is the subnormal code * 2^-24, which the matrix
-// cores multiply exactly (2^24 goes into the scale).  The min / bias term is
-// one more MFMA per 512 elements on the rows' prepared block sums.
+// A weight block is scale * code + min: the codes are integers that f16 holds
+// exactly, so they go to the matrix cores as they are and the block's scale
+// is applied in f32 to the block's 32 x 32 MFMA result:
+//   T = sum over the block's two halves of mfma(x hi, codes) + mfma(x lo,
+//   codes); acc += scale * T
+// with one f32 scale per lane (lane j of a result holds column j).  Against
+// carrying every weight as two f16 operands (hi and lo) that is two products
+// per weight for f32 activations instead of three or four, and no conversion
+// of weights beyond picking the code bits out.  (The code bits themselves as
+// subnormal f16, code * 2^-24, would save the offset's addition, but the
+// matrix cores align such products by their exponent field and lose about ten
+// bits of the sum: 3e-6 against 2e-7 off float64.)  The min / bias term is
+// one or two more MFMAs per 256 elements on the rows' prepared block sums.
+// Q6_K has a scale per 16 weights, which is a block's half: code * scale as
+// an f16 and what its rounding left (exact), three products.
 //
-// The weights never pass through LDS: lane (j, g) = (lane % 16, lane / 16)
-// loads block 4c + g of weight row j (a 128-element chunk c of the row per
-// four lanes), and a 4 x 4 transpose over the four 16-lane rows
-// (v_permlane16_swap, v_permlane32_swap: 4 instructions for 4 registers)
-// gives it the codes of positions 8g .. 8g + 7 of all four blocks, which is
-// the MFMA's operand layout with one block per MFMA.  The activation
-// fragments of a chunk are shared by the workgroup's four waves through LDS
-// (double buffered, one barrier per chunk).
+// A wave owns 32 weight rows: their 256-element unit is read as row-contiguous
+// 16-byte pieces one unit ahead and laid into the wave's own LDS region, from
+// where lane (j, h) = (lane % 32, lane / 32) takes the code dwords of
+// positions 8h .. and 16 + 8h .. of row j.  The activation fragments of a
+// step (two blocks) are shared by the workgroup's four waves through LDS.
+//
+// What bounds it: the issue slots beside the MFMAs (per half-block MFMA about
+// four VALU instructions: the scale FMAs and the unpacking) and LDS reads of
+// the activation fragments; 30-35% of the MFMA rate.  Measured with f32 x and
+// y, activation preparation and split-K sums included: Q4_1 4096->24576 at 64
+// rows 90 -> 53 us, at 512 rows 377 -> 260 us; Q4_K at 197 rows 310 -> 131 us.
 #include "common.hip.h"
 #include "bs_args.h"
 #include "f16dq.hip.h"
@@ -39,11 +46,18 @@ typedef float f32x16_t __attribute__((ext_vector_type(16)));
 // that 16 rows' reads at one offset spread over the banks).
 template <int SCH> constexpr int bs_seg() {
   return SCH == SCH_Q4_1 ? 160 : SCH == SCH_Q4_0 ? 144 : SCH == SCH_Q8_0 ? 272 : SCH == SCH_Q4_K ? 144
-         : SCH == SCH_Q5_K ? 176 : SCH == SCH_MLX4 ? 128 : SCH == SCH_MLX8 ? 256 : 0;
+         : SCH == SCH_Q5_K ? 176 : SCH == SCH_MLX4 ? 128 : SCH == SCH_MLX8 ? 256 : SCH == SCH_Q6_K ? 208 : 0;
 }
-template <int SCH> constexpr int bs_lrow() { return (bs_seg<SCH>() / 16) % 2 ? bs_seg<SCH>() : bs_seg<SCH>() + 16; }
+// (Q6_K: 210-byte super-blocks at 2-byte alignment, read from the dword they
+// start in: 13 pieces and a last dword)
+template <int SCH> constexpr int bs_lrow() {
+  if (SCH == SCH_Q6_K) return 240;
+  return (bs_seg<SCH>() / 16) % 2 ? bs_seg<SCH>() : bs_seg<SCH>() + 16;
+}
 template <int SCH> constexpr bool bs_mlx() { return SCH == SCH_MLX4 || SCH == SCH_MLX8; }
 template <int SCH> constexpr bool bs_kq() { return SCH == SCH_Q4_K || SCH == SCH_Q5_K; }
+// Operands per half-block: code, or for Q6_K code * scale as f16 hi and lo.
+template <int SCH> constexpr int bs_nop() { return SCH == SCH_Q6_K ? 2 : 1; }
 template <int SCH> constexpr bool bs_has_m() { return sk_has_m<SCH>(); }
 // Power of two on the f16 min / bias halves (sk_wscale: MLX's f32 biases).
 template <int SCH> constexpr float bs_mscale() { return 1.f / sk_wscale<SCH>(); }
@@ -64,19 +78,28 @@ RLXQ_DEV uint32_t lds_u32(const uint8_t* p) { return *reinterpret_cast<const uin
 template <int SCH>
 struct BsRow {
   uint32_t sa, sb, d;
-  uint32_t qh[4];
+  uint32_t qh[4];   // (Q6_K: the 16 int8 scales)
+  uint32_t off;     // (Q6_K: 0 or 2, the super-block's first byte in the region)
   uint32_t sc[bs_mlx<SCH>() ? 8 : 1];
   uint32_t mn[4];
 };
 // A block as read from LDS: code dwords (raw) and the header dword.
+template <int SCH>
 struct BsRaw {
-  uint32_t c[6], h;
+  uint32_t c[SCH == SCH_Q6_K ? 12 : 6], h;
 };
 
 // Reads the row's unit header (rp: the row in LDS; lane half h).
 template <int SCH>
 RLXQ_DEV void bs_row_head(const uint8_t* rp, int h, BsRow<SCH>& r) {
-  if constexpr (SCH == SCH_Q4_1) {
+  if constexpr (SCH == SCH_Q6_K) {
+    uint32_t w[5];
+#pragma unroll
+    for (int q = 0; q < 5; q++) w[q] = lds_u32(rp + 192 + 4 * q);
+#pragma unroll
+    for (int q = 0; q < 4; q++) r.qh[q] = align_bytes(w[q + 1], w[q], r.off);
+    r.d = __float_as_uint(f16_bits_to_f32((w[4] >> (8 * r.off)) & 0xffffu));
+  } else if constexpr (SCH == SCH_Q4_1) {
 #pragma unroll
     for (int q = 0; q < 4; q++) r.mn[q] = lds_u32(rp + 80 * h + 20 * q) >> 16;
   } else if constexpr (bs_kq<SCH>()) {
@@ -102,7 +125,7 @@ RLXQ_DEV void bs_row_head(const uint8_t* rp, int h, BsRow<SCH>& r) {
 // Block b (0..7, compile time) of the row as raw dwords: those holding the
 // codes of positions 8h .. 8h + 7 and 16 + 8h .. 16 + 8h + 7.
 template <int SCH, int b>
-RLXQ_DEV void bs_fetch(const uint8_t* rp, int h, BsRaw& q) {
+RLXQ_DEV void bs_fetch(const uint8_t* rp, int h, const BsRow<SCH>& r, BsRaw<SCH>& q) {
   if constexpr (SCH == SCH_Q4_1) {
     q.h = lds_u32(rp + 20 * b);
     q.c[0] = lds_u32(rp + 20 * b + 4 + 4 * h);
@@ -133,6 +156,14 @@ RLXQ_DEV void bs_fetch(const uint8_t* rp, int h, BsRaw& q) {
     constexpr int o = (SCH == SCH_Q4_K ? 16 : 48) + 32 * (b / 2);
 #pragma unroll
     for (int i = 0; i < 4; i++) q.c[i] = lds_u32(rp + o + 4 * h + 8 * (i >> 1) + 16 * (i & 1));
+  } else if constexpr (SCH == SCH_Q6_K) {
+    // ql bytes 64 (b / 4) + 32 (b % 2) .., qh bytes 32 (b / 4) .. (three
+    // dwords per eight bytes: the region's bytes lie r.off further)
+#pragma unroll
+    for (int i = 0; i < 6; i++) {
+      q.c[i] = lds_u32(rp + 64 * (b / 4) + 32 * (b & 1) + 8 * h + 16 * (i / 3) + 4 * (i % 3));
+      q.c[6 + i] = lds_u32(rp + 128 + 32 * (b / 4) + 8 * h + 16 * (i / 3) + 4 * (i % 3));
+    }
   } else if constexpr (SCH == SCH_MLX4) {
     q.c[0] = lds_u32(rp + 16 * b + 4 * h);
     q.c[1] = lds_u32(rp + 16 * b + 8 + 4 * h);
@@ -146,7 +177,7 @@ RLXQ_DEV void bs_fetch(const uint8_t* rp, int h, BsRaw& q) {
 // The lane's operand of half m of block b: the codes of positions 16m + 8h ..
 // + 7, exact in f16 (1024 + code by bit pattern, then the offset off).
 template <int SCH, int b, int m>
-RLXQ_DEV f16x8_t bs_operand(const BsRaw& q, const BsRow<SCH>& r) {
+RLXQ_DEV void bs_operand(const BsRaw<SCH>& q, const BsRow<SCH>& r, f16x8_t (&o)[bs_nop<SCH>()]) {
   uint32_t u0, u1;
   if constexpr (SCH == SCH_Q4_1 || SCH == SCH_Q4_0 || SCH == SCH_MLX4) {
     const uint32_t c = (SCH == SCH_Q4_0 && b % 2 == 0) ? align_bytes(q.c[2 * m + 1], q.c[2 * m], 2) : q.c[m];
@@ -162,23 +193,47 @@ RLXQ_DEV f16x8_t bs_operand(const BsRaw& q, const BsRow<SCH>& r) {
   } else if constexpr (SCH == SCH_Q8_0) {
     u0 = (b % 2 == 0 ? align_bytes(q.c[3 * m + 1], q.c[3 * m], 2) : q.c[2 * m]) ^ 0x80808080u;
     u1 = (b % 2 == 0 ? align_bytes(q.c[3 * m + 2], q.c[3 * m + 1], 2) : q.c[2 * m + 1]) ^ 0x80808080u;
+  } else if constexpr (SCH == SCH_Q6_K) {
+    // code (0..63) + 96 per byte, so that code - 32 = byte - 128
+    constexpr int sl = 4 * ((b & 3) >> 1), sh = 2 * (b & 3);
+    const uint32_t l0 = align_bytes(q.c[3 * m + 1], q.c[3 * m], r.off), l1 = align_bytes(q.c[3 * m + 2], q.c[3 * m + 1], r.off);
+    const uint32_t h0 = align_bytes(q.c[3 * m + 7], q.c[3 * m + 6], r.off), h1 = align_bytes(q.c[3 * m + 8], q.c[3 * m + 7], r.off);
+    u0 = (((l0 >> sl) & 0x0F0F0F0Fu) | (((h0 >> sh) & 0x03030303u) << 4)) + 0x60606060u;
+    u1 = (((l1 >> sl) & 0x0F0F0F0Fu) | (((h1 >> sh) & 0x03030303u) << 4)) + 0x60606060u;
   } else {
     u0 = q.c[2 * m];
     u1 = q.c[2 * m + 1];
   }
-  const _Float16 off = SCH == SCH_Q4_0 ? (_Float16)-1032.f : SCH == SCH_Q8_0 ? (_Float16)-1152.f : (_Float16)-1024.f;
+  const _Float16 off = SCH == SCH_Q4_0 ? (_Float16)-1032.f
+                       : (SCH == SCH_Q8_0 || SCH == SCH_Q6_K) ? (_Float16)-1152.f
+                                                               : (_Float16)-1024.f;
   const f16x2_t o2 = {off, off};
-  const f16x2_t w0 = magic_lo(u0) + o2, w1 = magic_hi(u0) + o2, w2 = magic_lo(u1) + o2, w3 = magic_hi(u1) + o2;
-  return f16x8_t{w0.x, w0.y, w1.x, w1.y, w2.x, w2.y, w3.x, w3.y};
+  f16x2_t w[4] = {magic_lo(u0) + o2, magic_hi(u0) + o2, magic_lo(u1) + o2, magic_hi(u1) + o2};
+  if constexpr (SCH == SCH_Q6_K) {
+    // the half's int8 scale 2b + m: code * scale rounded to f16, and the rest
+    // (an integer of at most 13 bits: both exact)
+    const _Float16 sc = (_Float16)(float)(int8_t)((r.qh[b / 2] >> (8 * (2 * (b & 1) + m))) & 0xffu);
+    const f16x2_t s2 = {sc, sc};
+    f16x2_t v[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const f16x2_t p = w[i] * s2;
+      v[i] = __builtin_elementwise_fma(w[i], s2, -p);
+      w[i] = p;
+    }
+    o[bs_nop<SCH>() - 1] = f16x8_t{v[0].x, v[0].y, v[1].x, v[1].y, v[2].x, v[2].y, v[3].x, v[3].y};
+  }
+  o[0] = f16x8_t{w[0].x, w[0].y, w[1].x, w[1].y, w[2].x, w[2].y, w[3].x, w[3].y};
 }
 
 // The block's f32 scale.
 template <int SCH, int b>
-RLXQ_DEV float bs_scale(const BsRaw& q, const BsRow<SCH>& r) {
+RLXQ_DEV float bs_scale(const BsRaw<SCH>& q, const BsRow<SCH>& r) {
   float s;
   if constexpr (SCH == SCH_Q4_1) s = f16_bits_to_f32(q.h & 0xffffu);
   else if constexpr (SCH == SCH_Q4_0 || SCH == SCH_Q8_0) s = f16_bits_to_f32(b % 2 ? q.h >> 16 : q.h & 0xffffu);
   else if constexpr (bs_kq<SCH>()) s = __uint_as_float(r.d) * (float)(((b < 4 ? r.sa : r.sb) >> (8 * (b & 3))) & 0xffu);
+  else if constexpr (SCH == SCH_Q6_K) s = __uint_as_float(r.d);
   else s = __uint_as_float(r.sc[b]);
   // (kept in f32: folded into the FMAs as a mixed-precision operand it would
   // be converted again by each of them)
@@ -214,7 +269,8 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
     xoff[p] = (int)((pc / (64 * XB)) * bstep) + rt0 * NH * 128 + pc % (64 * XB);
   }
   const int s1 = 4 * u1 - 1;   // last step
-  constexpr int XD = 2;   // steps of activations in flight to registers
+  // steps of activations in flight to registers (two spilled for Q6_K and Q8_0)
+  constexpr int XD = SCH == SCH_Q6_K || SCH == SCH_Q8_0 ? 1 : 2;
   u32x4_t xr[XD][NX];
   auto load_x = [&](int s, auto Q) {
     const u32x4_t* xs = xg + 2 * (int64_t)(s < s1 ? s : s1) * bstep;
@@ -237,13 +293,34 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
     src[u] = (uint32_t)(roff(p / PPR) - roff(0)) + (p % PPR) * 16;
     dst[u] = (p / PPR) * LROW + (p % PPR) * 16;
   }
+  const uint32_t tsrc = SCH == SCH_Q6_K ? (uint32_t)(roff(j) - roff(0)) : 0u;
   u32x4_t wr[NL];
+  uint32_t tail = 0u;   // Q6_K: the last dword of row j
   float ms[MLX ? TN : 1][4], mb[MLX ? TN : 1][4];
   const int ufull = (int)(ga.K / 256);   // units wholly inside K
   const int nblk = (int)(ga.K / 32);
   auto load_w = [&](int u) {
     const int uu = u < u1 ? u : u1 - 1;
     const uint8_t* ws = wbase + (int64_t)uu * SEG;
+    if constexpr (SCH == SCH_Q6_K) {
+      static_assert(TN == 1, "a row's last dword per lane");
+      // (K is whole units.)  Row offsets are even: the dword a super-block
+      // starts in lies 0 or 2 bytes before it, and everything read here stays
+      // inside the super-block and those two bytes
+      const uint32_t uo = (uint32_t)((reinterpret_cast<uintptr_t>(wbase) & 3u) + (uint64_t)uu * 210);
+      const uint8_t* w4 = wbase - (reinterpret_cast<uintptr_t>(wbase) & 3u);
+#pragma unroll
+      for (int q = 0; q < NL; q++) {
+        const uint32_t c = dst[q] % LROW;
+        const uint4 v = ld_u128(w4 + ((src[q] - c + uo) & ~3u) + c);
+        wr[q] = u32x4_t{v.x, v.y, v.z, v.w};
+      }
+      const uint32_t so = tsrc + uo, so4 = so & ~3u;
+      const uint16_t* p = reinterpret_cast<const uint16_t*>(w4 + so4 + 208);
+      const uint32_t lo = p[0], hi = p[so & 2u ? 1 : 0];
+      tail = lo | (hi << 16);
+      return;
+    }
     if (uu < ufull) {
 #pragma unroll
       for (int q = 0; q < NL; q++) {
@@ -296,8 +373,10 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
   // stored into the third halfway through step s, so that the barrier at the
   // step's end finds the stores done.
   load_w(u0);
-  static_for<2>([&](auto I) { load_x(4 * u0 + I.value, I); });
-  static_for<2>([&](auto I) { put_x(I.value * SLOT, I); });
+  static_for<2 / XD>([&](auto O) {   // steps 0 and 1, XD at a time
+    static_for<XD>([&](auto I) { load_x(4 * u0 + O.value * XD + I.value, I); });
+    static_for<XD>([&](auto I) { put_x((O.value * XD + I.value) * SLOT, I); });
+  });
   // (step s's register set is (s - 2) % XD)
   static_for<XD>([&](auto I) { load_x(4 * u0 + 2 + I.value, I); });
   barrier();
@@ -319,11 +398,16 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
 
   for (int u = u0; u < u1; u++) {
     // the wave's region is its own: its stores and reads are ordered by the
-    // wave's in-order LDS queue
+    // wave's in-order LDS queue.  (Every lane stores, those past the last
+    // piece that piece again: a conditional store would let the compiler move
+    // the other lanes' reads before it.)
 #pragma unroll
-    for (int q = 0; q < NL; q++)
-      if (lane + 64 * q < NP) *reinterpret_cast<u32x4_t*>(reg + dst[q]) = wr[q];
+    for (int q = 0; q < NL; q++) *reinterpret_cast<u32x4_t*>(reg + dst[q]) = wr[q];
     BsRow<SCH> row[TN];
+    if constexpr (SCH == SCH_Q6_K) {
+      *reinterpret_cast<uint32_t*>(reg + j * LROW + 208) = tail;
+      row[0].off = (uint32_t)((reinterpret_cast<uintptr_t>(wbase) & 3u) + tsrc + (uint32_t)u * 210) & 2u;
+    }
     if constexpr (MLX) {
 #pragma unroll
       for (int t = 0; t < TN; t++)
@@ -333,6 +417,7 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
           row[t].mn[q] = f16_split(mb[t][q] * sk_wscale<SCH>());
         }
     }
+    asm volatile("" ::: "memory");
     load_w(u + 1);
     u32x4_t sf[HM ? RT : 1];
     if constexpr (HM) {
@@ -350,14 +435,14 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
     // 32 x 32 MFMA overlaps with VALU work of the other waves: 23 clocks for
     // one half of it with four FMAs against 30 for a 16 x 16 one with four,
     // two waves per SIMD.)
-    BsRaw raw[2];
-    f16x8_t op[2][2];
+    BsRaw<SCH> raw[2];
+    f16x8_t op[2][2][bs_nop<SCH>()];
     float fs[2];
     f32x16_t T[2];
-    bs_fetch<SCH, 0>(rp[0], h, raw[0]);
-    bs_fetch<SCH, 1 / TN>(rp[1 % TN], h, raw[1]);
-    op[0][0] = bs_operand<SCH, 0, 0>(raw[0], row[0]);
-    op[0][1] = bs_operand<SCH, 0, 1>(raw[0], row[0]);
+    bs_fetch<SCH, 0>(rp[0], h, row[0], raw[0]);
+    bs_fetch<SCH, 1 / TN>(rp[1 % TN], h, row[1 % TN], raw[1]);
+    bs_operand<SCH, 0, 0>(raw[0], row[0], op[0][0]);
+    bs_operand<SCH, 0, 1>(raw[0], row[0], op[0][1]);
     fs[0] = bs_scale<SCH, 0>(raw[0], row[0]);
     static_for<8 * TN * RT>([&](auto S) {
       constexpr int s = S.value, pr = s / RT, rt = s % RT, b = pr / TN, t = pr % TN, q = pr & 1, z = s & 1;
@@ -366,12 +451,16 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
         if constexpr (b % 2 == 0) read_x(std::integral_constant<int, 1>{}, std::integral_constant<int, rt>{}, sc);
         else read_x(std::integral_constant<int, 0>{}, std::integral_constant<int, rt>{}, sn);
       }
-      if constexpr (rt == 0 && pr + 2 < 8 * TN) bs_fetch<SCH, (pr + 2) / TN>(rp[(pr + 2) % TN], h, raw[q]);
+      if constexpr (rt == 0 && pr + 2 < 8 * TN) bs_fetch<SCH, (pr + 2) / TN>(rp[(pr + 2) % TN], h, row[(pr + 2) % TN], raw[q]);
       const f16x8_t(&xf)[2][NH] = xa[b & 1][rt];
-      T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][0], op[q][0], zero, 0, 0, 0);
-      if constexpr (NH == 2) T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][1], op[q][0], T[z], 0, 0, 0);
-      T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][0], op[q][1], T[z], 0, 0, 0);
-      if constexpr (NH == 2) T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][1], op[q][1], T[z], 0, 0, 0);
+      T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][0], op[q][0][0], zero, 0, 0, 0);
+      if constexpr (NH == 2) T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][1], op[q][0][0], T[z], 0, 0, 0);
+      T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][0], op[q][1][0], T[z], 0, 0, 0);
+      if constexpr (NH == 2) T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][1], op[q][1][0], T[z], 0, 0, 0);
+      if constexpr (bs_nop<SCH>() == 2) {   // (the lo x lo products, ~2^-22 of a term, are skipped)
+        T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][0], op[q][0][1], T[z], 0, 0, 0);
+        T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][0], op[q][1][1], T[z], 0, 0, 0);
+      }
       if constexpr (s > 0) {
         constexpr int pp = (s - 1) / RT, rp1 = (s - 1) % RT, tp = pp % TN;
 #pragma unroll
@@ -380,18 +469,18 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
       if constexpr (pr + 1 < 8 * TN) {
         constexpr int nb = (pr + 1) / TN, nt = (pr + 1) % TN;
         if constexpr (RT == 1) {
-          op[q ^ 1][0] = bs_operand<SCH, nb, 0>(raw[q ^ 1], row[nt]);
-          op[q ^ 1][1] = bs_operand<SCH, nb, 1>(raw[q ^ 1], row[nt]);
+          bs_operand<SCH, nb, 0>(raw[q ^ 1], row[nt], op[q ^ 1][0]);
+          bs_operand<SCH, nb, 1>(raw[q ^ 1], row[nt], op[q ^ 1][1]);
           fs[q ^ 1] = bs_scale<SCH, nb>(raw[q ^ 1], row[nt]);
         } else {
-          if constexpr (rt == RT - 2) op[q ^ 1][0] = bs_operand<SCH, nb, 0>(raw[q ^ 1], row[nt]);
+          if constexpr (rt == RT - 2) bs_operand<SCH, nb, 0>(raw[q ^ 1], row[nt], op[q ^ 1][0]);
           if constexpr (rt == RT - 1) {
-            op[q ^ 1][1] = bs_operand<SCH, nb, 1>(raw[q ^ 1], row[nt]);
+            bs_operand<SCH, nb, 1>(raw[q ^ 1], row[nt], op[q ^ 1][1]);
             fs[q ^ 1] = bs_scale<SCH, nb>(raw[q ^ 1], row[nt]);
           }
         }
       }
-      static_for<2 * NH>([&](auto V) {
+      static_for<2 * (NH + bs_nop<SCH>() - 1)>([&](auto V) {
         constexpr int rd = (t == 0 ? 1 : 0) + (rt == 0 ? 2 : 0);
         __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);                             // an MFMA
         if constexpr (rd > 0) __builtin_amdgcn_sched_group_barrier(0x100, rd, 0);    // LDS reads
@@ -674,4 +763,5 @@ RLXQ_BS_SCHEME(q8_0, SCH_Q8_0, rlxq_gemm_q8_0_t256w8xs)
 #if RLXQ_PART_IS(2)
 RLXQ_BS_SCHEME(q4_k, SCH_Q4_K, rlxq_gemm_q4_k_t256w8p2xs)
 RLXQ_BS_SCHEME(q5_k, SCH_Q5_K, rlxq_gemm_q5_k_t256w8xs)
+RLXQ_BS_SCHEME(q6_k, SCH_Q6_K, rlxq_gemm_q6_k_t256w8lxs)
 #endif

@@ -14,8 +14,8 @@ from conftest import announce
 
 pytestmark = pytest.mark.gpu
 
-Q8_0, Q4_0, Q4_1, MLX4, MLX8, Q4_K, Q5_K = 1, 2, 3, 4, 5, 7, 10
-NAMES = {Q8_0: "q8_0", Q4_0: "q4_0", Q4_1: "q4_1", MLX4: "mlx4", MLX8: "mlx8", Q4_K: "q4_k", Q5_K: "q5_k"}
+Q8_0, Q4_0, Q4_1, MLX4, MLX8, Q4_K, Q6_K, Q5_K = 1, 2, 3, 4, 5, 7, 8, 10
+NAMES = {Q8_0: "q8_0", Q4_0: "q4_0", Q4_1: "q4_1", MLX4: "mlx4", MLX8: "mlx8", Q4_K: "q4_k", Q6_K: "q6_k", Q5_K: "q5_k"}
 
 
 def _t(a):
@@ -71,7 +71,8 @@ def test_batched(ctx, orc, scheme, mkn):
 
 @pytest.mark.parametrize("scheme,mkn", [(Q4_1, (300, 64 * 13, 301)), (Q4_0, (257, 64 * 5, 130)), (Q8_0, (259, 64 * 7, 33)),
                                         (MLX4, (258, 64 * 9, 65)), (Q4_1, (18, 384, 5)), (MLX8, (20, 128, 40)),
-                                        (Q4_K, (513, 2560, 385)), (Q5_K, (321, 256, 256))], ids=str)
+                                        (Q4_K, (513, 2560, 385)), (Q5_K, (321, 256, 256)),
+                                        (Q6_K, (300, 1280, 131)), (Q6_K, (65, 256, 3))], ids=str)
 @pytest.mark.parametrize("ydt", ["f32", "bf16"])
 def test_partial_units_and_prefill(ctx, orc, scheme, mkn, ydt):
     import torch
@@ -85,7 +86,7 @@ def test_partial_units_and_prefill(ctx, orc, scheme, mkn, ydt):
 @pytest.mark.parametrize("cfg", ["1,1", "1,3", "2,1", "2,5", "2,32"])
 def test_row_tiles_and_splits(ctx, orc, monkeypatch, cfg):
     monkeypatch.setenv("RLXQ_BS", cfg)
-    for scheme, mkn in ((Q4_1, (70, 1792, 200)), (Q4_K, (40, 2816, 129))):
+    for scheme, mkn in ((Q4_1, (70, 1792, 200)), (Q4_K, (40, 2816, 129)), (Q6_K, (70, 1792, 133))):
         announce(f"block-scaled {cfg} {NAMES[scheme]} {mkn}")
         kern = _check(ctx, orc, scheme, *mkn)
         assert kern == f"rlxq_skinnyns_{NAMES[scheme]}_bs_rt{cfg[0]}", kern
