@@ -26,7 +26,7 @@ int64_t bs_seg_bytes(int scheme) {
     case RLXQ_GGUF_Q5_K: return 176;
     case RLXQ_MLX_AFFINE4: return 128;
     case RLXQ_MLX_AFFINE8: return 256;
-    case RLXQ_GGUF_Q6_K: return 240;   // (210 bytes from the dword they start in, and padding)
+    case RLXQ_GGUF_Q6_K: return 240;   // (210 bytes from the dword they start in)
     default: return 0;
   }
 }
@@ -35,6 +35,14 @@ int64_t bs_seg_bytes(int scheme) {
 bool bs_scheme(int scheme) {
   return bs_seg_bytes(scheme) > 0;
 }
+
+// (rows an odd number of 16-byte pieces apart)
+int64_t bs_lds_row(int scheme) {
+  const int64_t seg = bs_seg_bytes(scheme);
+  return (seg / 16) % 2 ? seg : seg + 16;
+}
+
+int bs_order(int scheme) { return scheme == RLXQ_GGUF_Q5_K ? 1 : sk_order(scheme); }
 
 int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
                 int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, const char* gemm_name) {
@@ -88,7 +96,7 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   p.rtiles = (int32_t)rtiles;
   p.nh = nh;
   p.kb8 = (int32_t)(8 * nu);
-  p.order = scheme == RLXQ_GGUF_Q5_K ? 1 : sk_order(scheme);
+  p.order = bs_order(scheme);
   p.x_bf16 = x_dtype == RLXQ_BF16;
   p.rdiv = 1;
   hipFunction_t fn;
@@ -125,9 +133,8 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   if ((rc = get_fn(ctx, name, &fn))) return rc;
   void* args[] = {&a};
   // three activation slots (two 32-element blocks each), the waves' weight
-  // regions (rows an odd number of 16-byte pieces apart)
-  const int64_t seg = bs_seg_bytes(scheme), lrow = (seg / 16) % 2 ? seg : seg + 16;
-  const size_t lds = (size_t)(3 * RT * nh) * 4096 + (size_t)(128 * lrow);
+  // regions
+  const size_t lds = (size_t)(3 * RT * nh) * 4096 + (size_t)(128 * bs_lds_row(scheme));
   if ((rc = launch(ctx, fn, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(256), lds, stream, args, name)))
     return rc;
   if (splits > 1) {

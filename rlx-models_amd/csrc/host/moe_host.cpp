@@ -11,6 +11,7 @@
 #include <cstring>
 #include <string>
 
+#include "bs_args.h"
 #include "moe_args.h"
 #include "rlxq.h"
 #include "skinny_args.h"
@@ -226,13 +227,20 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
   // gathered rows per chunk (f32 activations: x16 row pairs, so half the
   // entries per 16 MT-row chunk)
   const bool sk_pairs = !xbf;
-  const int64_t rpc = sk_pairs ? 8 * sk_mt : 16 * sk_mt;
+  // f32 activations on the block-scaled kernel (chunks of 32 entries; row
+  // offsets within an expert's slab fit 32 bits): Q6_K's SwiGLU and the
+  // tuning switches keep the row-pair kernels
+  const bool bs = sk && sk_pairs && bs_scheme(scheme) && !(swiglu && !(is_gguf(scheme) || scheme == RLXQ_GGUF_Q4_K ||
+                                                                       scheme == RLXQ_GGUF_Q5_K)) &&
+                  n * rb < ((int64_t)1 << 31) && !std::getenv("RLXQ_MOE_SK") && !std::getenv("RLXQ_MOE_KERNEL");
+  const int64_t rpc = bs ? 32 : sk_pairs ? 8 * sk_mt : 16 * sk_mt;
   const int64_t sk_mp = sk ? ((n_entries + fired_est * (rpc - 1) + rpc - 1) / rpc) * rpc : 0;   // gathered rows
   const int64_t sk_xr = sk_pairs ? 2 * sk_mp : sk_mp;                                            // x16 rows
   auto r256 = [](size_t b) { return (b + 255) & ~size_t(255); };
   const size_t cmap_bytes = sk ? r256((size_t)(1 + sk_mp / rpc) * 4) : 0, emap_bytes = sk ? r256((size_t)sk_mp * 4) : 0;
-  const size_t x16_bytes = sk ? r256((size_t)sk_xr * k * 2) : 0, is_bytes = sk ? r256((size_t)sk_xr * 4) : 0;
-  const size_t sum_bytes = sk ? r256((size_t)sk_xr * (k / 32) * 4) : 0;   // block sums of the x16 rows
+  const int64_t bs_nu = (k + 255) / 256;   // (block-scaled: whole 256-element units)
+  const size_t x16_bytes = sk ? r256((size_t)sk_xr * (bs ? bs_nu * 256 : k) * 2) : 0, is_bytes = sk ? r256((size_t)sk_xr * 4) : 0;
+  const size_t sum_bytes = sk ? r256((size_t)sk_xr * (bs ? bs_nu * 8 : k / 32) * 4) : 0;   // block sums of the x16 rows
   const size_t total_ws = table_bytes + tmp_bytes + cmap_bytes + emap_bytes + x16_bytes + is_bytes + sum_bytes;
   void* ws = nullptr;
   if (total_ws && (rc = workspace(ctx, total_ws, &ws, stream))) return rc;
@@ -271,6 +279,56 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
     if ((rc = get_fn(ctx, "rlxq_moe_pad_k", &fp))) return rc;
     void* pargs[] = {&pa};
     if ((rc = launch(ctx, fp, dim3(1), dim3(1024), 0, stream, pargs, "rlxq_moe_pad_k"))) return rc;
+    if (bs) {
+      // 2b, 2c. the gathered rows as f16 fragments, then the block-scaled
+      // kernel over (chunk, 128 columns)
+      rlxq_bs_prep_args bp;
+      std::memset(&bp, 0, sizeof bp);
+      bp.x = x;
+      bp.x16 = reinterpret_cast<uint8_t*>(skb + cmap_bytes + emap_bytes);
+      bp.inv_s = reinterpret_cast<float*>(skb + cmap_bytes + emap_bytes + x16_bytes);
+      bp.ssum = reinterpret_cast<uint32_t*>(skb + cmap_bytes + emap_bytes + x16_bytes + is_bytes);
+      bp.rmap = pa.emap;
+      bp.cmap = pa.cmap;
+      bp.K = k;
+      bp.rtiles = (int32_t)(sk_mp / 32);
+      bp.nh = 2;
+      bp.kb8 = (int32_t)(bs_nu * 8);
+      bp.order = bs_order(scheme);
+      bp.rdiv = x_div;
+      hipFunction_t fb;
+      if ((rc = get_fn(ctx, "rlxq_bs_prep", &fb))) return rc;
+      void* bargs[] = {&bp};
+      if ((rc = launch(ctx, fb, dim3((unsigned)sk_mp), dim3(512), 0, stream, bargs, "rlxq_bs_prep"))) return rc;
+      rlxq_moe_sk_args ka;
+      std::memset(&ka, 0, sizeof ka);
+      ka.x16 = reinterpret_cast<const uint16_t*>(bp.x16);
+      ka.inv_s = bp.inv_s;
+      ka.ssum = reinterpret_cast<const float*>(bp.ssum);
+      ka.cmap = pa.cmap;
+      ka.emap = pa.emap;
+      ka.bank = static_cast<const uint8_t*>(bank);
+      ka.y = combine ? static_cast<void*>(tmp) : y;
+      ka.N = n;
+      ka.K = k;
+      ka.rb = rb;
+      ka.y_ld = width;
+      ka.Mp = sk_mp;
+      ka.tiles_n = (int32_t)((width + 127) / 128);
+      ka.y_bf16 = (!combine && y_dtype == RLXQ_BF16) ? 1 : 0;
+      ka.scales = scales;
+      ka.biases = biases;
+      ka.group = is_mlx(scheme) ? group : 32;
+      ka.sb_bf16 = sb_code(sb_dtype);
+      std::snprintf(name, sizeof name, "rlxq_moesk_%s_bs%s", scheme_name(scheme), swiglu ? "_sw" : "");
+      if ((rc = get_fn(ctx, name, &fb))) return rc;
+      // (whole eights: the kernel deals the workgroups in use over the XCDs)
+      const int64_t grid = (sk_mp / 32 * ka.tiles_n + 7) / 8 * 8;
+      if (grid > 0x7fffffff) return fail(ctx, RLXQ_E_SHAPE, std::string(what) + ": grid too large");
+      const size_t lds = (size_t)3 * 2 * 4096 + (size_t)((swiglu ? 256 : 128) * bs_lds_row(scheme));
+      void* kargs[] = {&ka};
+      if ((rc = launch(ctx, fb, dim3((unsigned)grid), dim3(256), lds, stream, kargs, name))) return rc;
+    } else {
     // 2b. the gathered rows to f16 (scaled per row, code-unpacking order)
     rlxq_x16_args xa;
     std::memset(&xa, 0, sizeof xa);
@@ -337,6 +395,7 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
     const size_t lds = 2 * (size_t)(sk_mt * NT * 4) * 64 * 4;
     void* kargs[] = {&ka};
     if ((rc = launch(ctx, fk, dim3((unsigned)grid), dim3(256), lds, stream, kargs, name))) return rc;
+    }
   } else {
   // 2. grouped GEMV over (expert or chunk, tile)
   hipFunction_t fg;

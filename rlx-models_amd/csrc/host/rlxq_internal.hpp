@@ -159,6 +159,8 @@ int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const
 // Block-scaled MFMA matmul (f32 activations): its formats, and the call.
 // gemm_name: kernel name for prefill sizes (more than 256 rows), else NULL.
 bool bs_scheme(int scheme);
+int64_t bs_lds_row(int scheme);   // bytes of a weight row's unit in LDS
+int bs_order(int scheme);         // code order of its prepared activations
 int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
                 int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, const char* gemm_name);
 int i8b_dispatch(rlxq_ctx* ctx, int group, const void* x, int x_dtype, const void* w, const void* scales,

@@ -20,8 +20,9 @@ typedef struct rlxq_bs_prep_args {
   uint8_t* x16;
   float* inv_s;           /* [32 rtiles]                                   */
   uint32_t* ssum;         /* [kb8 / 8][rtiles][64][4] or NULL             */
-  const int32_t* rmap;    /* row r is x row rmap[r] / rdiv, zero where
-                             rmap[r] < 0; NULL: x row r                    */
+  const int32_t* rmap;    /* row r is x row rmap[r] / rdiv, unused where
+                             rmap[r] < 0; NULL: x row r                  */
+  const int32_t* cmap;    /* with rmap: cmap[0] 32-row tiles are in use  */
   int64_t M, K;
   int32_t rtiles, nh, kb8, order, x_bf16, rdiv;
 } rlxq_bs_prep_args;

@@ -614,6 +614,76 @@ RLXQ_DEV void bs_body(const rlxq_bs_args& a) {
   }
 }
 
+// Grouped (MoE) form for prefill-sized calls: a workgroup takes one chunk of 32
+// gathered rows, all of one expert, and 128 weight rows of that expert's slab
+// (SwiGLU: 128 gate rows and the matching up rows N / 2 further on, a wave's
+// second column tile, and the epilogue writes silu(g) * u).  Output rows go to
+// the rows' entries.  Replaces the backend kernel of Op::DequantGroupedMatMul
+// and the MoE expert FFN (crates/rlx-models-core/src/standard_decoder.rs:
+// 12634-12760) at prefill sizes with F32 activations.  Against 16-row MFMA
+// tiles on hi / lo row pairs (8 entries per weight pass, four products) it is
+// one weight pass per 32 entries and two products: a 256-token layer of Q4_K
+// experts (2048 -> 1536 and 768 -> 2048, 16 entries per expert), gate|up 242
+// -> 95 us, down 150 -> 60 us.
+struct BsMoeRows {
+  int64_t n0, width, rb, kg, e0;   // e0: the expert's first row of the bank
+  RLXQ_DEV int64_t row(int r) const {
+    const int64_t c = n0 + (r & 31) < width ? n0 + (r & 31) : width - 1;
+    return r < 32 ? c : width + c;
+  }
+  RLXQ_DEV int64_t operator()(int r) const { return row(r) * rb; }
+  RLXQ_DEV int64_t slab(int r) const { return (e0 + row(r)) * kg; }
+};
+
+template <int SCH, bool SW>
+RLXQ_DEV void bs_moe_body(const rlxq_moe_sk_args& a) {
+  constexpr int TN = SW ? 2 : 1;
+  extern __shared__ __align__(16) uint8_t bs_lds[];
+  // The grid is sized for the most chunks there can be: the chunks there are
+  // go to the XCDs in contiguous ranges (workgroups b, b + 8, ... share one),
+  // so that a chunk's activations stay in one L2.
+  const int total = a.cmap[0] * a.tiles_n, per = (total + 7) / 8;
+  const int L = (int)(blockIdx.x % 8) * per + (int)(blockIdx.x / 8);
+  if ((int)(blockIdx.x / 8) >= per || L >= total) return;
+  const int chunk = L / a.tiles_n, tn = L % a.tiles_n;
+  const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int j = lane & 31, h = lane >> 5;
+  const int e = a.cmap[1 + chunk];
+  const int64_t width = SW ? a.N / 2 : a.N;
+  const int64_t n0 = (int64_t)tn * 128 + wv * 32;
+  rlxq_gemm_args ga;
+  ga.w = a.bank + (int64_t)e * a.N * a.rb;
+  ga.rb = a.rb;
+  ga.K = a.K;
+  ga.group = a.group;
+  ga.sb_bf16 = a.sb_bf16;
+  ga.scales = a.scales;
+  ga.biases = a.biases;
+  const BsMoeRows roff{n0, width, a.rb, bs_mlx<SCH>() ? a.K / a.group : 0, (int64_t)e * a.N};
+  f32x16_t acc[1][TN];
+  bs_core<SCH, 1, TN, 2>(ga, roff, reinterpret_cast<const uint8_t*>(a.x16), reinterpret_cast<const uint32_t*>(a.ssum),
+                         (int)(a.Mp / 32), chunk, 0, (int)((a.K + 255) / 256), acc, bs_lds);
+  typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
+  const int64_t m0 = (int64_t)chunk * 32 + 4 * h, c = n0 + j;
+  i32x4_t ent[4];
+  f32x4_t is[4];
+#pragma unroll
+  for (int q = 0; q < 4; q++) {
+    ent[q] = *reinterpret_cast<const i32x4_t*>(a.emap + m0 + 8 * q);
+    is[q] = *reinterpret_cast<const f32x4_t*>(a.inv_s + m0 + 8 * q);
+  }
+  if (c >= width) return;
+#pragma unroll
+  for (int r = 0; r < 16; r++) {
+    if (ent[r / 4][r % 4] < 0) continue;
+    float o = acc[0][0][r] * is[r / 4][r % 4];
+    if constexpr (SW) o = o / (1.f + expf(-o)) * (acc[0][TN - 1][r] * is[r / 4][r % 4]);
+    const int64_t off = (int64_t)ent[r / 4][r % 4] * a.y_ld + c;
+    if (a.y_bf16) reinterpret_cast<uint16_t*>(a.y)[off] = (uint16_t)f32_to_bf16_bits(o);
+    else reinterpret_cast<float*>(a.y)[off] = o;
+  }
+}
+
 // Activation preparation: a workgroup of 512 threads per x16 row, thread t
 // on pieces t, t + 512, ... (piece = 8 positions of a block), the first NP of
 // them kept in registers between the row maximum and the conversion.
@@ -627,9 +697,12 @@ RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
   int64_t src = r;
   bool live = r < a.M;
   if (a.rmap) {
-    const int32_t ent = a.rmap[r];
-    live = ent >= 0;
-    src = (live ? ent : 0) / a.rdiv;
+    // (a padding row's fragments are left as they are: they reach only its own
+    // output row, which is not stored)
+    const int32_t ent = r < a.cmap[0] * 32 ? a.rmap[r] : -1;
+    if (ent < 0) return;
+    live = true;
+    src = ent / a.rdiv;
   }
   auto load = [&](int p, float* v) {
     const int b = p >> 2;
@@ -750,18 +823,30 @@ extern "C" __global__ __launch_bounds__(512) void rlxq_bs_prep(rlxq_bs_prep_args
 #define RLXQ_BS_SCHEME(SNAME, SCH, GEMM)                                                       \
   RLXQ_BS_INST(rlxq_skinnyns_##SNAME##_bs_rt1, SCH, 1)                                          \
   RLXQ_BS_INST(rlxq_skinnyns_##SNAME##_bs_rt2, SCH, 2)                                          \
-  RLXQ_BS_INST(GEMM, SCH, 2)
+  RLXQ_BS_INST(GEMM, SCH, 2)                                                                   \
+  extern "C" __global__ __launch_bounds__(256, 2) void rlxq_moesk_##SNAME##_bs(rlxq_moe_sk_args a) { \
+    rlxq::bs_moe_body<SCH, false>(a);                                                          \
+  }
+#define RLXQ_BS_SW(SNAME, SCH)                                                                 \
+  extern "C" __global__ __launch_bounds__(256, 2) void rlxq_moesk_##SNAME##_bs_sw(rlxq_moe_sk_args a) { \
+    rlxq::bs_moe_body<SCH, true>(a);                                                           \
+  }
 #if RLXQ_PART_IS(0)
 RLXQ_BS_SCHEME(q4_1, SCH_Q4_1, rlxq_gemm_q4_1_t256w8p2xs)
+RLXQ_BS_SW(q4_1, SCH_Q4_1)
 RLXQ_BS_SCHEME(mlx4, SCH_MLX4, rlxq_gemm_mlx4_t256w8xs)
 RLXQ_BS_SCHEME(mlx8, SCH_MLX8, rlxq_gemm_mlx8_t256w8p2xs)
 #endif
 #if RLXQ_PART_IS(1)
 RLXQ_BS_SCHEME(q4_0, SCH_Q4_0, rlxq_gemm_q4_0_t256w8p2xs)
+RLXQ_BS_SW(q4_0, SCH_Q4_0)
+RLXQ_BS_SW(q8_0, SCH_Q8_0)
 RLXQ_BS_SCHEME(q8_0, SCH_Q8_0, rlxq_gemm_q8_0_t256w8xs)
 #endif
 #if RLXQ_PART_IS(2)
 RLXQ_BS_SCHEME(q4_k, SCH_Q4_K, rlxq_gemm_q4_k_t256w8p2xs)
+RLXQ_BS_SW(q4_k, SCH_Q4_K)
+RLXQ_BS_SW(q5_k, SCH_Q5_K)
 RLXQ_BS_SCHEME(q5_k, SCH_Q5_K, rlxq_gemm_q5_k_t256w8xs)
 RLXQ_BS_SCHEME(q6_k, SCH_Q6_K, rlxq_gemm_q6_k_t256w8lxs)
 #endif
