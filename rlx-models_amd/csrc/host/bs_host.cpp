@@ -44,6 +44,20 @@ int64_t bs_lds_row(int scheme) {
 
 int bs_order(int scheme) { return scheme == RLXQ_GGUF_Q5_K ? 1 : sk_order(scheme); }
 
+// Eight rows per workgroup once those fill the chip (2048 gathered rows of
+// 2048: 12.8 us, against 18 with a row per workgroup), two below (512 rows of
+// 4096 took 12.9 us eight a workgroup, 9.6 one).
+int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream) {
+  const int64_t rows = (int64_t)32 * p.rtiles;
+  const int per = rows >= 2048 ? 8 : 2;
+  const char* name = per == 8 ? "rlxq_bs_prep8" : "rlxq_bs_prep2";
+  hipFunction_t fn;
+  if (int rc = get_fn(ctx, name, &fn)) return rc;
+  rlxq_bs_prep_args a = p;
+  void* args[] = {&a};
+  return launch(ctx, fn, dim3((unsigned)(rows / per)), dim3(1024), 0, stream, args, name);
+}
+
 int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
                 int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, const char* gemm_name) {
   const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
@@ -64,11 +78,25 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   const int64_t tiles_m = (m + 32 * RT - 1) / (32 * RT), tiles_n = (n + 127) / 128;
   const int64_t rtiles = tiles_m * RT;
   int64_t splits = 1;
-  if (want > 0) splits = std::min<int64_t>(want, nu);
-  else   // K splits until two workgroups per CU are there, of at least two units, at most 24 MiB of partial sums
-    while (tiles_m * tiles_n * splits < 2 * cus && nu / (splits * 2) >= 2 && splits < 32 &&
-           splits * 2 * m * n * 4 <= ((int64_t)24 << 20))
-      splits *= 2;
+  if (want > 0) {
+    splits = std::min<int64_t>(want, nu);
+  } else {
+    // K splits by what the rounds of workgroups cost: a 64-row unit takes
+    // about 2.65 us per workgroup and CU (3.1 alone on the CU; 32-row ones
+    // 1.6 and 1.9), the reduction 3.5 us and the partial sums' traffic at
+    // about 5 TB/s.  At most 24 MiB of partial sums.  (64 rows of Q4_1:
+    // 4096->24576 four splits 51 us, none 56; 4096->4096 eight 21 us, four 23,
+    // sixteen 25.)
+    double best = 1e30;
+    for (int64_t t = 1; t <= 32 && t <= nu; t++) {
+      const int64_t us = (nu + t - 1) / t, sp = (nu + us - 1) / us;
+      if (sp != t || (t > 1 && t * m * n * 4 > ((int64_t)24 << 20))) continue;
+      const int64_t per_cu = (tiles_m * tiles_n * t + cus - 1) / cus;
+      const double unit = RT == 2 ? (per_cu > 1 ? 2.65 : 3.1) : (per_cu > 1 ? 1.6 : 1.9);
+      const double cost = (double)(per_cu * us) * unit + (t > 1 ? 3.5 + (double)(t * m * n) * 8 / 5e6 : 0.0);
+      if (cost < best) best = cost, splits = t;
+    }
+  }
   const int64_t uslice = (nu + splits - 1) / splits;
   splits = (nu + uslice - 1) / uslice;
   if (tiles_m * tiles_n * splits > 0x7fffffff || rtiles > 0x3ffffff)
@@ -99,10 +127,8 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   p.order = bs_order(scheme);
   p.x_bf16 = x_dtype == RLXQ_BF16;
   p.rdiv = 1;
+  if ((rc = bs_prep(ctx, p, stream))) return rc;
   hipFunction_t fn;
-  if ((rc = get_fn(ctx, "rlxq_bs_prep", &fn))) return rc;
-  void* pargs[] = {&p};
-  if ((rc = launch(ctx, fn, dim3((unsigned)(32 * rtiles)), dim3(512), 0, stream, pargs, "rlxq_bs_prep"))) return rc;
 
   rlxq_bs_args a;
   std::memset(&a, 0, sizeof a);

@@ -248,37 +248,35 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
   float* tmp = combine ? reinterpret_cast<float*>(static_cast<char*>(ws) + table_bytes) : nullptr;
   char* skb = static_cast<char*>(ws) + table_bytes + tmp_bytes;
 
-  // 1. routing table
-  if (!fused) {
+  // 1. routing: the gathered-row layout (MFMA kernels) or the routing table
+  rlxq_moe_layout_args pa;
+  std::memset(&pa, 0, sizeof pa);
+  pa.t.ids = ids;
+  pa.t.idx_f32 = idx;
+  pa.t.table = table;
+  pa.t.zero_rows = combine ? static_cast<void*>(tmp) : y;
+  pa.t.n = n_entries;
+  pa.t.N = width;
+  pa.t.zero_ld = width;
+  pa.t.E = (int32_t)num_experts;
+  pa.t.zero_bf16 = (!combine && y_dtype == RLXQ_BF16) ? 1 : 0;
+  if (!fused && !sk) {
     hipFunction_t ft;
     if ((rc = get_fn(ctx, "rlxq_moe_table_k", &ft))) return rc;
-    rlxq_moe_table_args ta;
-    ta.ids = ids;
-    ta.idx_f32 = idx;
-    ta.table = table;
-    ta.zero_rows = combine ? static_cast<void*>(tmp) : y;
-    ta.n = n_entries;
-    ta.N = width;
-    ta.zero_ld = width;
-    ta.E = (int32_t)num_experts;
-    ta.zero_bf16 = (!combine && y_dtype == RLXQ_BF16) ? 1 : 0;
-    void* targs[] = {&ta};
+    void* targs[] = {&pa.t};
     if ((rc = launch(ctx, ft, dim3(1), dim3(1024), 0, stream, targs, "rlxq_moe_table_k"))) return rc;
   }
 
   if (sk) {
-    // 2a. gathered-row layout of the table's entries
-    rlxq_moe_pad_args pa;
-    pa.table = table;
+    // 2a. gathered-row layout of the entries
     pa.cmap = reinterpret_cast<int32_t*>(skb);
     pa.emap = reinterpret_cast<int32_t*>(skb + cmap_bytes);
     pa.Mp = sk_mp;
-    pa.E = (int32_t)num_experts;
     pa.rows_per_chunk = (int32_t)rpc;
     hipFunction_t fp;
-    if ((rc = get_fn(ctx, "rlxq_moe_pad_k", &fp))) return rc;
+    if ((rc = get_fn(ctx, "rlxq_moe_layout_k", &fp))) return rc;
     void* pargs[] = {&pa};
-    if ((rc = launch(ctx, fp, dim3(1), dim3(1024), 0, stream, pargs, "rlxq_moe_pad_k"))) return rc;
+    if ((rc = launch(ctx, fp, dim3(1), dim3(1024), 0, stream, pargs, "rlxq_moe_layout_k"))) return rc;
     if (bs) {
       // 2b, 2c. the gathered rows as f16 fragments, then the block-scaled
       // kernel over (chunk, 128 columns)
@@ -297,9 +295,7 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
       bp.order = bs_order(scheme);
       bp.rdiv = x_div;
       hipFunction_t fb;
-      if ((rc = get_fn(ctx, "rlxq_bs_prep", &fb))) return rc;
-      void* bargs[] = {&bp};
-      if ((rc = launch(ctx, fb, dim3((unsigned)sk_mp), dim3(512), 0, stream, bargs, "rlxq_bs_prep"))) return rc;
+      if ((rc = bs_prep(ctx, bp, stream))) return rc;
       rlxq_moe_sk_args ka;
       std::memset(&ka, 0, sizeof ka);
       ka.x16 = reinterpret_cast<const uint16_t*>(bp.x16);

@@ -54,6 +54,7 @@ struct rlxq_ctx {
   std::string fixed_msg = "not set up";
 };
 
+#include "bs_args.h"
 #include "skinny_args.h"
 
 namespace rlxq {
@@ -159,6 +160,7 @@ int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const
 // Block-scaled MFMA matmul (f32 activations): its formats, and the call.
 // gemm_name: kernel name for prefill sizes (more than 256 rows), else NULL.
 bool bs_scheme(int scheme);
+int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream);
 int64_t bs_lds_row(int scheme);   // bytes of a weight row's unit in LDS
 int bs_order(int scheme);         // code order of its prepared activations
 int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,

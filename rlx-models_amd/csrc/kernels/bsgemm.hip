@@ -624,7 +624,7 @@ RLXQ_DEV void bs_body(const rlxq_bs_args& a) {
 // tiles on hi / lo row pairs (8 entries per weight pass, four products) it is
 // one weight pass per 32 entries and two products: a 256-token layer of Q4_K
 // experts (2048 -> 1536 and 768 -> 2048, 16 entries per expert), gate|up 242
-// -> 95 us, down 150 -> 60 us.
+// -> 91 us, down 150 -> 57 us.
 struct BsMoeRows {
   int64_t n0, width, rb, kg, e0;   // e0: the expert's first row of the bank
   RLXQ_DEV int64_t row(int r) const {
@@ -684,25 +684,31 @@ RLXQ_DEV void bs_moe_body(const rlxq_moe_sk_args& a) {
   }
 }
 
-// Activation preparation: a workgroup of 512 threads per x16 row, thread t
-// on pieces t, t + 512, ... (piece = 8 positions of a block), the first NP of
-// them kept in registers between the row maximum and the conversion.
-template <int ORD>
+// Activation preparation: a workgroup of 1024 threads for ROWS rows, 1024 /
+// ROWS threads a row: thread t of a row on pieces t, t + PT, ... (piece = 8
+// positions of a block), the first NP of them kept in registers between the
+// row maximum and the conversion.  Eight rows fill whole 128-byte lines of
+// the fragments (a line holds one piece of eight rows), which the L2 then
+// writes back once; with a row per workgroup the lines' parts came from
+// several XCDs: 2048 gathered rows of 2048 took 18 us.  Two rows a workgroup
+// where rows are few and the work has to spread over the CUs.
+template <int ORD, int ROWS>
 RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
-  constexpr int NP = 4;
-  __shared__ float red[8];
-  const int r = blockIdx.x, t = threadIdx.x, lane = t & 63;
-  const int i = t & 3;   // the thread's piece of its blocks (512 is a multiple of 4)
+  constexpr int PT = 1024 / ROWS, NP = ROWS == 8 ? 4 : 3, NW = PT / 64;
+  __shared__ float red[16];
+  const int t = threadIdx.x % PT, rw = __builtin_amdgcn_readfirstlane(threadIdx.x / PT), lane = threadIdx.x & 63;
+  const int r = blockIdx.x * ROWS + rw;
+  const int i = t & 3;   // the thread's piece of its blocks (PT is a multiple of 4)
   const int nblk = (int)(a.K / 32), np = a.kb8 * 4;
   int64_t src = r;
   bool live = r < a.M;
   if (a.rmap) {
-    // (a padding row's fragments are left as they are: they reach only its own
-    // output row, which is not stored)
-    const int32_t ent = r < a.cmap[0] * 32 ? a.rmap[r] : -1;
-    if (ent < 0) return;
-    live = true;
-    src = ent / a.rdiv;
+    // (a gathered padding row's fragments are left as they are: they reach only
+    // its own output row, which is not stored)
+    if ((int)(blockIdx.x * ROWS) >= a.cmap[0] * 32) return;
+    const int32_t ent = a.rmap[r];
+    live = ent >= 0;
+    src = (live ? ent : 0) / a.rdiv;
   }
   auto load = [&](int p, float* v) {
     const int b = p >> 2;
@@ -738,12 +744,12 @@ RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
   if (live) {
 #pragma unroll
     for (int q = 0; q < NP; q++)
-      if (t + 512 * q < np) {
-        load(t + 512 * q, v[q]);
+      if (t + PT * q < np) {
+        load(t + PT * q, v[q]);
 #pragma unroll
         for (int e = 0; e < 8; e++) amax = fmaxf(amax, fabsf(v[q][e]));
       }
-    for (int p = t + 512 * NP; p < np; p += 512) {
+    for (int p = t + PT * NP; p < np; p += PT) {
       float u[8];
       load(p, u);
 #pragma unroll
@@ -751,10 +757,12 @@ RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
     }
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, 64));
-    if (lane == 0) red[t >> 6] = amax;
-    __syncthreads();
+    if (lane == 0) red[threadIdx.x >> 6] = amax;
+  }
+  __syncthreads();
+  if (live) {
 #pragma unroll
-    for (int w = 0; w < 8; w++) amax = fmaxf(amax, red[w]);
+    for (int w = 0; w < NW; w++) amax = fmaxf(amax, red[rw * NW + w]);
     // the power of two that puts the row maximum in [2^9, 2^10): a block sum
     // then stays below 2^15, inside f16
     inv = 1.f;
@@ -765,6 +773,7 @@ RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
       inv = ldexpf(1.f, -sh);
     }
   }
+  if (a.rmap && !live) return;
   if (t == 0) a.inv_s[r] = inv;
   const int rt = r >> 5, j = r & 31;
   auto put = [&](int p, const float* u) {
@@ -796,8 +805,8 @@ RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
   };
 #pragma unroll
   for (int q = 0; q < NP; q++)
-    if (t + 512 * q < np) put(t + 512 * q, v[q]);
-  for (int p = t + 512 * NP; p < np; p += 512) {
+    if (t + PT * q < np) put(t + PT * q, v[q]);
+  for (int p = t + PT * NP; p < np; p += PT) {
     float u[8];
     if (live) load(p, u);
     put(p, u);
@@ -807,11 +816,14 @@ RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
 }  // namespace rlxq
 
 #if RLXQ_PART_IS(0)
-extern "C" __global__ __launch_bounds__(512) void rlxq_bs_prep(rlxq_bs_prep_args a) {
-  if (a.order == 1) rlxq::bs_prep_body<1>(a);
-  else if (a.order == 2) rlxq::bs_prep_body<2>(a);
-  else rlxq::bs_prep_body<0>(a);
-}
+#define RLXQ_BS_PREP(NAME, ROWS)                                                               \
+  extern "C" __global__ __launch_bounds__(1024) void NAME(rlxq_bs_prep_args a) {               \
+    if (a.order == 1) rlxq::bs_prep_body<1, ROWS>(a);                                          \
+    else if (a.order == 2) rlxq::bs_prep_body<2, ROWS>(a);                                     \
+    else rlxq::bs_prep_body<0, ROWS>(a);                                                       \
+  }
+RLXQ_BS_PREP(rlxq_bs_prep2, 2)
+RLXQ_BS_PREP(rlxq_bs_prep8, 8)
 #endif
 
 // rlxq_skinnyns_<scheme>_bs_rt<RT>: up to 256 rows; the prefill sizes run the

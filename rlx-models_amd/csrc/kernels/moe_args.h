@@ -51,18 +51,19 @@ typedef struct rlxq_moe_gemv_args {
   int32_t top_k, out_bf16;
 } rlxq_moe_gemv_args;
 
-/* Grouped batched-decode MFMA path (prefill-sized MoE calls): the entries of
- * each fired expert (table order) are laid out in gathered activation rows,
- * each expert's run padded to whole chunks of rows_per_chunk rows.
- * rlxq_moe_pad_k writes cmap ([0]: chunks, [1 + c]: expert of chunk c) and
- * emap ([Mp]: entry of gathered row, -1 for padding).                     */
-typedef struct rlxq_moe_pad_args {
-  const int32_t* table;
+/* Grouped MFMA path (prefill-sized MoE calls): the entries of each fired
+ * expert are laid out in gathered activation rows, each expert's run padded
+ * to whole chunks of rows_per_chunk rows.  rlxq_moe_layout_k writes cmap ([0]:
+ * chunks, [1 + c]: expert of chunk c) and emap ([Mp]: entry of gathered row,
+ * -1 for padding) from the entries' experts, and zeroes the rows of invalid
+ * entries (t.table is not used).                                           */
+typedef struct rlxq_moe_layout_args {
+  rlxq_moe_table_args t;
   int32_t* cmap;
   int32_t* emap;
   int64_t Mp;
-  int32_t E, rows_per_chunk;
-} rlxq_moe_pad_args;
+  int32_t rows_per_chunk, pad;
+} rlxq_moe_layout_args;
 
 typedef struct rlxq_moe_sk_args {
   const uint16_t* x16;    /* gathered f16 rows, fragment-major over Mp    */
