@@ -318,6 +318,39 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   return rc;
 }
 
+// One to four rows on the matrix cores (mfgemv.hip): whole 256-element units
+// of Q4_1, Q4_K, Q8_0, Q6_K (rows of whole dwords) and MLX 4-bit (group a
+// power of two), at least eight units (one per wave).  Where it is the faster
+// kernel (us, the other one's first; 4096 -> 4096 | 4096 -> 6144 | 4096 ->
+// 24576 | 12288 -> 4096):
+//   Q8_0: always (one f32 row 8.6 7.0 | 13.9 10.6 | 31.9 21.2 | 19.6 14.9,
+//   one bf16 row 7.0 6.8 | 12.0 9.7 | 25.5 20.5 | 15.7 14.3).
+//   Q6_K: from two rows (two f32 rows 42.5 25.0 at 24576), one row only with
+//   many weight rows (f32 7.0 7.4 | 10.4 11.0 | 26.0 23.8 | 15.3 15.2).
+//   4-bit codes, f32 rows: from two (Q4_K, two rows 39.9 18.9 at 24576, 18.9
+//   14.5 at 12288).  bf16 rows: where the register kernel does not hold K
+//   (Q4_1 at 12288, two rows 17.8 12.7, four 18.8 16.5), and three or four
+//   rows with many weight rows (MLX 8.0 7.5 | 9.6 10.1 | 23.7 18.3, Q4_1 6.9
+//   7.3 | 8.7 10.1 | 22.5 18.9) or Q4_K (8.3 7.2 | 10.4 10.2 | 24.7 19.1).
+// RLXQ_GEMV_MF=0 turns it off, =1 takes it wherever it applies (tuning); the
+// other kernels' tuning variables pick those.
+bool mf_applies(int scheme, int group, bool xbf, int64_t m, int64_t k, int64_t n, int64_t rb) {
+  const bool q4 = scheme == RLXQ_GGUF_Q4_1 || scheme == RLXQ_GGUF_Q4_K || scheme == RLXQ_MLX_AFFINE4;
+  if (!q4 && scheme != RLXQ_GGUF_Q8_0 && scheme != RLXQ_GGUF_Q6_K) return false;
+  if (scheme == RLXQ_MLX_AFFINE4 && (group & (group - 1)) != 0) return false;
+  if (scheme == RLXQ_GGUF_Q6_K && rb % 4 != 0) return false;
+  if (m > 4 || k % 256 != 0 || k < 2048 || n < 16 || n >= (int64_t(1) << 31) || rb >= (1 << 27)) return false;
+  if (std::getenv("RLXQ_GEMV_CFG") || (q4 && (std::getenv("RLXQ_GEMV_XR") || std::getenv("RLXQ_GEMV_XSM")))) return false;
+  if (const char* e = std::getenv("RLXQ_GEMV_MF")) return e[0] != '0';
+  if (scheme == RLXQ_GGUF_Q8_0) return true;
+  if (scheme == RLXQ_GGUF_Q6_K) return m > 1 || n >= 16384;
+  if (m == 1) return false;
+  if (!xbf) return true;
+  const int64_t per = scheme == RLXQ_GGUF_Q4_K ? 4096 : 2048;   // K per unit chunk of the register kernel
+  if (k > per * (scheme == RLXQ_GGUF_Q4_K ? (m == 2 ? 2 : 1) : (m == 2 ? 4 : 2))) return true;
+  return m > 2 && (scheme == RLXQ_GGUF_Q4_K || n >= 16384);
+}
+
 int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dtype, const void* w,
                   const void* scales, const void* biases, int sb_dtype, int64_t m, int64_t k,
                   int64_t n, void* y, int y_dtype, void* stream) {
@@ -403,6 +436,35 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   void* args[] = {&a};
   char name[96];
   hipFunction_t fn;
+
+  if (mf_applies(scheme, group, xbf, m, k, n, rb)) {
+    // rows per launch: all of them, or two where four rows' fragments do not
+    // fit the LDS (f32 past K = 8192, bf16 past 18432)
+    const bool has_m = scheme == RLXQ_GGUF_Q4_1 || scheme == RLXQ_GGUF_Q4_K || scheme == RLXQ_MLX_AFFINE4;
+    const int64_t row_lds = scheme == RLXQ_GGUF_Q4_1 ? 176 : scheme == RLXQ_GGUF_Q8_0 ? 272
+                            : scheme == RLXQ_GGUF_Q6_K ? 240 : 144;   // a weight row's unit in LDS
+    auto lds_bytes = [&](int64_t mr) {
+      const int64_t fs = xbf ? mr : 2 * mr, ms = mr > 2 ? mr : fs;   // fragments and sums per block
+      return (size_t)((k / 32 + 8) * 64 * fs + (has_m ? (k / 32) * 4 * ms : 0) + 4096 + 144 + 8 * 16 * row_lds);
+    };
+    int64_t mr = m <= 2 ? m : 4;
+    if (mr == 4 && lds_bytes(mr) > ctx->max_lds) mr = 2;
+    if (lds_bytes(mr) <= ctx->max_lds) {
+      const size_t lds = lds_bytes(mr);
+      std::snprintf(name, sizeof name, xbf ? "rlxq_gemv%s_%s_mf_M%d" : "rlxq_gemv%s_%s_mf%d_F", has_m ? "xs" : "",
+                    scheme_name(scheme), (int)mr);
+      if ((rc = get_fn(ctx, name, &fn))) return rc;
+      const int per_cu = std::max(1, blocks_per_cu(ctx, name, fn, 512, lds));
+      const int64_t gx = std::min<int64_t>((int64_t)ctx->cu_count * per_cu, (n + 15) / 16);
+      for (int64_t r0 = 0; r0 < m; r0 += mr) {
+        a.x = static_cast<const char*>(x) + r0 * k * (xbf ? 2 : 4);
+        a.y = static_cast<char*>(y) + r0 * n * (y_dtype == RLXQ_BF16 ? 2 : 4);
+        a.M = std::min<int64_t>(mr, m - r0);
+        if ((rc = launch(ctx, fn, dim3((unsigned)gx, 1, 1), dim3(512, 1, 1), lds, stream, args, name))) return rc;
+      }
+      return RLXQ_OK;
+    }
+  }
 
   // Single activation row, bf16, 4-bit codes, at most 4 unit chunks of 64 per
   // row (6 for the one-block units): activations held in registers.  By

@@ -50,6 +50,7 @@ RLXQ_EMBED(rlxq_co_skinny, "skinny.co")
 RLXQ_EMBED(rlxq_co_bsgemm0, "bsgemm0.co")
 RLXQ_EMBED(rlxq_co_bsgemm1, "bsgemm1.co")
 RLXQ_EMBED(rlxq_co_bsgemm2, "bsgemm2.co")
+RLXQ_EMBED(rlxq_co_mfgemv, "mfgemv.co")
 
 namespace {
 
@@ -78,6 +79,7 @@ const Image kImages[] = {
     {rlxq_co_bsgemm0_begin, rlxq_co_bsgemm0_end, "bsgemm0"},
     {rlxq_co_bsgemm1_begin, rlxq_co_bsgemm1_end, "bsgemm1"},
     {rlxq_co_bsgemm2_begin, rlxq_co_bsgemm2_end, "bsgemm2"},
+    {rlxq_co_mfgemv_begin, rlxq_co_mfgemv_end, "mfgemv"},
 };
 
 std::string hip_msg(hipError_t e) { return std::string(hipGetErrorName(e)) + ": " + hipGetErrorString(e); }
