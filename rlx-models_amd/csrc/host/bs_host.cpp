@@ -155,7 +155,8 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   a.sb_bf16 = sb.sb_bf16;
   char name[64];
   if (gemm_name) std::snprintf(name, sizeof name, "%s", gemm_name);
-  else std::snprintf(name, sizeof name, "rlxq_skinnyns_%s_bs_rt%d", scheme_name(scheme), RT);
+  else std::snprintf(name, sizeof name, "rlxq_skinny%s_%s_bs_rt%d", scheme == RLXQ_GGUF_Q5_K ? "xr" : "ns",
+                     scheme_name(scheme), RT);
   if ((rc = get_fn(ctx, name, &fn))) return rc;
   void* args[] = {&a};
   // three activation slots (two 32-element blocks each), the waves' weight

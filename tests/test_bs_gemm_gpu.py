@@ -66,7 +66,7 @@ def _check(ctx, orc, scheme, m, k, n, y_dtype=None):
 def test_batched(ctx, orc, scheme, mkn):
     announce(f"block-scaled {NAMES[scheme]} {mkn}")
     kern = _check(ctx, orc, scheme, *mkn)
-    assert kern.startswith(f"rlxq_skinnyns_{NAMES[scheme]}_bs_rt"), kern
+    assert f"_{NAMES[scheme]}_bs_rt" in kern, kern
 
 
 @pytest.mark.parametrize("scheme,mkn", [(Q4_1, (300, 64 * 13, 301)), (Q4_0, (257, 64 * 5, 130)), (Q8_0, (259, 64 * 7, 33)),
@@ -89,7 +89,7 @@ def test_row_tiles_and_splits(ctx, orc, monkeypatch, cfg):
     for scheme, mkn in ((Q4_1, (70, 1792, 200)), (Q4_K, (40, 2816, 129)), (Q6_K, (70, 1792, 133))):
         announce(f"block-scaled {cfg} {NAMES[scheme]} {mkn}")
         kern = _check(ctx, orc, scheme, *mkn)
-        assert kern == f"rlxq_skinnyns_{NAMES[scheme]}_bs_rt{cfg[0]}", kern
+        assert kern.endswith(f"_{NAMES[scheme]}_bs_rt{cfg[0]}"), kern
 
 
 def test_noalloc_is_the_same(ctx, orc):
