@@ -323,15 +323,21 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
 // power of two), at least eight units (one per wave).  Where it is the faster
 // kernel (us, the other one's first; 4096 -> 4096 | 4096 -> 6144 | 4096 ->
 // 24576 | 12288 -> 4096):
-//   Q8_0: always (one f32 row 8.6 7.0 | 13.9 10.6 | 31.9 21.2 | 19.6 14.9,
-//   one bf16 row 7.0 6.8 | 12.0 9.7 | 25.5 20.5 | 15.7 14.3).
-//   Q6_K: from two rows (two f32 rows 42.5 25.0 at 24576), one row only with
-//   many weight rows (f32 7.0 7.4 | 10.4 11.0 | 26.0 23.8 | 15.3 15.2).
-//   4-bit codes, f32 rows: from two (Q4_K, two rows 39.9 18.9 at 24576, 18.9
-//   14.5 at 12288).  bf16 rows: where the register kernel does not hold K
-//   (Q4_1 at 12288, two rows 17.8 12.7, four 18.8 16.5), and three or four
-//   rows with many weight rows (MLX 8.0 7.5 | 9.6 10.1 | 23.7 18.3, Q4_1 6.9
-//   7.3 | 8.7 10.1 | 22.5 18.9) or Q4_K (8.3 7.2 | 10.4 10.2 | 24.7 19.1).
+//   Q8_0: always (one f32 row 8.6 6.5 | 13.9 9.0 | 31.9 21.6 | 19.6 13.0,
+//   one bf16 row 7.0 6.3 | 12.0 8.9 | 25.5 21.4 | 15.7 12.7).
+//   Q6_K: f32 rows and from two bf16 rows always (one f32 row 6.9 6.9 | 10.5
+//   9.4 | 26.0 23.3 | 15.2 13.8, two 42.5 24.3 at 24576); one bf16 row with
+//   many weight rows or a long K (6.7 7.0 | 9.2 9.5 | 24.2 23.0 | 13.8 13.8,
+//   14336 -> 6144 27.4 24.4).
+//   4-bit codes, f32: from two rows (Q4_K, two rows 39.9 18.0 at 24576, 18.9
+//   12.2 at 12288); one row past the K the register kernel is good at (12288
+//   -> 4096, Q4_K 11.9 10.8, MLX 11.8 10.4, Q4_1 10.3 10.3; 8192 -> 2048,
+//   Q4_K 7.8 7.4, MLX 5.8 7.5, Q4_1 6.4 6.7).
+//   4-bit codes, bf16: where the register kernel does not hold K (Q4_1 at
+//   12288, two rows 17.8 10.8, four 18.8 13.1; Q4_K at 8192, two rows 8.7
+//   7.9), and three or four rows (MLX 7.7 6.8 | 9.5 9.2 | 23.7 17.7, Q4_K 8.3
+//   6.9 | 10.4 9.3 | 24.7 18.3), Q4_1 only with many weight rows (7.1 6.8 |
+//   8.6 9.1 | 22.5 18.4).
 // RLXQ_GEMV_MF=0 turns it off, =1 takes it wherever it applies (tuning); the
 // other kernels' tuning variables pick those.
 bool mf_applies(int scheme, int group, bool xbf, int64_t m, int64_t k, int64_t n, int64_t rb) {
@@ -343,12 +349,12 @@ bool mf_applies(int scheme, int group, bool xbf, int64_t m, int64_t k, int64_t n
   if (std::getenv("RLXQ_GEMV_CFG") || (q4 && (std::getenv("RLXQ_GEMV_XR") || std::getenv("RLXQ_GEMV_XSM")))) return false;
   if (const char* e = std::getenv("RLXQ_GEMV_MF")) return e[0] != '0';
   if (scheme == RLXQ_GGUF_Q8_0) return true;
-  if (scheme == RLXQ_GGUF_Q6_K) return m > 1 || n >= 16384;
+  if (scheme == RLXQ_GGUF_Q6_K) return m > 1 || !xbf || n >= 16384 || k > 12288;
+  if (!xbf) return m > 1 || k > (scheme == RLXQ_GGUF_Q4_K ? 4096 : scheme == RLXQ_MLX_AFFINE4 ? 8192 : 12288);
   if (m == 1) return false;
-  if (!xbf) return true;
-  const int64_t per = scheme == RLXQ_GGUF_Q4_K ? 4096 : 2048;   // K per unit chunk of the register kernel
-  if (k > per * (scheme == RLXQ_GGUF_Q4_K ? (m == 2 ? 2 : 1) : (m == 2 ? 4 : 2))) return true;
-  return m > 2 && (scheme == RLXQ_GGUF_Q4_K || n >= 16384);
+  // (the register kernel's unit chunks are 4096 of K for Q4_K, else 2048)
+  if (k > (scheme == RLXQ_GGUF_Q4_K ? 4096 : m == 2 ? 8192 : 4096)) return true;
+  return m > 2 && (scheme != RLXQ_GGUF_Q4_1 || n >= 16384);
 }
 
 int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dtype, const void* w,
@@ -445,7 +451,7 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
                             : scheme == RLXQ_GGUF_Q6_K ? 240 : 144;   // a weight row's unit in LDS
     auto lds_bytes = [&](int64_t mr) {
       const int64_t fs = xbf ? mr : 2 * mr, ms = mr > 2 ? mr : fs;   // fragments and sums per block
-      return (size_t)((k / 32 + 8) * 64 * fs + (has_m ? (k / 32) * 4 * ms : 0) + 4096 + 144 + 8 * 16 * row_lds);
+      return (size_t)((k / 32 + 8) * 64 * fs + (has_m ? (k / 32) * 4 * ms : 0) + 4096 + 8 * 16 * row_lds);
     };
     int64_t mr = m <= 2 ? m : 4;
     if (mr == 4 && lds_bytes(mr) > ctx->max_lds) mr = 2;

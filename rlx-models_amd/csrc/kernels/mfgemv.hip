@@ -22,10 +22,14 @@
 // Q4_1 against 16.6.)
 //
 // What bounds it: 8-bit codes the weights' bandwidth (Q8_0 4096->24576, one
-// f32 row 31.9 -> 21.2 us, 5.0 TB/s); 4-bit ones the instructions per weight
-// (MLX, four bf16 rows 23.7 -> 18.3 us; Q4_K, four f32 rows 46.1 -> 21.4);
-// small calls the activations' two passes ahead of the first product (about
-// 2 us; Q8_0 2048->2048 5.1 -> 4.3 us).
+// f32 row 31.9 -> 21.5 us, 5.0 TB/s; 12288->4096 19.6 -> 13.0); 4-bit ones the
+// instructions per weight and the start (MLX, four bf16 rows 23.7 -> 17.7 us,
+// 12288->4096 20.6 -> 13.1; Q4_K, four f32 rows 46.1 -> 19.5); small calls the
+// activations' way to the first product (Q8_0 2048->2048 5.1 -> 4.3 us).  So
+// each wave prepares the activations of its own units, without a barrier, and
+// asks for them ahead of the weights (12288->4096, MLX, four bf16 rows: 16.6
+// us with the workgroup's maxima and the weights first, 15.2 by wave, 13.1
+// with the activations first).
 #include "common.hip.h"
 #include "f16dq.hip.h"
 #include "gemv_args.h"
@@ -150,10 +154,10 @@ RLXQ_DEV f16x8_t mf_codes(const MfRaw<SCH>& r) {
 
 // LDS: x fragments [K / 32][4][MS NH] of 16 bytes, 8 * 4 * MS NH zero
 // fragments' worth, block sums [K / 32][MS] f32 (formats with a min / bias),
-// partial sums [2][8 waves][64] f32, row maxima [4][8] and scales [4].
-template <int SCH, bool XBF, int MR>
+// partial sums [2][8 waves][64] f32, then the waves' weight regions.
+template <int SCH, bool XBF, int MR, int D>
 RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
-  constexpr int W = 8, D = SCH == SCH_Q8_0 || SCH == SCH_Q6_K ? 2 : 3;
+  constexpr int W = 8;
   // f32 rows are f16 hi and lo: as rows of their own up to two, as two
   // products into the same sums past that
   constexpr int NH = !XBF && MR > 2 ? 2 : 1, MS = XBF || MR > 2 ? MR : 2 * MR, FS = MS * NH;
@@ -168,9 +172,7 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
   uint8_t* zs = xs + nblk * 64 * FS;
   float* sums = reinterpret_cast<float*>(zs + 8 * 64 * FS);
   float* red = sums + (HM ? nblk * MS : 0);
-  float* rmax = red + 2 * W * 64;
-  float* rinv = rmax + 32;
-  uint8_t* reg = reinterpret_cast<uint8_t*>(rinv + 4) + wv * (16 * LROW);
+  uint8_t* reg = reinterpret_cast<uint8_t*>(red + 2 * W * 64) + wv * (16 * LROW);
 
   // the wave's units of every tile of 16 weight rows (the last tile ends with
   // row N - 1 and shares rows with the one before it: the same sums, written
@@ -232,117 +234,142 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
     }
     if (++lu == cnt) lu = 0, lt += gridDim.x;
   };
-  static_for<D>([&](auto Q) { load(Q); });
 
-  // The activation rows: maxima, then f16 fragments (each row scaled by the
-  // power of two that puts its maximum in [2^9, 2^10)) and block sums.  Piece
-  // p: positions 8 (p % 4) .. of block p / 4 in code order (natural, GGUF
-  // nibbles, MLX nibbles).
-  auto ldx = [&](int row, int p, float* v) {
+  // The activation rows over the wave's own units: maxima, then f16 fragments
+  // (each row scaled by the power of two that puts its maximum there in [2^9,
+  // 2^10)) and block sums.  Piece p: positions 8 (p % 4) .. of block p / 4 in
+  // code order (natural, GGUF nibbles, MLX nibbles).  A wave reads only what
+  // it wrote: no barrier before the first tile's end.
+  const int p0 = u0 * 32, p1 = (u0 + cnt) * 32;
+  struct Piece { uint32_t w[XBF ? 4 : 8]; };   // as read (bf16 pairs or f32)
+  auto ldx = [&](int row, int p) {
     const int i = p & 3;
     const int64_t e0 = (int64_t)(row < a.M ? row : a.M - 1) * K + (p >> 2) * 32 + (ORD == 1 ? 4 * i : 8 * i);
     const int64_t e1 = e0 + (ORD == 1 ? 16 : 4);
-    float n[8];
+    Piece v;
     if constexpr (XBF) {
       const uint16_t* x = reinterpret_cast<const uint16_t*>(a.x);
       const uint2 c0 = *reinterpret_cast<const uint2*>(x + e0), c1 = *reinterpret_cast<const uint2*>(x + e1);
-      const uint32_t w[4] = {c0.x, c0.y, c1.x, c1.y};
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        n[2 * e] = __uint_as_float(w[e] << 16);
-        n[2 * e + 1] = __uint_as_float(w[e] & 0xffff0000u);
-      }
+      v.w[0] = c0.x; v.w[1] = c0.y; v.w[2] = c1.x; v.w[3] = c1.y;
     } else {
-      const float* x = reinterpret_cast<const float*>(a.x);
-      const float4 f0 = *reinterpret_cast<const float4*>(x + e0), f1 = *reinterpret_cast<const float4*>(x + e1);
-      n[0] = f0.x; n[1] = f0.y; n[2] = f0.z; n[3] = f0.w;
-      n[4] = f1.x; n[5] = f1.y; n[6] = f1.z; n[7] = f1.w;
+      const uint32_t* x = reinterpret_cast<const uint32_t*>(a.x);
+      const uint4 c0 = *reinterpret_cast<const uint4*>(x + e0), c1 = *reinterpret_cast<const uint4*>(x + e1);
+      v.w[0] = c0.x; v.w[1] = c0.y; v.w[2] = c0.z; v.w[3] = c0.w;
+      v.w[4] = c1.x; v.w[5] = c1.y; v.w[6] = c1.z; v.w[7] = c1.w;
     }
-#pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = n[ORD == 2 ? (e < 4 ? 2 * e : 2 * (e - 4) + 1) : e];
+    return v;
   };
+  float inv[MR];
   {
-    const int np = nblk * 4;
-    float mx[MR], v0[MR][8];   // (each thread's first piece of a row stays in registers)
+    // Each lane's first NV pieces of a row stay in registers, and are asked
+    // for ahead of the weights: loads return in order.
+    constexpr int NV = XBF || MR <= 2 ? 3 : 1;
+    Piece v0[NV][MR];
+    float mx[MR];
 #pragma unroll
-    for (int r = 0; r < MR; r++) {
-      ldx(r, tid < np ? tid : np - 1, v0[r]);
-      mx[r] = 0.f;
-    }
-    for (int p = tid + 64 * W; p < np; p += 64 * W)
+    for (int q = 0; q < NV; q++)
+      if (p0 + 64 * q < p1) {
+        const int p = p0 + 64 * q + lane < p1 ? p0 + 64 * q + lane : p1 - 1;
 #pragma unroll
-      for (int r = 0; r < MR; r++) {
-        float v[8];
-        ldx(r, p, v);
-#pragma unroll
-        for (int e = 0; e < 8; e++) mx[r] = fmaxf(mx[r], fabsf(v[e]));
+        for (int r = 0; r < MR; r++) v0[q][r] = ldx(r, p);
       }
+    static_for<D>([&](auto Q) { load(Q); });
+#pragma unroll
+    for (int r = 0; r < MR; r++) mx[r] = 0.f;
+    // bf16: the magnitudes' maximum per half, as integers
+    typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+    u16x2_t mh[MR];
+#pragma unroll
+    for (int r = 0; r < MR; r++) mh[r] = u16x2_t{0, 0};
+    auto take = [&](int r, const Piece& v) {
+      if constexpr (XBF) {
+#pragma unroll
+        for (int e = 0; e < 4; e++)
+          mh[r] = __builtin_elementwise_max(mh[r], __builtin_bit_cast(u16x2_t, v.w[e] & 0x7fff7fffu));
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; e++) mx[r] = fmaxf(mx[r], fabsf(__uint_as_float(v.w[e])));
+      }
+    };
+#pragma unroll
+    for (int q = 0; q < NV; q++)
+      if (p0 + 64 * q < p1) {
+#pragma unroll
+        for (int r = 0; r < MR; r++) take(r, v0[q][r]);
+      }
+    for (int p = p0 + 64 * NV + lane; p < p1; p += 64)
+#pragma unroll
+      for (int r = 0; r < MR; r++) take(r, ldx(r, p));
+    for (int p = lane; p < 8 * 4 * FS; p += 64) *reinterpret_cast<u32x4_t*>(zs + 16 * p) = u32x4_t{0u, 0u, 0u, 0u};
 #pragma unroll
     for (int r = 0; r < MR; r++) {
-#pragma unroll
-      for (int e = 0; e < 8; e++) mx[r] = fmaxf(mx[r], fabsf(v0[r][e]));
+      if constexpr (XBF) {
+        const uint32_t h = mh[r].x > mh[r].y ? mh[r].x : mh[r].y;
+        // (a NaN's bits are above every number's, and fmaxf would drop it)
+        mx[r] = __uint_as_float(h > 0x7f80u ? 0x7f800000u : h << 16);
+      }
       mx[r] = fmaxf(mx[r], mf_dpp<0x128>(mx[r]));   // (row_ror 8, 4, 2, 1)
       mx[r] = fmaxf(mx[r], mf_dpp<0x124>(mx[r]));
       mx[r] = fmaxf(mx[r], mf_dpp<0x122>(mx[r]));
       mx[r] = fmaxf(mx[r], mf_dpp<0x121>(mx[r]));
       mx[r] = mf_rows(mx[r], [](float p, float q) { return fmaxf(p, q); });
-      if (lane == 0) rmax[r * W + wv] = mx[r];
-    }
-    for (int p = tid; p < 8 * 4 * FS; p += 64 * W) *reinterpret_cast<u32x4_t*>(zs + 16 * p) = u32x4_t{0u, 0u, 0u, 0u};
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-    for (int r = 0; r < MR; r++) {
-      const f32x4_t m0 = *reinterpret_cast<const f32x4_t*>(rmax + r * W), m1 = *reinterpret_cast<const f32x4_t*>(rmax + r * W + 4);
-      const float amax = fmaxf(fmaxf(fmaxf(m0.x, m0.y), fmaxf(m0.z, m0.w)), fmaxf(fmaxf(m1.x, m1.y), fmaxf(m1.z, m1.w)));
       // (by exponent; a zero row and one that is not finite stay as they are)
-      const uint32_t ex = __float_as_uint(amax) >> 23;
+      const uint32_t ex = __float_as_uint(mx[r]) >> 23;
       int sh = 136 - (int)ex;
       sh = sh > 126 ? 126 : sh;
-      if (amax == 0.f || ex >= 255u) sh = 0;
-      const float s = __uint_as_float((uint32_t)(127 + sh) << 23), inv = __uint_as_float((uint32_t)(127 - sh) << 23);
-      if (tid == 0) rinv[r] = inv;
-      auto put = [&](int p, const float* v) {
+      if (mx[r] == 0.f || ex >= 255u) sh = 0;
+      const float s = __uint_as_float((uint32_t)(127 + sh) << 23);
+      inv[r] = __uint_as_float((uint32_t)(127 - sh) << 23);
+      auto put = [&](int p, const Piece& v) {
         uint32_t hi[4], lo[4];
-        float sh = 0.f, sl = 0.f;
+        float th = 0.f, tl = 0.f;
+        const f16x2_t one = {(_Float16)1.f, (_Float16)1.f};
+        float w[8];
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+          const int q = ORD == 2 ? (e < 4 ? 2 * e : 2 * (e - 4) + 1) : e;
+          if constexpr (XBF) w[e] = __uint_as_float(q & 1 ? v.w[q / 2] & 0xffff0000u : v.w[q / 2] << 16) * s;
+          else w[e] = __uint_as_float(v.w[q]) * s;
+        }
 #pragma unroll
         for (int e = 0; e < 4; e++) {
-          const float w0 = v[2 * e] * s, w1 = v[2 * e + 1] * s;
-          const uint32_t h0 = f32_to_f16_bits(w0), h1 = f32_to_f16_bits(w1);
+          const uint32_t h0 = f32_to_f16_bits(w[2 * e]), h1 = f32_to_f16_bits(w[2 * e + 1]);
           hi[e] = h0 | (h1 << 16);
-          const float g0 = f16_bits_to_f32(h0), g1 = f16_bits_to_f32(h1);
-          sh += g0 + g1;
+          if constexpr (HM) th = __builtin_amdgcn_fdot2(as_h2(hi[e]), one, th, false);
           if constexpr (!XBF) {
             // (the remainder is exact in f32; rounded once more)
-            const uint32_t l0 = f32_to_f16_bits(w0 - g0), l1 = f32_to_f16_bits(w1 - g1);
+            const uint32_t l0 = f32_to_f16_bits(w[2 * e] - f16_bits_to_f32(h0));
+            const uint32_t l1 = f32_to_f16_bits(w[2 * e + 1] - f16_bits_to_f32(h1));
             lo[e] = l0 | (l1 << 16);
-            sl += f16_bits_to_f32(l0) + f16_bits_to_f32(l1);
+            if constexpr (HM) tl = __builtin_amdgcn_fdot2(as_h2(lo[e]), one, tl, false);
           }
         }
         *reinterpret_cast<u32x4_t*>(xs + (p * FS + r) * 16) = u32x4_t{hi[0], hi[1], hi[2], hi[3]};
         if constexpr (!XBF) *reinterpret_cast<u32x4_t*>(xs + (p * FS + MR + r) * 16) = u32x4_t{lo[0], lo[1], lo[2], lo[3]};
         if constexpr (HM) {
-          // the block's four pieces are four neighbouring lanes
+          // the block's four pieces are four neighbouring lanes, which all
+          // store their sum
           auto sum = [&](float t, int slot) {
             t += mf_dpp<0xB1>(t);
             t += mf_dpp<0x4E>(t);
-            if ((p & 3) == 0) sums[(p >> 2) * MS + slot] = t;
+            sums[(p >> 2) * MS + slot] = t;
           };
           if constexpr (MS == MR) {
-            sum(sh + sl, r);
+            sum(th + tl, r);
           } else {
-            sum(sh, r);
-            sum(sl, MR + r);
+            sum(th, r);
+            sum(tl, MR + r);
           }
         }
       };
-      if (tid < np) put(tid, v0[r]);
-      for (int p = tid + 64 * W; p < np; p += 64 * W) {
-        float v[8];
-        ldx(r, p, v);
-        put(p, v);
-      }
+#pragma unroll
+      for (int q = 0; q < NV; q++)
+        if (p0 + 64 * q + lane < p1) put(p0 + 64 * q + lane, v0[q][r]);
+      for (int p = p0 + 64 * NV + lane; p < p1; p += 64) put(p, ldx(r, p));
     }
-    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    // (the lanes' reads below cross lanes: not before these stores, some of
+    // which are conditional)
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
 
   // The lane's x operand: row 4G + r of an MFMA's 16 takes row r's values of
@@ -439,7 +466,7 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
         // follows this one's reads.)
         cu = 0;
 #pragma unroll
-        for (int q = 0; q < MS; q++) acc[q] = mf_rows(acc[q], [](float p, float q) { return p + q; });
+        for (int q = 0; q < MS; q++) acc[q] = mf_rows(acc[q], [](float p, float q) { return p + q; }) * inv[q % MR];
         float v = acc[0];
 #pragma unroll
         for (int q = 1; q < MS; q++) v = g == q ? acc[q] : v;
@@ -452,7 +479,6 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
             o += red[(buf * W + w) * 64 + lane];
             if constexpr (MS > MR) o += red[(buf * W + w) * 64 + lane + 16 * MR];
           }
-          o *= rinv[g];
           const int64_t n = tile_row(ct) + j;
           if (g < a.M) {
             if (a.y_bf16) reinterpret_cast<uint16_t*>(a.y)[g * a.y_ld + n] = (uint16_t)f32_to_bf16_bits(o);
@@ -471,19 +497,21 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
 
 }  // namespace rlxq
 
-#define RLXQ_MF_INST(NAME, SCH, XBF, MR)                                                  \
+#define RLXQ_MF_INST(NAME, SCH, XBF, MR, D)                                               \
   extern "C" __global__ __launch_bounds__(512, 4) void NAME(rlxq_gemv_args a) {          \
-    rlxq::mf_body<SCH, XBF, MR>(a);                                                       \
+    rlxq::mf_body<SCH, XBF, MR, D>(a);                                                    \
   }
-#define RLXQ_MF_SCHEME(PRE, SNAME, SCH)                     \
-  RLXQ_MF_INST(PRE##_##SNAME##_mf_M1, SCH, true, 1)         \
-  RLXQ_MF_INST(PRE##_##SNAME##_mf_M2, SCH, true, 2)         \
-  RLXQ_MF_INST(PRE##_##SNAME##_mf_M4, SCH, true, 4)         \
-  RLXQ_MF_INST(PRE##_##SNAME##_mf1_F, SCH, false, 1)        \
-  RLXQ_MF_INST(PRE##_##SNAME##_mf2_F, SCH, false, 2)        \
-  RLXQ_MF_INST(PRE##_##SNAME##_mf4_F, SCH, false, 4)
-RLXQ_MF_SCHEME(rlxq_gemvxs, q4_1, SCH_Q4_1)
-RLXQ_MF_SCHEME(rlxq_gemvxs, q4_k, SCH_Q4_K)
-RLXQ_MF_SCHEME(rlxq_gemvxs, mlx4, SCH_MLX4)
-RLXQ_MF_SCHEME(rlxq_gemv, q8_0, SCH_Q8_0)
-RLXQ_MF_SCHEME(rlxq_gemv, q6_k, SCH_Q6_K)
+// (D units in flight per wave; six, with one workgroup per CU and twice the
+// registers, were slower everywhere: Q8_0 12288->4096 13.0 us and 15.0)
+#define RLXQ_MF_SCHEME(PRE, SCH, D)              \
+  RLXQ_MF_INST(PRE##_mf_M1, SCH, true, 1, D)     \
+  RLXQ_MF_INST(PRE##_mf_M2, SCH, true, 2, D)     \
+  RLXQ_MF_INST(PRE##_mf_M4, SCH, true, 4, D)     \
+  RLXQ_MF_INST(PRE##_mf1_F, SCH, false, 1, D)    \
+  RLXQ_MF_INST(PRE##_mf2_F, SCH, false, 2, D)    \
+  RLXQ_MF_INST(PRE##_mf4_F, SCH, false, 4, D)
+RLXQ_MF_SCHEME(rlxq_gemvxs_q4_1, SCH_Q4_1, 3)
+RLXQ_MF_SCHEME(rlxq_gemvxs_q4_k, SCH_Q4_K, 3)
+RLXQ_MF_SCHEME(rlxq_gemvxs_mlx4, SCH_MLX4, 3)
+RLXQ_MF_SCHEME(rlxq_gemv_q8_0, SCH_Q8_0, 2)
+RLXQ_MF_SCHEME(rlxq_gemv_q6_k, SCH_Q6_K, 2)
