@@ -402,6 +402,8 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   // once for all rows through the f16-MFMA kernel (MXFP4 with E8M0 scales
   // through its bf16-MFMA twin).  bf16 activations are exact in f16 once
   // scaled; f32 activations run as hi + lo row pairs (~22 significant bits).
+  // (f32 activations past 16 rows, formats of bs_scheme: the block-scaled
+  // matmul.  Q4_1 4096->24576 at 64 rows 90 us here, 51 there.)
   // RLXQ_DECODE=gemv|skinny forces one where both apply.
   {
     const bool sk_ok = skinny_applies(scheme, group, sb_dtype, m, k);
