@@ -65,14 +65,22 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   // 64-row tiles past 32 rows (197 rows of Q4_K, 4096->24576: 131 us in four
   // of them, 151 in seven 32-row ones; 64 rows of Q4_1: 51 and 55); 128
   // columns.  RLXQ_BS="RT,splits" (tuning) sets the 32-row tiles per
-  // workgroup (1 or 2) and, unless 0, the K splits.
+  // workgroup (1 or 2; 0: the form with 64-bit row offsets) and, unless 0,
+  // the K splits.
   const int64_t r32 = (m + 31) / 32;
+  // (32 weight rows past 4 GB: the form with 64-bit row offsets)
+  bool wide = rb >= ((int64_t)1 << 27);
   int RT = gemm_name || m > 32 ? 2 : 1;
   int64_t want = 0;
   if (const char* e = std::getenv("RLXQ_BS")) {
     int a1, a2;
-    if (std::sscanf(e, "%d,%d", &a1, &a2) == 2 && (a1 == 1 || a1 == 2)) RT = gemm_name ? 2 : a1, want = a2;
+    if (std::sscanf(e, "%d,%d", &a1, &a2) == 2 && a1 >= 0 && a1 <= 2) {
+      want = a2;
+      if (a1 == 0) wide = true;
+      else if (!gemm_name) RT = a1;
+    }
   }
+  if (wide) RT = 1;
   if (gemm_name)
     if (const char* e = std::getenv("RLXQ_GEMM_SPLITS")) want = std::max(1, std::atoi(e));
   const int64_t tiles_m = (m + 32 * RT - 1) / (32 * RT), tiles_n = (n + 127) / 128;
@@ -154,7 +162,8 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   a.y_bf16 = y_dtype == RLXQ_BF16;
   a.sb_bf16 = sb.sb_bf16;
   char name[64];
-  if (gemm_name) std::snprintf(name, sizeof name, "%s", gemm_name);
+  if (wide) std::snprintf(name, sizeof name, "rlxq_bs_%s_wide", scheme_name(scheme));
+  else if (gemm_name) std::snprintf(name, sizeof name, "%s", gemm_name);
   else std::snprintf(name, sizeof name, "rlxq_skinny%s_%s_bs_rt%d", scheme == RLXQ_GGUF_Q5_K ? "xr" : "ns",
                      scheme_name(scheme), RT);
   if ((rc = get_fn(ctx, name, &fn))) return rc;

@@ -244,8 +244,9 @@ RLXQ_DEV float bs_scale(const BsRaw<SCH>& q, const BsRow<SCH>& r) {
 // The contraction of 32 RT activation rows (32-row tiles rt0 ..) with the
 // wave's 32 TN weight rows (row r of them at w + roff(r)) over units [u0, u1).
 // lds: three activation slots of RT NH 4 KB, then the four waves' weight
-// regions of 32 TN LROW bytes.
-template <int SCH, int RT, int TN, int NH, class RowOff>
+// regions of 32 TN LROW bytes.  Off: type of the byte offsets between the
+// wave's weight rows (32 bits while 32 rows lie within 4 GB).
+template <int SCH, int RT, int TN, int NH, class Off, class RowOff>
 RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16, const uint32_t* ssum, int rtiles,
                       int rt0, int u0, int u1, f32x16_t (&acc)[RT][TN], uint8_t* lds) {
   constexpr int XB = RT * NH * 2;                 // fragments (1 KB) per block
@@ -283,17 +284,17 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
   };
   // weight pieces of a unit, in row order: piece p is 16-byte unit p % PPR of
   // row p / PPR
-  // (byte offsets from the wave's first row: a few rows apart, 32 bits)
+  // (byte offsets from the wave's first row)
   const uint8_t* wbase = ga.w + roff(0);
-  uint32_t src[NL];
+  Off src[NL];
   int dst[NL];
 #pragma unroll
   for (int u = 0; u < NL; u++) {
     const int p = lane + 64 * u < NP ? lane + 64 * u : NP - 1;
-    src[u] = (uint32_t)(roff(p / PPR) - roff(0)) + (p % PPR) * 16;
+    src[u] = (Off)(roff(p / PPR) - roff(0)) + (p % PPR) * 16;
     dst[u] = (p / PPR) * LROW + (p % PPR) * 16;
   }
-  const uint32_t tsrc = SCH == SCH_Q6_K ? (uint32_t)(roff(j) - roff(0)) : 0u;
+  const Off tsrc = SCH == SCH_Q6_K ? (Off)(roff(j) - roff(0)) : 0u;
   u32x4_t wr[NL];
   uint32_t tail = 0u;   // Q6_K: the last dword of row j
   float ms[MLX ? TN : 1][4], mb[MLX ? TN : 1][4];
@@ -307,15 +308,15 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
       // (K is whole units.)  Row offsets are even: the dword a super-block
       // starts in lies 0 or 2 bytes before it, and everything read here stays
       // inside the super-block and those two bytes
-      const uint32_t uo = (uint32_t)((reinterpret_cast<uintptr_t>(wbase) & 3u) + (uint64_t)uu * 210);
+      const Off uo = (Off)((reinterpret_cast<uintptr_t>(wbase) & 3u) + (uint64_t)uu * 210);
       const uint8_t* w4 = wbase - (reinterpret_cast<uintptr_t>(wbase) & 3u);
 #pragma unroll
       for (int q = 0; q < NL; q++) {
         const uint32_t c = dst[q] % LROW;
-        const uint4 v = ld_u128(w4 + ((src[q] - c + uo) & ~3u) + c);
+        const uint4 v = ld_u128(w4 + ((src[q] - c + uo) & ~(Off)3) + c);
         wr[q] = u32x4_t{v.x, v.y, v.z, v.w};
       }
-      const uint32_t so = tsrc + uo, so4 = so & ~3u;
+      const Off so = tsrc + uo, so4 = so & ~(Off)3;
       const uint16_t* p = reinterpret_cast<const uint16_t*>(w4 + so4 + 208);
       const uint32_t lo = p[0], hi = p[so & 2u ? 1 : 0];
       tail = lo | (hi << 16);
@@ -406,7 +407,7 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
     BsRow<SCH> row[TN];
     if constexpr (SCH == SCH_Q6_K) {
       *reinterpret_cast<uint32_t*>(reg + j * LROW + 208) = tail;
-      row[0].off = (uint32_t)((reinterpret_cast<uintptr_t>(wbase) & 3u) + tsrc + (uint32_t)u * 210) & 2u;
+      row[0].off = (uint32_t)((reinterpret_cast<uintptr_t>(wbase) & 3u) + (uint32_t)tsrc + (uint32_t)u * 210) & 2u;
     }
     if constexpr (MLX) {
 #pragma unroll
@@ -543,7 +544,7 @@ struct BsDenseRows {
 };
 
 // Dense form: workgroup = (32 RT rows, 128 TN weight rows, K split).
-template <int SCH, int RT, int TN, int NH>
+template <int SCH, int RT, int TN, int NH, class Off>
 RLXQ_DEV void bs_body(const rlxq_bs_args& a) {
   extern __shared__ __align__(16) uint8_t bs_lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -574,7 +575,7 @@ RLXQ_DEV void bs_body(const rlxq_bs_args& a) {
   ga.biases = a.biases;
   const BsDenseRows roff{n0, a.N, a.rb, bs_mlx<SCH>() ? a.K / a.group : 0};
   f32x16_t acc[RT][TN];
-  bs_core<SCH, RT, TN, NH>(ga, roff, a.x16, a.ssum, a.rtiles, mc * RT, u0, u1, acc, bs_lds);
+  bs_core<SCH, RT, TN, NH, Off>(ga, roff, a.x16, a.ssum, a.rtiles, mc * RT, u0, u1, acc, bs_lds);
   // C[i][j] of a 32 x 32 tile sits in lane j + 32 ((i / 4) % 2), register
   // 4 (i / 8) + i % 4.  The row factors come as vector loads and the bounds
   // and the destination are decided once per workgroup (a load and a branch
@@ -661,7 +662,7 @@ RLXQ_DEV void bs_moe_body(const rlxq_moe_sk_args& a) {
   ga.biases = a.biases;
   const BsMoeRows roff{n0, width, a.rb, bs_mlx<SCH>() ? a.K / a.group : 0, (int64_t)e * a.N};
   f32x16_t acc[1][TN];
-  bs_core<SCH, 1, TN, 2>(ga, roff, reinterpret_cast<const uint8_t*>(a.x16), reinterpret_cast<const uint32_t*>(a.ssum),
+  bs_core<SCH, 1, TN, 2, uint32_t>(ga, roff, reinterpret_cast<const uint8_t*>(a.x16), reinterpret_cast<const uint32_t*>(a.ssum),
                          (int)(a.Mp / 32), chunk, 0, (int)((a.K + 255) / 256), acc, bs_lds);
   typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
   const int64_t m0 = (int64_t)chunk * 32 + 4 * h, c = n0 + j;
@@ -828,15 +829,17 @@ RLXQ_BS_PREP(rlxq_bs_prep8, 8)
 
 // rlxq_skinnyns_<scheme>_bs_rt<RT> (Q5_K: skinnyxr, the batched kernel it has
 // besides): up to 256 rows; the prefill sizes run the 64-row form under the
-// exact GEMM's names.
-#define RLXQ_BS_INST(NAME, SCH, RT)                                                            \
+// exact GEMM's names.  rlxq_bs_<scheme>_wide: rows of 128 MB and more, whose
+// offsets take 64 bits (a register more per piece: the others stay on 32).
+#define RLXQ_BS_INST(NAME, SCH, RT, OFF)                                                       \
   extern "C" __global__ __launch_bounds__(256, 2) void NAME(rlxq_bs_args a) {                  \
-    rlxq::bs_body<SCH, RT, 1, 2>(a);                                                           \
+    rlxq::bs_body<SCH, RT, 1, 2, OFF>(a);                                                      \
   }
 #define RLXQ_BS_SCHEME(SNAME, SCH, KIND, GEMM)                                                 \
-  RLXQ_BS_INST(rlxq_skinny##KIND##_##SNAME##_bs_rt1, SCH, 1)                                    \
-  RLXQ_BS_INST(rlxq_skinny##KIND##_##SNAME##_bs_rt2, SCH, 2)                                    \
-  RLXQ_BS_INST(GEMM, SCH, 2)                                                                   \
+  RLXQ_BS_INST(rlxq_skinny##KIND##_##SNAME##_bs_rt1, SCH, 1, uint32_t)                          \
+  RLXQ_BS_INST(rlxq_skinny##KIND##_##SNAME##_bs_rt2, SCH, 2, uint32_t)                          \
+  RLXQ_BS_INST(GEMM, SCH, 2, uint32_t)                                                         \
+  RLXQ_BS_INST(rlxq_bs_##SNAME##_wide, SCH, 1, uint64_t)                                        \
   extern "C" __global__ __launch_bounds__(256, 2) void rlxq_moesk_##SNAME##_bs(rlxq_moe_sk_args a) { \
     rlxq::bs_moe_body<SCH, false>(a);                                                          \
   }

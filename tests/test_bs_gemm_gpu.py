@@ -106,3 +106,50 @@ def test_noalloc_is_the_same(ctx, orc):
         ctx.dequant_matmul_noalloc(x, w, Q4_1, n, y=y)
         torch.cuda.synchronize()
         assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("scheme", list(NAMES), ids=lambda s: NAMES[s])
+def test_wide_rows_form(ctx, orc, monkeypatch, scheme):
+    """The form with 64-bit row offsets, on rows that do not need it."""
+    monkeypatch.setenv("RLXQ_BS", "0,0")
+    for mkn in ((17, 512, 33), (70, 1792, 200), (300, 1280, 129)):
+        announce(f"block-scaled 64-bit row offsets {NAMES[scheme]} {mkn}")
+        kern = _check(ctx, orc, scheme, *mkn)
+        assert kern == f"rlxq_bs_{NAMES[scheme]}_wide", kern
+
+
+@pytest.mark.parametrize("scheme", [Q8_0, Q6_K], ids=lambda s: NAMES[s])
+def test_rows_past_4_gb(orc, scheme):
+    """32 weight rows past 4 GB.  x is zero but for three stretches of K, so
+    that the bound above holds with those alone."""
+    import rlxq
+    import torch
+
+    m, n, k = 17, 32, 21 << 23 if scheme == Q6_K else 1 << 27
+    rb = orc.row_bytes(scheme, k)
+    assert 31 * rb >= 1 << 32
+    announce(f"block-scaled rows of {rb} bytes {NAMES[scheme]} k={k}")
+    seg = [(0, 2048), (k // 2 - 1024, k // 2 + 1024), (k - 2048, k)]
+    gen = torch.Generator(device="cuda").manual_seed(scheme)
+    # (bytes below 60: every f16 and int8 scale finite)
+    w = torch.randint(0, 60, (n, rb), device="cuda", dtype=torch.uint8, generator=gen)
+    x = torch.zeros((m, k), device="cuda")
+    for a, b in seg:
+        x[:, a:b] = torch.randn((m, b - a), device="cuda", generator=gen)
+    c = rlxq.Context(0)
+    try:
+        y = c.dequant_matmul(x, w.view(-1), scheme, n)
+        kern = c.last_kernel
+        torch.cuda.synchronize()
+    finally:
+        c.close()
+    xs = torch.cat([x[:, a:b] for a, b in seg], 1).cpu().numpy().astype(np.float64)
+    wd = np.concatenate([orc.dequantize(scheme, w[:, orc.row_bytes(scheme, a) if a else 0:orc.row_bytes(scheme, b)]
+                                        .cpu().numpy(), b - a).astype(np.float64) for a, b in seg], 1)
+    want = xs @ wd.T
+    ks = wd.shape[1]
+    wmax = np.repeat(np.abs(wd).reshape(n, ks // 32, 32).max(2), 32, 1)
+    lim = (2.0 ** -21 + (ks / 32 + 8) * 2.0 ** -23) * (np.abs(xs) @ (3 * wmax).T)
+    got = y.double().cpu().numpy()
+    assert np.all(np.abs(got - want) <= lim), (kern, float(np.max(np.abs(got - want) / lim)))
+    assert kern == f"rlxq_bs_{NAMES[scheme]}_wide", kern
