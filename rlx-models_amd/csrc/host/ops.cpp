@@ -447,13 +447,14 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
 
   if (mf_applies(scheme, group, xbf, m, k, n, rb)) {
     // rows per launch: all of them, or two where four rows' fragments do not
-    // fit the LDS (f32 past K = 8192, bf16 past 18432)
+    // fit the LDS (f32 past K = 8192, bf16 past 16128)
     const bool has_m = scheme == RLXQ_GGUF_Q4_1 || scheme == RLXQ_GGUF_Q4_K || scheme == RLXQ_MLX_AFFINE4;
     const int64_t row_lds = scheme == RLXQ_GGUF_Q4_1 ? 176 : scheme == RLXQ_GGUF_Q8_0 ? 272
                             : scheme == RLXQ_GGUF_Q6_K ? 240 : 144;   // a weight row's unit in LDS
     auto lds_bytes = [&](int64_t mr) {
-      const int64_t fs = xbf ? mr : 2 * mr, ms = mr > 2 ? mr : fs;   // fragments and sums per block
-      return (size_t)((k / 32 + 8) * 64 * fs + (has_m ? (k / 32) * 4 * ms : 0) + 4096 + 8 * 16 * row_lds);
+      // fragments, and dwords of the record, per block
+      const int64_t fs = xbf ? mr : 2 * mr, rec = (mr == 4 ? 1 : mr) + (has_m ? mr : 0);
+      return (size_t)((k / 32 + 8) * 64 * fs + (k / 32) * 4 * rec + 4096 + 8 * 16 * row_lds);
     };
     int64_t mr = m <= 2 ? m : 4;
     if (mr == 4 && lds_bytes(mr) > ctx->max_lds) mr = 2;

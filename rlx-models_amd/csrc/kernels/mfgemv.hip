@@ -109,8 +109,8 @@ RLXQ_DEV void mf_read(const uint8_t* rp, int g, uint32_t off, MfRaw<SCH>& r) {
   }
 }
 
-// Lane exchanges on the VALU: v of the lane's 16-lane row rotated by n, of lane
-// ^ 1 and ^ 2 (quad permutations), and sums / maxima with lanes ^ 16, ^ 32.
+// Lane exchanges on the VALU: v of lane ^ 1 and ^ 2 (quad permutations), and
+// sums with lanes ^ 16, ^ 32.
 template <int ctrl>
 RLXQ_DEV float mf_dpp(float v) {
   return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v), ctrl, 0xf, 0xf, true));
@@ -152,9 +152,42 @@ RLXQ_DEV f16x8_t mf_codes(const MfRaw<SCH>& r) {
   return f16x8_t{w[0].x, w[0].y, w[1].x, w[1].y, w[2].x, w[2].y, w[3].x, w[3].y};
 }
 
+// A block's record in LDS: the inverse of each row's scale, a power of two,
+// and for formats with a min / bias each row's sum.  One and two rows: MR (2
+// MR) f32; four: the exponents as the bytes of a dword, and the sums in an
+// array of their own behind those (four f32 rows then still fit the LDS at K =
+// 8192).
+template <int MR, bool HM> constexpr int mf_rec() { return MR == 4 ? 1 : HM ? 2 * MR : MR; }   // dwords
+template <int MR, bool HM>
+RLXQ_DEV void mf_record(const uint32_t* recs, const float* sums, int blk, float (&inv)[MR], float (&sum)[MR]) {
+  const uint32_t* p = recs + blk * mf_rec<MR, HM>();
+  if constexpr (MR == 4) {
+    const uint32_t e = *p;
+#pragma unroll
+    for (int r = 0; r < 4; r++) inv[r] = __uint_as_float((r < 3 ? e << (23 - 8 * r) : e >> 1) & 0x7f800000u);
+    if constexpr (HM) {
+      const f32x4_t v = *reinterpret_cast<const f32x4_t*>(sums + 4 * blk);
+#pragma unroll
+      for (int r = 0; r < 4; r++) sum[r] = v[r];
+    }
+  } else if constexpr (mf_rec<MR, HM>() == 1) {
+    inv[0] = __uint_as_float(*p);
+  } else if constexpr (mf_rec<MR, HM>() == 2) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    inv[0] = __uint_as_float(v.x);
+    (HM ? sum[0] : inv[MR - 1]) = __uint_as_float(v.y);
+  } else {
+    const u32x4_t v = *reinterpret_cast<const u32x4_t*>(p);
+    inv[0] = __uint_as_float(v[0]);
+    inv[1] = __uint_as_float(v[1]);
+    sum[0] = __uint_as_float(v[2]);
+    sum[1] = __uint_as_float(v[3]);
+  }
+}
+
 // LDS: x fragments [K / 32][4][MS NH] of 16 bytes, 8 * 4 * MS NH zero
-// fragments' worth, block sums [K / 32][MS] f32 (formats with a min / bias),
-// partial sums [2][8 waves][64] f32, then the waves' weight regions.
+// fragments' worth, the blocks' records, partial sums [2][8 waves][64] f32,
+// then the waves' weight regions.
 template <int SCH, bool XBF, int MR, int D>
 RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
   constexpr int W = 8;
@@ -164,14 +197,16 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
   constexpr int SEG = mf_seg<SCH>(), PPR = SEG / 16, LROW = mf_lrow<SCH>(), ORD = mf_order<SCH>();
   constexpr int NP = 16 * PPR, NL = (NP + 63) / 64;
   constexpr bool HM = mf_has_m<SCH>(), MLX = SCH == SCH_MLX4, Q6 = SCH == SCH_Q6_K;
+  constexpr int RF = mf_rec<MR, HM>();
   extern __shared__ __align__(16) uint8_t mf_lds[];
   const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int j = lane & 15, g = lane >> 4;
   const int K = a.K, nu = K / 256, nblk = K / 32;
   uint8_t* xs = mf_lds;
   uint8_t* zs = xs + nblk * 64 * FS;
-  float* sums = reinterpret_cast<float*>(zs + 8 * 64 * FS);
-  float* red = sums + (HM ? nblk * MS : 0);
+  uint32_t* recs = reinterpret_cast<uint32_t*>(zs + 8 * 64 * FS);
+  float* sums = reinterpret_cast<float*>(recs + nblk * RF);
+  float* red = sums + (MR == 4 && HM ? 4 * nblk : 0);
   uint8_t* reg = reinterpret_cast<uint8_t*>(red + 2 * W * 64) + wv * (16 * LROW);
 
   // the wave's units of every tile of 16 weight rows (the last tile ends with
@@ -235,11 +270,17 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
     if (++lu == cnt) lu = 0, lt += gridDim.x;
   };
 
-  // The activation rows over the wave's own units: maxima, then f16 fragments
-  // (each row scaled by the power of two that puts its maximum there in [2^9,
-  // 2^10)) and block sums.  Piece p: positions 8 (p % 4) .. of block p / 4 in
-  // code order (natural, GGUF nibbles, MLX nibbles).  A wave reads only what
-  // it wrote: no barrier before the first tile's end.
+  // The activation rows over the wave's own units as f16 fragments, each
+  // block of 32 scaled by the power of two that puts its maximum in [2^14,
+  // 2^15): what a block keeps does not depend on the others', and within it an
+  // element loses bits only 2^-17 below the maximum (f32, of 22) or 2^-31
+  // (bf16).  (One power of two for a wave's whole stretch: what lies 2^-24
+  // below its largest element kept ten bits, though that element may meet
+  // zero weights alone.  The scale per block costs Q6_K 3 to 5%, 4096->24576
+  // with one f32 row 23.8 -> 24.6 us, and the others up to 2%.)  Piece p: positions 8 (p % 4) .. of block p / 4 in
+  // code order (natural, GGUF nibbles, MLX nibbles); a block's four pieces are
+  // four neighbouring lanes.  A wave reads only what it wrote: no barrier
+  // before the first tile's end.
   const int p0 = u0 * 32, p1 = (u0 + cnt) * 32;
   struct Piece { uint32_t w[XBF ? 4 : 8]; };   // as read (bf16 pairs or f32)
   auto ldx = [&](int row, int p) {
@@ -259,13 +300,11 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
     }
     return v;
   };
-  float inv[MR];
   {
-    // Each lane's first NV pieces of a row stay in registers, and are asked
-    // for ahead of the weights: loads return in order.
+    // Each lane's first NV pieces of a row are asked for ahead of the weights:
+    // loads return in order.
     constexpr int NV = XBF || MR <= 2 ? 3 : 1;
     Piece v0[NV][MR];
-    float mx[MR];
 #pragma unroll
     for (int q = 0; q < NV; q++)
       if (p0 + 64 * q < p1) {
@@ -274,99 +313,75 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
         for (int r = 0; r < MR; r++) v0[q][r] = ldx(r, p);
       }
     static_for<D>([&](auto Q) { load(Q); });
-#pragma unroll
-    for (int r = 0; r < MR; r++) mx[r] = 0.f;
-    // bf16: the magnitudes' maximum per half, as integers
-    typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
-    u16x2_t mh[MR];
-#pragma unroll
-    for (int r = 0; r < MR; r++) mh[r] = u16x2_t{0, 0};
-    auto take = [&](int r, const Piece& v) {
+    for (int p = lane; p < 8 * 4 * FS; p += 64) *reinterpret_cast<u32x4_t*>(zs + 16 * p) = u32x4_t{0u, 0u, 0u, 0u};
+    auto put = [&](int r, int p, const Piece& v) {
+      float mx = 0.f;
       if constexpr (XBF) {
+        // (as integers: a NaN's bits are above every number's)
+        typedef uint16_t u16x2_t __attribute__((ext_vector_type(2)));
+        u16x2_t mh = {0, 0};
 #pragma unroll
         for (int e = 0; e < 4; e++)
-          mh[r] = __builtin_elementwise_max(mh[r], __builtin_bit_cast(u16x2_t, v.w[e] & 0x7fff7fffu));
+          mh = __builtin_elementwise_max(mh, __builtin_bit_cast(u16x2_t, v.w[e] & 0x7fff7fffu));
+        const uint32_t h = mh.x > mh.y ? mh.x : mh.y;
+        mx = __uint_as_float(h > 0x7f80u ? 0x7f800000u : h << 16);
       } else {
 #pragma unroll
-        for (int e = 0; e < 8; e++) mx[r] = fmaxf(mx[r], fabsf(__uint_as_float(v.w[e])));
+        for (int e = 0; e < 8; e++) mx = fmaxf(mx, fabsf(__uint_as_float(v.w[e])));
+      }
+      mx = fmaxf(mx, mf_dpp<0xB1>(mx));
+      mx = fmaxf(mx, mf_dpp<0x4E>(mx));
+      // (by exponent; a block that is not finite stays as it is)
+      const uint32_t ex = __float_as_uint(mx) >> 23;
+      int sh = 141 - (int)ex;
+      sh = ex >= 255u ? 0 : (sh > 126 ? 126 : sh);
+      const float s = __uint_as_float((uint32_t)(127 + sh) << 23), inv = __uint_as_float((uint32_t)(127 - sh) << 23);
+      uint32_t hi[4], lo[4];
+      float th = 0.f, tl = 0.f;
+      const f16x2_t one = {(_Float16)1.f, (_Float16)1.f};
+      float w[8];
+#pragma unroll
+      for (int e = 0; e < 8; e++) {
+        const int q = ORD == 2 ? (e < 4 ? 2 * e : 2 * (e - 4) + 1) : e;
+        if constexpr (XBF) w[e] = __uint_as_float(q & 1 ? v.w[q / 2] & 0xffff0000u : v.w[q / 2] << 16) * s;
+        else w[e] = __uint_as_float(v.w[q]) * s;
+      }
+#pragma unroll
+      for (int e = 0; e < 4; e++) {
+        const uint32_t h0 = f32_to_f16_bits(w[2 * e]), h1 = f32_to_f16_bits(w[2 * e + 1]);
+        hi[e] = h0 | (h1 << 16);
+        if constexpr (HM) th = __builtin_amdgcn_fdot2(as_h2(hi[e]), one, th, false);
+        if constexpr (!XBF) {
+          // (the remainder is exact in f32; rounded once more)
+          const uint32_t l0 = f32_to_f16_bits(w[2 * e] - f16_bits_to_f32(h0));
+          const uint32_t l1 = f32_to_f16_bits(w[2 * e + 1] - f16_bits_to_f32(h1));
+          lo[e] = l0 | (l1 << 16);
+          if constexpr (HM) tl = __builtin_amdgcn_fdot2(as_h2(lo[e]), one, tl, false);
+        }
+      }
+      *reinterpret_cast<u32x4_t*>(xs + (p * FS + r) * 16) = u32x4_t{hi[0], hi[1], hi[2], hi[3]};
+      if constexpr (!XBF) *reinterpret_cast<u32x4_t*>(xs + (p * FS + MR + r) * 16) = u32x4_t{lo[0], lo[1], lo[2], lo[3]};
+      // (all four lanes of a block store its record)
+      const int blk = p >> 2;
+      if constexpr (MR == 4) reinterpret_cast<uint8_t*>(recs + blk)[r] = (uint8_t)(127 - sh);
+      else recs[blk * RF + r] = __float_as_uint(inv);
+      if constexpr (HM) {
+        float t = th + tl;
+        t += mf_dpp<0xB1>(t);
+        t += mf_dpp<0x4E>(t);
+        if constexpr (MR == 4) sums[4 * blk + r] = t * inv;
+        else recs[blk * RF + MR + r] = __float_as_uint(t * inv);
       }
     };
 #pragma unroll
     for (int q = 0; q < NV; q++)
-      if (p0 + 64 * q < p1) {
+      if (p0 + 64 * q + lane < p1) {
 #pragma unroll
-        for (int r = 0; r < MR; r++) take(r, v0[q][r]);
+        for (int r = 0; r < MR; r++) put(r, p0 + 64 * q + lane, v0[q][r]);
       }
     for (int p = p0 + 64 * NV + lane; p < p1; p += 64)
 #pragma unroll
-      for (int r = 0; r < MR; r++) take(r, ldx(r, p));
-    for (int p = lane; p < 8 * 4 * FS; p += 64) *reinterpret_cast<u32x4_t*>(zs + 16 * p) = u32x4_t{0u, 0u, 0u, 0u};
-#pragma unroll
-    for (int r = 0; r < MR; r++) {
-      if constexpr (XBF) {
-        const uint32_t h = mh[r].x > mh[r].y ? mh[r].x : mh[r].y;
-        // (a NaN's bits are above every number's, and fmaxf would drop it)
-        mx[r] = __uint_as_float(h > 0x7f80u ? 0x7f800000u : h << 16);
-      }
-      mx[r] = fmaxf(mx[r], mf_dpp<0x128>(mx[r]));   // (row_ror 8, 4, 2, 1)
-      mx[r] = fmaxf(mx[r], mf_dpp<0x124>(mx[r]));
-      mx[r] = fmaxf(mx[r], mf_dpp<0x122>(mx[r]));
-      mx[r] = fmaxf(mx[r], mf_dpp<0x121>(mx[r]));
-      mx[r] = mf_rows(mx[r], [](float p, float q) { return fmaxf(p, q); });
-      // (by exponent; a zero row and one that is not finite stay as they are)
-      const uint32_t ex = __float_as_uint(mx[r]) >> 23;
-      int sh = 136 - (int)ex;
-      sh = sh > 126 ? 126 : sh;
-      if (mx[r] == 0.f || ex >= 255u) sh = 0;
-      const float s = __uint_as_float((uint32_t)(127 + sh) << 23);
-      inv[r] = __uint_as_float((uint32_t)(127 - sh) << 23);
-      auto put = [&](int p, const Piece& v) {
-        uint32_t hi[4], lo[4];
-        float th = 0.f, tl = 0.f;
-        const f16x2_t one = {(_Float16)1.f, (_Float16)1.f};
-        float w[8];
-#pragma unroll
-        for (int e = 0; e < 8; e++) {
-          const int q = ORD == 2 ? (e < 4 ? 2 * e : 2 * (e - 4) + 1) : e;
-          if constexpr (XBF) w[e] = __uint_as_float(q & 1 ? v.w[q / 2] & 0xffff0000u : v.w[q / 2] << 16) * s;
-          else w[e] = __uint_as_float(v.w[q]) * s;
-        }
-#pragma unroll
-        for (int e = 0; e < 4; e++) {
-          const uint32_t h0 = f32_to_f16_bits(w[2 * e]), h1 = f32_to_f16_bits(w[2 * e + 1]);
-          hi[e] = h0 | (h1 << 16);
-          if constexpr (HM) th = __builtin_amdgcn_fdot2(as_h2(hi[e]), one, th, false);
-          if constexpr (!XBF) {
-            // (the remainder is exact in f32; rounded once more)
-            const uint32_t l0 = f32_to_f16_bits(w[2 * e] - f16_bits_to_f32(h0));
-            const uint32_t l1 = f32_to_f16_bits(w[2 * e + 1] - f16_bits_to_f32(h1));
-            lo[e] = l0 | (l1 << 16);
-            if constexpr (HM) tl = __builtin_amdgcn_fdot2(as_h2(lo[e]), one, tl, false);
-          }
-        }
-        *reinterpret_cast<u32x4_t*>(xs + (p * FS + r) * 16) = u32x4_t{hi[0], hi[1], hi[2], hi[3]};
-        if constexpr (!XBF) *reinterpret_cast<u32x4_t*>(xs + (p * FS + MR + r) * 16) = u32x4_t{lo[0], lo[1], lo[2], lo[3]};
-        if constexpr (HM) {
-          // the block's four pieces are four neighbouring lanes, which all
-          // store their sum
-          auto sum = [&](float t, int slot) {
-            t += mf_dpp<0xB1>(t);
-            t += mf_dpp<0x4E>(t);
-            sums[(p >> 2) * MS + slot] = t;
-          };
-          if constexpr (MS == MR) {
-            sum(th + tl, r);
-          } else {
-            sum(th, r);
-            sum(tl, MR + r);
-          }
-        }
-      };
-#pragma unroll
-      for (int q = 0; q < NV; q++)
-        if (p0 + 64 * q + lane < p1) put(p0 + 64 * q + lane, v0[q][r]);
-      for (int p = p0 + 64 * NV + lane; p < p1; p += 64) put(p, ldx(r, p));
-    }
+      for (int r = 0; r < MR; r++) put(r, p, ldx(r, p));
     // (the lanes' reads below cross lanes: not before these stores, some of
     // which are conditional)
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -444,19 +459,21 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
           s = f16_bits_to_f32(r.h[0] & 0xffffu) * (float)((sc >> sh) & 0xffu);
           m = -f16_bits_to_f32(r.h[0] >> 16) * (float)((mn >> sh) & 0xffu);
         }
+        // lane group g's block: 8u + 2g + b (Q6_K: as its codes)
+        float inv[MR], sum[MR];
+        mf_record<MR, HM>(recs, sums, 8 * u + (Q6 ? 4 * (g >> 1) + (g & 1) : 2 * g) + B1 * b, inv, sum);
         if constexpr (Q6) {
           const float d = f16_bits_to_f32(r.h[2]);
           const float s0 = d * (float)(int8_t)(r.h[b] & 0xffu), s1 = d * (float)(int8_t)(r.h[b] >> 8);
 #pragma unroll
-          for (int q = 0; q < MS; q++) acc[q] = fmaf(s1, t[1][q], fmaf(s0, t[0][q], acc[q]));
+          for (int q = 0; q < MS; q++) acc[q] = fmaf(inv[q % MR], fmaf(s1, t[1][q], s0 * t[0][q]), acc[q]);
         } else {
 #pragma unroll
-          for (int q = 0; q < MS; q++) acc[q] = fmaf(s, t[0][q], acc[q]);
+          for (int q = 0; q < MS; q++) acc[q] = fmaf(s * inv[q % MR], t[0][q], acc[q]);
         }
         if constexpr (HM) {
-          const float* sp = sums + (8 * u + 2 * g + b) * MS;
 #pragma unroll
-          for (int q = 0; q < MS; q++) acc[q] = fmaf(m, sp[q], acc[q]);
+          for (int q = 0; q < MR; q++) acc[q] = fmaf(m, sum[q], acc[q]);
         }
       });
       if (++cu == cnt) {
@@ -466,7 +483,7 @@ RLXQ_DEV void mf_body(const rlxq_gemv_args& a) {
         // follows this one's reads.)
         cu = 0;
 #pragma unroll
-        for (int q = 0; q < MS; q++) acc[q] = mf_rows(acc[q], [](float p, float q) { return p + q; }) * inv[q % MR];
+        for (int q = 0; q < MS; q++) acc[q] = mf_rows(acc[q], [](float p, float q) { return p + q; });
         float v = acc[0];
 #pragma unroll
         for (int q = 1; q < MS; q++) v = g == q ? acc[q] : v;

@@ -4,12 +4,12 @@ divide over the waves, weight rows that end inside a tile, the rows of a tile
 per launch, and rows of very different size.
 
 Bound per output, f32 rows: the hi + lo f16 split keeps each element to 2^-22
-of itself or 2^-34 of the row's maximum, and each of the K / 32 block results
-is rounded a few times in f32 on its way into the sum, so |error| <= (2^-21 +
-(K / 32 + 8) 2^-23) sum_k (|x_k| + 2^-13 max|x|) 3 W_k, W_k the largest weight
-of k's block of 32 (scale * code and the min / bias are each at most three
-times that in the synthetic rows).  bf16 rows are exact in f16 above the same
-share of the maximum; their sums round alike."""
+of itself or 2^-39 of B_k, the largest |x| of k's block of 32, and each of the
+K / 32 block results is rounded a few times in f32 on its way into the sum, so
+|error| <= (2^-21 + (K / 32 + 8) 2^-23) sum_k (|x_k| + 2^-18 B_k) 3 W_k, W_k
+the largest weight of the block (scale * code and the min / bias are each at
+most three times that in the synthetic rows).  bf16 rows are exact in f16 above
+2^-31 of B_k, and 2^-39 of it off below; their sums round alike."""
 import numpy as np
 import pytest
 
@@ -21,7 +21,7 @@ pytestmark = pytest.mark.gpu
 SCHEMES = [Q8_0, Q4_1, MLX4, Q4_K, Q6_K]
 
 
-def _check(ctx, orc, scheme, m, k, n, bf16, y_dtype=None):
+def _check(ctx, orc, scheme, m, k, n, bf16, y_dtype=None, change=None):
     import torch
 
     rng = np.random.default_rng(m * 11 + k + n * 5 + scheme)
@@ -30,6 +30,8 @@ def _check(ctx, orc, scheme, m, k, n, bf16, y_dtype=None):
     x[0] *= 1e-6
     x[m // 2] *= 3e4
     x[m - 1, ::3] = 0.0
+    if change:
+        change(x, w, sc, bi, wd)
     xt = _t(x).to(torch.bfloat16) if bf16 else _t(x)
     x = xt.float().cpu().numpy().astype(np.float64)
     y = ctx.dequant_matmul(xt, w, scheme, n, group=group, scales=sc, biases=bi, y_dtype=y_dtype or torch.float32)
@@ -37,7 +39,7 @@ def _check(ctx, orc, scheme, m, k, n, bf16, y_dtype=None):
     torch.cuda.synchronize()
     want = x @ wd.T
     wmax = np.repeat(np.abs(wd).reshape(n, k // 32, 32).max(2), 32, 1)
-    xa = np.abs(x) + 2.0 ** -13 * np.abs(x).max(1, keepdims=True)
+    xa = np.abs(x) + 2.0 ** -18 * np.repeat(np.abs(x).reshape(m, k // 32, 32).max(2), 32, 1)
     lim = (2.0 ** -21 + (k / 32 + 8) * 2.0 ** -23) * (xa @ (3 * wmax).T)
     if y_dtype is not None:
         lim = lim + np.abs(want) * 2.0 ** -8   # one rounding to bf16
@@ -71,6 +73,36 @@ def test_rows_in_pairs_and_defaults(ctx, orc, scheme):
         assert "_mf2_F" in kern, kern
     for m, k, n in ((2, 1536, 64), (2, 4096, 15)) + (((2, 2176, 64),) if scheme in (Q8_0, Q4_1, MLX4) else ()):
         assert "_mf" not in _check(ctx, orc, scheme, m, k, n, True), (m, k, n)
+
+
+@pytest.mark.parametrize("scheme", SCHEMES, ids=lambda s: NAMES[s])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_large_elements_on_zero_weights(ctx, orc, monkeypatch, scheme, bf16):
+    """Elements 2^30 times the others, where every weight is zero, take
+    nothing from the rest: not from the blocks of their own 256 (but for their
+    own block of 32, whose weights are zero in the formats that have a scale
+    for it alone) nor from the same wave's next 256."""
+    monkeypatch.setenv("RLXQ_GEMV_MF", "1")
+    k, n = 6144, 48
+    unit = scheme in (Q4_K, Q6_K)   # (a scale, and so zeros, for 256 weights)
+
+    def change(x, w, sc, bi, wd):
+        for u in range(0, k // 256, 3):   # every wave has three units
+            a, b = 256 * u + 64, 256 * u + (256 if unit else 128)
+            a -= 64 if unit else 0
+            x[:, a:b] *= 2.0 ** 30
+            wd[:, a:b] = 0.0
+            if sc is not None:
+                sc[:, a // 64:b // 64] = 0.0
+                bi[:, a // 64:b // 64] = 0.0
+            else:
+                rows = w.view(n, -1)
+                rows[:, orc.row_bytes(scheme, a) if a else 0:orc.row_bytes(scheme, b)] = 0
+
+    for m in (1, 2, 4):
+        announce(f"matrix-core decode, large elements on zero weights {NAMES[scheme]} m={m} bf16={bf16}")
+        kern = _check(ctx, orc, scheme, m, k, n, bf16, change=change)
+        assert "_mf" in kern, kern
 
 
 def test_a_row_that_is_not_finite_stays_alone(ctx, orc):
