@@ -59,7 +59,7 @@ int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream) {
 }
 
 int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
-                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, const char* gemm_name) {
+                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, bool prefill) {
   const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
   const int64_t nu = (k + 255) / 256;   // 256-element units
   // 64-row tiles past 32 rows (197 rows of Q4_K, 4096->24576: 131 us in four
@@ -70,18 +70,18 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   const int64_t r32 = (m + 31) / 32;
   // (32 weight rows past 4 GB: the form with 64-bit row offsets)
   bool wide = rb >= ((int64_t)1 << 27);
-  int RT = gemm_name || m > 32 ? 2 : 1;
+  int RT = m > 32 ? 2 : 1;
   int64_t want = 0;
   if (const char* e = std::getenv("RLXQ_BS")) {
     int a1, a2;
     if (std::sscanf(e, "%d,%d", &a1, &a2) == 2 && a1 >= 0 && a1 <= 2) {
       want = a2;
       if (a1 == 0) wide = true;
-      else if (!gemm_name) RT = a1;
+      else RT = a1;
     }
   }
   if (wide) RT = 1;
-  if (gemm_name)
+  if (prefill)
     if (const char* e = std::getenv("RLXQ_GEMM_SPLITS")) want = std::max(1, std::atoi(e));
   const int64_t tiles_m = (m + 32 * RT - 1) / (32 * RT), tiles_n = (n + 127) / 128;
   const int64_t rtiles = tiles_m * RT;
@@ -163,9 +163,7 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   a.sb_bf16 = sb.sb_bf16;
   char name[64];
   if (wide) std::snprintf(name, sizeof name, "rlxq_bs_%s_wide", scheme_name(scheme));
-  else if (gemm_name) std::snprintf(name, sizeof name, "%s", gemm_name);
-  else std::snprintf(name, sizeof name, "rlxq_skinny%s_%s_bs_rt%d", scheme == RLXQ_GGUF_Q5_K ? "xr" : "ns",
-                     scheme_name(scheme), RT);
+  else std::snprintf(name, sizeof name, "rlxq_bs_%s_rt%d", scheme_name(scheme), RT);
   if ((rc = get_fn(ctx, name, &fn))) return rc;
   void* args[] = {&a};
   // three activation slots (two 32-element blocks each), the waves' weight

@@ -194,7 +194,8 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   // two for the others.
   const bool split = x_dtype == RLXQ_F32;
   const bool want_exact = split || y_dtype == RLXQ_F32;
-  // (the "...xs" kernels take f32 activations as hi / lo x16 rows)
+  // (the "...xs" kernels take f32 activations as hi / lo x16 rows: Q3_K, Q2_K,
+  // Q8_K; the other formats' f32 calls go to the block-scaled matmul below)
   std::string vs = var;
   if (!te && want_exact && has_exact_gemm(scheme))
     vs = scheme == RLXQ_GGUF_Q6_K ? "w8lx"
@@ -242,16 +243,17 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   }
   const int64_t kslice = ((ksteps + splits - 1) / splits) * 64;
   splits = (k + kslice - 1) / kslice;
-  char name[64];
-  std::snprintf(name, sizeof name, "rlxq_gemm_%s_t%d%s", scheme_name(scheme), tile, vs.c_str());
+  // (f32 activations, formats of bs_scheme: the block-scaled matmul)
   if (split && bs_scheme(scheme)) {
     SkinnySb sb;
     sb.scales = scales;
     sb.biases = biases;
     sb.group = is_mlx(scheme) ? group : 32;
     sb.sb_bf16 = sb_code(sb_dtype);
-    return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, name);
+    return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, true);
   }
+  char name[64];
+  std::snprintf(name, sizeof name, "rlxq_gemm_%s_t%d%s", scheme_name(scheme), tile, vs.c_str());
   hipFunction_t fn;
   int rc;
   if ((rc = get_fn(ctx, name, &fn))) return rc;
@@ -404,13 +406,14 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   // scaled; f32 activations run as hi + lo row pairs (~22 significant bits).
   // (f32 activations past 16 rows, formats of bs_scheme: the block-scaled
   // matmul.  Q4_1 4096->24576 at 64 rows 90 us here, 51 there.)
-  // RLXQ_DECODE=gemv|skinny forces one where both apply.
+  // RLXQ_DECODE=gemv|skinny forces one where both apply (skinny: also ahead of
+  // the block-scaled matmul).
   {
     const bool sk_ok = skinny_applies(scheme, group, sb_dtype, m, k);
-    bool use_sk = sk_ok && m >= 5;
+    bool use_sk = sk_ok && m >= 5, use_bs = !xbf && m > 16 && bs_scheme(scheme);
     if (const char* e = std::getenv("RLXQ_DECODE")) {
       if (!std::strcmp(e, "gemv")) use_sk = false;
-      if (!std::strcmp(e, "skinny")) use_sk = sk_ok;
+      if (!std::strcmp(e, "skinny")) use_sk = sk_ok, use_bs = false;
     }
     if (use_sk) {
       SkinnySb sb;
@@ -418,9 +421,9 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
       sb.biases = biases;
       sb.group = is_mlx(scheme) ? group : 32;
       sb.sb_bf16 = sb_code(sb_dtype);
-      if (!xbf && m > 16 && bs_scheme(scheme) && !std::getenv("RLXQ_SKINNY_XR") && !std::getenv("RLXQ_SKINNY_NS") &&
+      if (use_bs && !std::getenv("RLXQ_SKINNY_XR") && !std::getenv("RLXQ_SKINNY_NS") &&
           !std::getenv("RLXQ_SKINNY_XL"))
-        return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, nullptr);
+        return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, false);
       return skinny_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb);
     }
   }

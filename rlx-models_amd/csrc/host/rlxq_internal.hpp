@@ -158,13 +158,14 @@ int sk_post_exp(int scheme);
 int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
                     int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb = SkinnySb());
 // Block-scaled MFMA matmul (f32 activations): its formats, and the call.
-// gemm_name: kernel name for prefill sizes (more than 256 rows), else NULL.
+// prefill: a call of the exact GEMM's (more than 256 rows, or bf16 output),
+// whose tuning variables it obeys.
 bool bs_scheme(int scheme);
 int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream);
 int64_t bs_lds_row(int scheme);   // bytes of a weight row's unit in LDS
 int bs_order(int scheme);         // code order of its prepared activations
 int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
-                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, const char* gemm_name);
+                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, bool prefill);
 int i8b_dispatch(rlxq_ctx* ctx, int group, const void* x, int x_dtype, const void* w, const void* scales,
                  const void* zp, int sb_dtype, int64_t m, int64_t k, int64_t n, void* y, int y_dtype,
                  void* stream);

@@ -827,18 +827,17 @@ RLXQ_BS_PREP(rlxq_bs_prep2, 2)
 RLXQ_BS_PREP(rlxq_bs_prep8, 8)
 #endif
 
-// rlxq_skinnyns_<scheme>_bs_rt<RT> (Q5_K: skinnyxr, the batched kernel it has
-// besides): up to 256 rows; the prefill sizes run the 64-row form under the
-// exact GEMM's names.  rlxq_bs_<scheme>_wide: rows of 128 MB and more, whose
-// offsets take 64 bits (a register more per piece: the others stay on 32).
+// rlxq_bs_<scheme>_rt<RT>: 32 RT rows a workgroup.  rlxq_bs_<scheme>_wide:
+// rows of 128 MB and more, whose offsets take 64 bits (a register more per
+// piece: the others stay on 32).  rlxq_moesk_<scheme>_bs[_sw]: the grouped
+// form, with SwiGLU.
 #define RLXQ_BS_INST(NAME, SCH, RT, OFF)                                                       \
   extern "C" __global__ __launch_bounds__(256, 2) void NAME(rlxq_bs_args a) {                  \
     rlxq::bs_body<SCH, RT, 1, 2, OFF>(a);                                                      \
   }
-#define RLXQ_BS_SCHEME(SNAME, SCH, KIND, GEMM)                                                 \
-  RLXQ_BS_INST(rlxq_skinny##KIND##_##SNAME##_bs_rt1, SCH, 1, uint32_t)                          \
-  RLXQ_BS_INST(rlxq_skinny##KIND##_##SNAME##_bs_rt2, SCH, 2, uint32_t)                          \
-  RLXQ_BS_INST(GEMM, SCH, 2, uint32_t)                                                         \
+#define RLXQ_BS_SCHEME(SNAME, SCH)                                                             \
+  RLXQ_BS_INST(rlxq_bs_##SNAME##_rt1, SCH, 1, uint32_t)                                         \
+  RLXQ_BS_INST(rlxq_bs_##SNAME##_rt2, SCH, 2, uint32_t)                                         \
   RLXQ_BS_INST(rlxq_bs_##SNAME##_wide, SCH, 1, uint64_t)                                        \
   extern "C" __global__ __launch_bounds__(256, 2) void rlxq_moesk_##SNAME##_bs(rlxq_moe_sk_args a) { \
     rlxq::bs_moe_body<SCH, false>(a);                                                          \
@@ -848,21 +847,21 @@ RLXQ_BS_PREP(rlxq_bs_prep8, 8)
     rlxq::bs_moe_body<SCH, true>(a);                                                           \
   }
 #if RLXQ_PART_IS(0)
-RLXQ_BS_SCHEME(q4_1, SCH_Q4_1, ns, rlxq_gemm_q4_1_t256w8p2xs)
+RLXQ_BS_SCHEME(q4_1, SCH_Q4_1)
 RLXQ_BS_SW(q4_1, SCH_Q4_1)
-RLXQ_BS_SCHEME(mlx4, SCH_MLX4, ns, rlxq_gemm_mlx4_t256w8xs)
-RLXQ_BS_SCHEME(mlx8, SCH_MLX8, ns, rlxq_gemm_mlx8_t256w8p2xs)
+RLXQ_BS_SCHEME(mlx4, SCH_MLX4)
+RLXQ_BS_SCHEME(mlx8, SCH_MLX8)
 #endif
 #if RLXQ_PART_IS(1)
-RLXQ_BS_SCHEME(q4_0, SCH_Q4_0, ns, rlxq_gemm_q4_0_t256w8p2xs)
+RLXQ_BS_SCHEME(q4_0, SCH_Q4_0)
 RLXQ_BS_SW(q4_0, SCH_Q4_0)
 RLXQ_BS_SW(q8_0, SCH_Q8_0)
-RLXQ_BS_SCHEME(q8_0, SCH_Q8_0, ns, rlxq_gemm_q8_0_t256w8xs)
+RLXQ_BS_SCHEME(q8_0, SCH_Q8_0)
 #endif
 #if RLXQ_PART_IS(2)
-RLXQ_BS_SCHEME(q4_k, SCH_Q4_K, ns, rlxq_gemm_q4_k_t256w8p2xs)
+RLXQ_BS_SCHEME(q4_k, SCH_Q4_K)
 RLXQ_BS_SW(q4_k, SCH_Q4_K)
 RLXQ_BS_SW(q5_k, SCH_Q5_K)
-RLXQ_BS_SCHEME(q5_k, SCH_Q5_K, xr, rlxq_gemm_q5_k_t256w8xs)
-RLXQ_BS_SCHEME(q6_k, SCH_Q6_K, ns, rlxq_gemm_q6_k_t256w8lxs)
+RLXQ_BS_SCHEME(q5_k, SCH_Q5_K)
+RLXQ_BS_SCHEME(q6_k, SCH_Q6_K)
 #endif

@@ -66,7 +66,7 @@ def _check(ctx, orc, scheme, m, k, n, y_dtype=None):
 def test_batched(ctx, orc, scheme, mkn):
     announce(f"block-scaled {NAMES[scheme]} {mkn}")
     kern = _check(ctx, orc, scheme, *mkn)
-    assert f"_{NAMES[scheme]}_bs_rt" in kern, kern
+    assert kern == f"rlxq_bs_{NAMES[scheme]}_rt{2 if mkn[0] > 32 else 1}", kern
 
 
 @pytest.mark.parametrize("scheme,mkn", [(Q4_1, (300, 64 * 13, 301)), (Q4_0, (257, 64 * 5, 130)), (Q8_0, (259, 64 * 7, 33)),
@@ -80,7 +80,8 @@ def test_partial_units_and_prefill(ctx, orc, scheme, mkn, ydt):
     announce(f"block-scaled {NAMES[scheme]} {mkn} y={ydt}")
     if ydt == "bf16" and mkn[0] < 64:
         pytest.skip("bf16 output takes this kernel from 64 rows")
-    _check(ctx, orc, scheme, *mkn, y_dtype=torch.bfloat16 if ydt == "bf16" else None)
+    kern = _check(ctx, orc, scheme, *mkn, y_dtype=torch.bfloat16 if ydt == "bf16" else None)
+    assert kern == f"rlxq_bs_{NAMES[scheme]}_rt{2 if mkn[0] > 32 else 1}", kern
 
 
 @pytest.mark.parametrize("cfg", ["1,1", "1,3", "2,1", "2,5", "2,32"])
@@ -89,7 +90,7 @@ def test_row_tiles_and_splits(ctx, orc, monkeypatch, cfg):
     for scheme, mkn in ((Q4_1, (70, 1792, 200)), (Q4_K, (40, 2816, 129)), (Q6_K, (70, 1792, 133))):
         announce(f"block-scaled {cfg} {NAMES[scheme]} {mkn}")
         kern = _check(ctx, orc, scheme, *mkn)
-        assert kern.endswith(f"_{NAMES[scheme]}_bs_rt{cfg[0]}"), kern
+        assert kern == f"rlxq_bs_{NAMES[scheme]}_rt{cfg[0]}", kern
 
 
 def test_noalloc_is_the_same(ctx, orc):

@@ -3,10 +3,10 @@ activations in, F32 output (Op::DequantMatMul, crates/rlx-laguna/src/
 device_matmul.rs:358-377, crates/rlx-qwen3/src/precision.rs:98-112), exactly
 as rlxq_dm_matmul passes them.
 
-f32 activations run on the prefill GEMM and the batched-decode kernels as a
-hi and a lo f16 row per activation row (hi = f16(s*x), lo = f16(s*x - hi),
-~22 significant bits), whose sums the epilogue adds; the single-row register
-GEMV holds them as a hi and a lo bf16 row (~16 bits).  Bars: max|got - want|
+f32 activations run on the batched-decode kernels, the block-scaled matmul
+(from 17 rows and at prefill sizes) and the exact GEMM as a hi and a lo f16 row
+per activation row (hi = f16(s*x), lo = f16(s*x - hi), ~22 significant bits),
+whose sums are added; the single-row register GEMV holds them as a hi and a lo bf16 row (~16 bits).  Bars: max|got - want|
 / max|want| <= 1e-3 against the float64 oracle on the f32 activations
 themselves.  Where the weights are exact in f16 (Q4_1 with d a power of two
 and m = 0) the only error left is the activations' representation and the
@@ -16,7 +16,7 @@ tests/test_f32_split.py checks on the CPU."""
 import numpy as np
 import pytest
 
-from conftest import announce
+from conftest import announce, batched_f32_kernel
 from test_gemv_gpu import _t, rel_err
 
 pytestmark = pytest.mark.gpu
@@ -54,14 +54,15 @@ def _want(orc, scheme, x32, packed, k):
 @pytest.mark.parametrize("mkn", [(5, 1024, 96), (16, 4096, 384), (33, 768, 200), (64, 4096, 256),
                                  (256, 2048, 160)], ids=str)
 def test_batched_decode_f32_activations(ctx, orc, scheme, mkn):
-    """5..256 rows of f32 activations on the batched-decode MFMA kernels."""
+    """5..256 rows of f32 activations on the batched-decode MFMA kernels and
+    the block-scaled matmul."""
     m, k, n = mkn
     announce(f"f32 contract skinny {NAMES[scheme]} {mkn}")
     rng = np.random.default_rng(m + k + n + scheme)
     packed = orc.synth(scheme, rng, n, k)
     x = rng.standard_normal((m, k)).astype(np.float32)
     got, kern = _f32_run(ctx, scheme, x, _t(packed), n)
-    assert kern.startswith("rlxq_skinny"), kern
+    assert kern.startswith(batched_f32_kernel(scheme, m)), kern
     assert rel_err(got, _want(orc, scheme, x, packed, k)) <= TOL, kern
 
 
@@ -74,7 +75,7 @@ def test_batched_decode_f32_exact_weights(ctx, orc, mkn):
     packed = _exact_f16_q4_1(orc, rng, n, k)
     x = rng.standard_normal((m, k)).astype(np.float32)
     got, kern = _f32_run(ctx, Q4_1, x, _t(packed), n)
-    assert kern.startswith("rlxq_skinny"), kern
+    assert kern.startswith(batched_f32_kernel(Q4_1, m)), kern
     assert rel_err(got, _want(orc, Q4_1, x, packed, k)) <= TOL_EXACT_W, kern
 
 
@@ -105,7 +106,7 @@ def test_batched_decode_f32_mlx4_and_mxfp4(ctx, orc):
     sc = rng.uniform(0.01, 0.1, (n, k // 64)).astype(np.float32)
     bi = rng.uniform(-0.5, 0.1, (n, k // 64)).astype(np.float32)
     got, kern = _f32_run(ctx, MLX4, x, _t(wq.view(np.uint8)), n, group=64, scales=_t(sc), biases=_t(bi))
-    assert kern.startswith("rlxq_skinny"), kern
+    assert kern.startswith(batched_f32_kernel(MLX4, m)), kern
     assert rel_err(got, orc.mlx_matmul_f64(x, wq, sc, bi, n, 4, 64)) <= TOL
     mc, eb = orc.synth_mxfp4(rng, n, k)
     got, kern = _f32_run(ctx, MXFP4, x, _t(mc), n, scales=_t(eb))
@@ -117,16 +118,15 @@ def test_batched_decode_f32_mlx4_and_mxfp4(ctx, orc):
 @pytest.mark.parametrize("scheme", [Q4_1, Q4_K, Q8_0, Q6_K, Q4_0], ids=lambda s: NAMES[s])
 @pytest.mark.parametrize("mkn", [(300, 1280, 272), (512, 4096, 1024), (257, 12288, 300)], ids=str)
 def test_prefill_f32_activations(ctx, orc, scheme, mkn):
-    """More than 256 rows of f32 activations with f32 output: the exact GEMM
-    (f16 hi + lo weight rows) on hi/lo activation row pairs (split-K on the
-    small grids)."""
+    """More than 256 rows of f32 activations with f32 output: the block-scaled
+    matmul on hi/lo activation fragments (K split on the small grids)."""
     m, k, n = mkn
     announce(f"f32 contract gemm {NAMES[scheme]} {mkn}")
     rng = np.random.default_rng(m + k + scheme)
     packed = orc.synth(scheme, rng, n, k)
     x = rng.standard_normal((m, k)).astype(np.float32)
     got, kern = _f32_run(ctx, scheme, x, _t(packed), n)
-    assert kern.startswith(f"rlxq_gemm_{NAMES[scheme]}_t256w8") and kern.endswith("xs"), kern
+    assert kern == f"rlxq_bs_{NAMES[scheme]}_rt2", kern
     assert rel_err(got, _want(orc, scheme, x, packed, k)) <= TOL, kern
 
 
@@ -139,12 +139,12 @@ def test_prefill_f32_exact_weights_and_bf16_out(ctx, orc):
     packed = _exact_f16_q4_1(orc, rng, n, k)
     x = rng.standard_normal((m, k)).astype(np.float32)
     got, kern = _f32_run(ctx, Q4_1, x, _t(packed), n)
-    assert kern == "rlxq_gemm_q4_1_t256w8p2xs", kern
+    assert kern == "rlxq_bs_q4_1_rt2", kern
     want = _want(orc, Q4_1, x, packed, k)
     assert rel_err(got, want) <= TOL_EXACT_W
     # bf16 output from f32 activations: the same kernel, rounded at the store
     y = ctx.dequant_matmul(_t(x), _t(packed), Q4_1, n, y_dtype=torch.bfloat16)
-    assert ctx.last_kernel == "rlxq_gemm_q4_1_t256w8p2xs", ctx.last_kernel
+    assert ctx.last_kernel == "rlxq_bs_q4_1_rt2", ctx.last_kernel
     torch.cuda.synchronize()
     assert rel_err(y.float().cpu().numpy(), want) <= 8e-3
 
@@ -167,7 +167,7 @@ def test_prefill_f32_config4_full_size_sampled(ctx, orc, scheme, kn):
     y = ctx.dequant_matmul(x, w, scheme, n, y_dtype=torch.float32)
     kern = ctx.last_kernel
     torch.cuda.synchronize()
-    assert kern == f"rlxq_gemm_{NAMES[scheme]}_t256w8p2xs", kern
+    assert kern == f"rlxq_bs_{NAMES[scheme]}_rt2", kern
     rs = np.random.default_rng(m + n)
     rows = np.sort(rs.choice(m, 48, replace=False))
     cols = np.sort(rs.choice(n, 384, replace=False))
@@ -271,7 +271,7 @@ def test_f32_activation_range(ctx, orc):
         x[2, 7] = 3e5
         x[3] = 0.0
         got, kern = _f32_run(ctx, Q4_1, x, _t(packed), n)
-        assert kern.startswith("rlxq_skinny" if m == 8 else "rlxq_gemm_q4_1"), kern
+        assert kern.startswith("rlxq_skinny" if m == 8 else "rlxq_bs_q4_1"), kern
         want = _want(orc, Q4_1, x, packed, k)
         for r in range(m):
             if r == 3:
@@ -309,8 +309,9 @@ def test_reference_structured_inputs_every_path(ctx, orc, scheme, m, xdt):
     0.8 sin(0.031 i), W = 0.35 cos(0.017 i + 0.3), quantized) at K = 1792,
     where rounding each weight once to f16 already costs 1.4e-3 and
     rounding the activations alone 7e-4: every f32-output path (the register
-    GEMV at M=1, the batched-decode kernels from 5 rows, the exact prefill
-    GEMM past 256) stays within 5e-5, far inside the 1e-3 bar."""
+    GEMV at M=1, the batched-decode kernels from 5 rows, past 256 the exact
+    prefill GEMM, for f32 from 17 the block-scaled matmul) stays within 5e-5,
+    far inside the 1e-3 bar."""
     import torch
     from test_gemv_gpu import _ref_input, _ref_weight
 
@@ -323,8 +324,10 @@ def test_reference_structured_inputs_every_path(ctx, orc, scheme, m, xdt):
     y = ctx.dequant_matmul(xt, _t(packed), scheme, n, y_dtype=torch.float32)
     kern = ctx.last_kernel
     torch.cuda.synchronize()
-    if m >= 300:
-        assert kern.startswith(f"rlxq_gemm_{NAMES[scheme]}_t256") and kern.endswith("xs" if xdt == "f32" else "x"), kern
+    if xdt == "f32" and m > 16:
+        assert kern == f"rlxq_bs_{NAMES[scheme]}_rt2", kern
+    elif m >= 300:
+        assert kern.startswith(f"rlxq_gemm_{NAMES[scheme]}_t256") and kern.endswith("x"), kern
     elif m >= 5:
         assert kern.startswith("rlxq_skinny"), kern
     assert rel_err(y.cpu().numpy(), _want(orc, scheme, xv, packed, k)) <= 5e-5, kern

@@ -235,8 +235,8 @@ def test_gemm_split_k(ctx, orc, monkeypatch, scheme, tile_ydt, splits):
 @pytest.mark.parametrize("case", ["f32_x", "n_odd", "bf16_x_f32_y"])
 @pytest.mark.parametrize("splits", [2, 3])
 def test_gemm_split_k_reduction_layouts(ctx, orc, monkeypatch, case, splits):
-    """The split-K partial sums of each layout: F32 activations on the exact
-    variant (hi / lo x16 rows, m_out output rows), an N that is no multiple
+    """The split-K partial sums of each layout: F32 activations on the
+    block-scaled matmul, an N that is no multiple
     of 4 (one output per reduction thread), bf16 x with f32 y (the exact
     variant's 128 output columns), all with row and column tails: within the
     bar against the oracle and within 1e-5 of the unsplit kernel."""
@@ -255,7 +255,7 @@ def test_gemm_split_k_reduction_layouts(ctx, orc, monkeypatch, case, splits):
         if case == "f32_x":
             xt = _t(x)
             y = ctx.dequant_matmul(xt, _t(packed), 3, n, y_dtype=torch.float32)
-            assert ctx.last_kernel.endswith("xs"), ctx.last_kernel
+            assert ctx.last_kernel == "rlxq_bs_q4_1_rt2", ctx.last_kernel
         else:
             xt = _t(x).to(torch.bfloat16)
             y = ctx.dequant_matmul(xt, _t(packed), 3, n, y_dtype=torch.float32)

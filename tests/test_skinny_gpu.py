@@ -111,9 +111,9 @@ def test_skinny_every_register_variant(ctx, orc, monkeypatch, cfg):
 
 def test_f32_activations_take_the_skinny_kernels(ctx, orc, monkeypatch):
     """f32 activations (the reference's operand type) run on the f16 kernels
-    as hi and lo row pairs by default; RLXQ_DECODE=gemv keeps them on the
+    as hi and lo row pairs where RLXQ_DECODE=skinny asks for them (by default
+    32 rows take the block-scaled matmul); RLXQ_DECODE=gemv keeps them on the
     GEMV, whose products are exact."""
-    monkeypatch.delenv("RLXQ_DECODE", raising=False)
     rng = np.random.default_rng(3)
     packed = orc.synth_q4_1(rng, 256, 1024)
     x = rng.standard_normal((32, 1024)).astype(np.float32)
