@@ -30,6 +30,14 @@ int64_t bs_seg_bytes(int scheme) {
     default: return 0;
   }
 }
+// What a unit costs against Q4_1's (the codes' conversion and scales).
+double bs_unit_factor(int scheme) {
+  switch (scheme) {
+    case RLXQ_MLX_AFFINE4: return 1.4;
+    case RLXQ_GGUF_Q6_K: case RLXQ_MLX_AFFINE8: return 1.5;
+    default: return 1.0;
+  }
+}
 }  // namespace
 
 bool bs_scheme(int scheme) {
@@ -41,6 +49,14 @@ int64_t bs_lds_row(int scheme) {
   const int64_t seg = bs_seg_bytes(scheme);
   return (seg / 16) % 2 ? seg : seg + 16;
 }
+
+namespace {
+// LDS of the dense form: three activation slots (two 32-element blocks each),
+// the waves' weight regions.
+size_t bs_lds_bytes(int scheme, int RT) {
+  return (size_t)(3 * RT * 2) * 4096 + (size_t)(128 * bs_lds_row(scheme));
+}
+}  // namespace
 
 int bs_order(int scheme) { return scheme == RLXQ_GGUF_Q5_K ? 1 : sk_order(scheme); }
 
@@ -90,18 +106,23 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
     splits = std::min<int64_t>(want, nu);
   } else {
     // K splits by what the rounds of workgroups cost: a 64-row unit takes
-    // about 2.65 us per workgroup and CU (3.1 alone on the CU; 32-row ones
-    // 1.6 and 1.9), the reduction 3.5 us and the partial sums' traffic at
-    // about 5 TB/s.  At most 24 MiB of partial sums.  (64 rows of Q4_1:
-    // 4096->24576 four splits 51 us, none 56; 4096->4096 eight 21 us, four 23,
-    // sixteen 25.)
+    // about 2.65 us per workgroup and CU (3.1 alone on the CU) times the
+    // format's factor, a 32-row one 1.6 (1.9), the reduction 3.5 us and the
+    // partial sums' traffic at about 5 TB/s.  At most 24 MiB of partial sums.
+    // Over 180 shapes a format (K 512 to 12288, N 128 to 24576, 32 to 512 rows)
+    // the choice is 0.3 to 0.8% behind the best of the measured splits.  (One
+    // factor for all, and two workgroups a CU where the LDS holds one, Q8_0 and
+    // MLX 8 bit: up to 2%, at worst 22%, 256 rows of Q6_K 4096->8192, 97 us and
+    // 80.)
+    const double f = RT == 2 ? bs_unit_factor(scheme) : 1.0;
+    const bool two = 2 * bs_lds_bytes(scheme, RT) <= ctx->max_lds;
     double best = 1e30;
     for (int64_t t = 1; t <= 32 && t <= nu; t++) {
       const int64_t us = (nu + t - 1) / t, sp = (nu + us - 1) / us;
       if (sp != t || (t > 1 && t * m * n * 4 > ((int64_t)24 << 20))) continue;
       const int64_t per_cu = (tiles_m * tiles_n * t + cus - 1) / cus;
-      const double unit = RT == 2 ? (per_cu > 1 ? 2.65 : 3.1) : (per_cu > 1 ? 1.6 : 1.9);
-      const double cost = (double)(per_cu * us) * unit + (t > 1 ? 3.5 + (double)(t * m * n) * 8 / 5e6 : 0.0);
+      const double unit = RT == 2 ? (two && per_cu > 1 ? 2.65 : 3.1) : (two && per_cu > 1 ? 1.6 : 1.9);
+      const double cost = (double)(per_cu * us) * unit * f + (t > 1 ? 3.5 + (double)(t * m * n) * 8 / 5e6 : 0.0);
       if (cost < best) best = cost, splits = t;
     }
   }
@@ -166,9 +187,7 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   else std::snprintf(name, sizeof name, "rlxq_bs_%s_rt%d", scheme_name(scheme), RT);
   if ((rc = get_fn(ctx, name, &fn))) return rc;
   void* args[] = {&a};
-  // three activation slots (two 32-element blocks each), the waves' weight
-  // regions
-  const size_t lds = (size_t)(3 * RT * nh) * 4096 + (size_t)(128 * bs_lds_row(scheme));
+  const size_t lds = bs_lds_bytes(scheme, RT);
   if ((rc = launch(ctx, fn, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(256), lds, stream, args, name)))
     return rc;
   if (splits > 1) {
