@@ -58,6 +58,62 @@ size_t bs_lds_bytes(int scheme, int RT) {
 }
 }  // namespace
 
+// Whether f32 rows take the block-scaled matmul or the kernels it stands
+// beside: the batched-decode kernels (17 to 256 rows) and the exact GEMM
+// (prefill), which both pad K to 128 and 64 where this one takes whole
+// 256-element units, and start up faster.  T: its tiles (32 rows up to 32, 64
+// past them, by 128 columns), two of which share a CU (Q8_0 and MLX 8 bit: one).
+// us here / there, Q4_1 unless named; over 20800 batched and 6100 prefill
+// shapes (K 64 to 16384, N 64 to 24576) the rule is 0.1 to 0.5% behind the
+// faster of the two, this kernel alone 0.5 to 5%, prefill of Q8_0 and MLX 8 bit
+// 4 and 12%.  RLXQ_BS=0 turns it off, any other value on (bs_dispatch).
+bool bs_applies(int scheme, int64_t m, int64_t k, int64_t n, bool prefill) {
+  if (!bs_scheme(scheme)) return false;
+  // (the K-quants have no other kernel for f32 rows at prefill)
+  if (prefill && !is_gguf(scheme) && !is_mlx(scheme)) return true;
+  if (const char* e = std::getenv("RLXQ_BS")) return std::strcmp(e, "0") != 0;
+  const int64_t rows = m <= 32 ? 32 : 64, T = (m + rows - 1) / rows * ((n + 127) / 128);
+  const bool part = k % 256 != 0, mlx8 = scheme == RLXQ_MLX_AFFINE8, q8 = scheme == RLXQ_GGUF_Q8_0;
+  if (prefill) {
+    // long K and few columns: preparation alone (4096 rows of 12288->128: 266
+    // and 165), which re-reads rows past 4096 elements
+    if (k > 8192 && n <= 256 && m > 1024) return false;
+    // the exact GEMM's tiles of 128 rows, filled
+    const bool full = m <= 256 && m % 128 == 0;
+    if (mlx8) {
+      // one workgroup a CU: a second round costs what the first did (1024 rows
+      // of 4096->24576: 990 and 812; 512 of 1024->4096, one round: 31 and 37), a first one from K = 2048 too
+      if (T > 256) return false;
+      if (part) return k > 64 && !full;
+      return m <= 64 || k <= 1024 || T <= (k <= 2048 ? 128 : 32);
+    }
+    if (!part || k >= 512) return true;
+    // K = 64 is a quarter of a unit, 128 half of one (1024 rows of 64->4096:
+    // 17.3 and 15.7, Q8_0 22.5 and 15.9; 128 rows of 128->4096: 10.5 and 9.4)
+    if (q8) return T <= 256 && k > 64 && !(full && k <= 128);
+    if (k == 64) return T <= 256 && !full;
+    return !full || (k > 128 && T <= 256);
+  }
+  const bool xr = q8 || scheme == RLXQ_GGUF_Q4_0 || scheme == RLXQ_GGUF_Q5_K;   // register-streamed beside it
+  if (mlx8 && m > 32 && ((T > 256 && 10 * T < 6 * 256 * ((T + 255) / 256)) || (part && k < 1024)))
+    return false;   // a second round nearly empty (160 rows of 1792->12288: 78 and 61)
+  // one to four tiles of a long K (64 rows of 16384->64: 24.5 and 20.2)
+  if (k >= 8192) return T > (xr ? 1 : 4) || (m <= 32 && (k < 12288 || T > 1));
+  if (k >= 1024) return true;
+  // short K: from so many tiles on that the other one's rounds grow (64 rows of
+  // 384->4096 13.3 and 10.8, 512->4096 12.3 and 11.5, 256->4096 9.7 and 9.6;
+  // 256 rows of 384->4096 14.5 and 14.6, 384->8192 15.6 and 23.2).  32 rows
+  // fill a tile of their own (256->4096: 8.2 and 9.5).
+  if (xr) {
+    if (T > 64) return true;
+    if (m <= 32) return !part && !(q8 && k == 768 && T > 16);
+    return T > 32 || k == 256 || (k == 128 && scheme == RLXQ_GGUF_Q4_0) || (k == 768 && T <= 12);
+  }
+  if (m <= 32) return !part || T > 128;
+  if (part) return T > 128;
+  return T > 64 || (k == 768 && T <= 32);
+}
+
 int bs_order(int scheme) { return scheme == RLXQ_GGUF_Q5_K ? 1 : sk_order(scheme); }
 
 // Eight rows per workgroup once those fill the chip (2048 gathered rows of

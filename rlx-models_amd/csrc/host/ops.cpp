@@ -194,8 +194,7 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   // two for the others.
   const bool split = x_dtype == RLXQ_F32;
   const bool want_exact = split || y_dtype == RLXQ_F32;
-  // (the "...xs" kernels take f32 activations as hi / lo x16 rows: Q3_K, Q2_K,
-  // Q8_K; the other formats' f32 calls go to the block-scaled matmul below)
+  // (the "...xs" kernels take f32 activations as hi / lo x16 rows)
   std::string vs = var;
   if (!te && want_exact && has_exact_gemm(scheme))
     vs = scheme == RLXQ_GGUF_Q6_K ? "w8lx"
@@ -243,8 +242,8 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   }
   const int64_t kslice = ((ksteps + splits - 1) / splits) * 64;
   splits = (k + kslice - 1) / kslice;
-  // (f32 activations, formats of bs_scheme: the block-scaled matmul)
-  if (split && bs_scheme(scheme)) {
+  // (f32 activations: the block-scaled matmul where bs_applies has it)
+  if (split && bs_applies(scheme, m, k, n, true)) {
     SkinnySb sb;
     sb.scales = scales;
     sb.biases = biases;
@@ -404,13 +403,13 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   // once for all rows through the f16-MFMA kernel (MXFP4 with E8M0 scales
   // through its bf16-MFMA twin).  bf16 activations are exact in f16 once
   // scaled; f32 activations run as hi + lo row pairs (~22 significant bits).
-  // (f32 activations past 16 rows, formats of bs_scheme: the block-scaled
+  // (f32 activations past 16 rows, where bs_applies has it: the block-scaled
   // matmul.  Q4_1 4096->24576 at 64 rows 90 us here, 51 there.)
   // RLXQ_DECODE=gemv|skinny forces one where both apply (skinny: also ahead of
   // the block-scaled matmul).
   {
     const bool sk_ok = skinny_applies(scheme, group, sb_dtype, m, k);
-    bool use_sk = sk_ok && m >= 5, use_bs = !xbf && m > 16 && bs_scheme(scheme);
+    bool use_sk = sk_ok && m >= 5, use_bs = !xbf && m > 16 && bs_applies(scheme, m, k, n, false);
     if (const char* e = std::getenv("RLXQ_DECODE")) {
       if (!std::strcmp(e, "gemv")) use_sk = false;
       if (!std::strcmp(e, "skinny")) use_sk = sk_ok, use_bs = false;

@@ -161,6 +161,7 @@ int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const
 // prefill: a call of the exact GEMM's (more than 256 rows, or bf16 output),
 // whose tuning variables it obeys.
 bool bs_scheme(int scheme);
+bool bs_applies(int scheme, int64_t m, int64_t k, int64_t n, bool prefill);
 int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream);
 int64_t bs_lds_row(int scheme);   // bytes of a weight row's unit in LDS
 int bs_order(int scheme);         // code order of its prepared activations

@@ -547,8 +547,9 @@ RLXQ_GEMM256N_INST(q2_k, SCH_Q2_K, 2, false)
 // (Q4_1 and Q8_K: the all-real-tiles variant for bf16 activations keeps one
 // register stage; with two it spilled)
 RLXQ_GEMM256XN_INST(q4_1, SCH_Q4_1, 1, , false)
-RLXQ_GEMM256XN_INST(q4_0, SCH_Q4_0, 2, p2, false)
-RLXQ_GEMM256XN_INST(q8_0, SCH_Q8_0, 1, , false)
+RLXQ_GEMM256XS_INST(q4_1, SCH_Q4_1, 2, p2, false)
+RLXQ_GEMM256X_INST(q4_0, SCH_Q4_0, 2, p2, false)
+RLXQ_GEMM256X_INST(q8_0, SCH_Q8_0, 1, , false)
 RLXQ_GEMM256XN_INST(q4_k, SCH_Q4_K, 2, p2, false)
 RLXQ_GEMM256XN_INST(q6_k, SCH_Q6_K, 1, l, true)
 RLXQ_GEMM256XN_INST(q5_k, SCH_Q5_K, 1, , false)
@@ -556,5 +557,5 @@ RLXQ_GEMM256X_INST(q3_k, SCH_Q3_K, 1, , false)
 RLXQ_GEMM256X_INST(q2_k, SCH_Q2_K, 2, p2, false)
 RLXQ_GEMM256XN_INST(q8_k, SCH_Q8_K, 1, , false)
 RLXQ_GEMM256XS_INST(q8_k, SCH_Q8_K, 2, p2, false)
-RLXQ_GEMM256XN_INST(mlx4, SCH_MLX4, 1, , false)
-RLXQ_GEMM256XN_INST(mlx8, SCH_MLX8, 2, p2, false)
+RLXQ_GEMM256X_INST(mlx4, SCH_MLX4, 1, , false)
+RLXQ_GEMM256X_INST(mlx8, SCH_MLX8, 2, p2, false)

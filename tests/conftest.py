@@ -55,11 +55,12 @@ def announce(msg: str) -> None:
 XL_FORMATS = {3, 2, 1, 7, 10}
 
 
-def batched_f32_kernel(scheme: int, m: int) -> str:
-    """Prefix of the kernel that 5 to 256 rows of f32 activations take by
-    default: from 17 rows the block-scaled matmul, in the formats that have it
-    (MXFP4 (9), Q3_K (11), Q2_K (12) and Q8_K (13) have not)."""
-    return "rlxq_bs_" if m > 16 and scheme not in (9, 11, 12, 13) else "rlxq_skinny"
+def batched_f32_kernel(scheme: int, m: int):
+    """Prefixes of the kernels that 5 to 256 rows of f32 activations can take:
+    the batched-decode kernels and, from 17 rows, the block-scaled matmul where
+    its rule has it (tests/test_bs_gemm_gpu.py), in the formats of it (MXFP4
+    (9), Q3_K (11), Q2_K (12) and Q8_K (13) have none)."""
+    return ("rlxq_skinny", "rlxq_bs_") if m > 16 and scheme not in (9, 11, 12, 13) else ("rlxq_skinny",)
 
 
 def skinny_xl_default(scheme: int, m: int, k: int, xdt: str = "bf16") -> bool:

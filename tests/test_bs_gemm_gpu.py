@@ -14,6 +14,13 @@ from conftest import announce
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(autouse=True)
+def _force_bs(monkeypatch):
+    """The block-scaled kernel wherever it applies (its rule: test_rule)."""
+    monkeypatch.setenv("RLXQ_BS", "1")
+
+
 Q8_0, Q4_0, Q4_1, MLX4, MLX8, Q4_K, Q6_K, Q5_K = 1, 2, 3, 4, 5, 7, 8, 10
 NAMES = {Q8_0: "q8_0", Q4_0: "q4_0", Q4_1: "q4_1", MLX4: "mlx4", MLX8: "mlx8", Q4_K: "q4_k", Q6_K: "q6_k", Q5_K: "q5_k"}
 
@@ -38,7 +45,7 @@ def _case(orc, scheme, rng, n, k):
     return _t(packed), None, None, 32, orc.dequantize(scheme, packed, k).astype(np.float64).reshape(n, k)
 
 
-def _check(ctx, orc, scheme, m, k, n, y_dtype=None):
+def _check(ctx, orc, scheme, m, k, n, y_dtype=None, bs_only=True):
     import torch
 
     rng = np.random.default_rng(m * 7 + k + n * 3 + scheme)
@@ -56,6 +63,8 @@ def _check(ctx, orc, scheme, m, k, n, y_dtype=None):
     got = y.double().cpu().numpy()
     if y_dtype is not None:
         lim = lim + np.abs(want) * 2.0 ** -8   # one rounding to bf16
+    if not bs_only:   # (the other kernels hold weights as f16 hi + lo: to 2^-22, or 2^-25 of 1)
+        lim = lim * 4 + 2.0 ** -24 * np.abs(x).astype(np.float64).sum(1, keepdims=True)
     assert np.all(np.abs(got - want) <= lim), (kern, float(np.max(np.abs(got - want) / lim)))
     return kern
 
@@ -154,3 +163,32 @@ def test_rows_past_4_gb(orc, scheme):
     got = y.double().cpu().numpy()
     assert np.all(np.abs(got - want) <= lim), (kern, float(np.max(np.abs(got - want) / lim)))
     assert kern == f"rlxq_bs_{NAMES[scheme]}_wide", kern
+
+
+@pytest.mark.parametrize("case", [
+    # 17 to 256 rows: (scheme, m, k, n, bf16 output, block-scaled?)
+    (Q4_1, 64, 4096, 4096, False, True), (Q4_1, 17, 256, 64, False, True), (Q4_1, 32, 384, 4096, False, False),
+    (Q4_1, 32, 384, 128 * 129, False, True), (Q4_1, 64, 512, 128 * 64, False, False), (Q4_K, 64, 512, 128 * 65, False, True),
+    (MLX4, 64, 384, 128 * 128, False, False), (MLX4, 64, 384, 128 * 129, False, True), (Q6_K, 33, 768, 128 * 32, False, True),
+    (Q6_K, 33, 768, 128 * 33, False, False), (Q4_1, 64, 1024, 64, False, True), (Q4_1, 64, 8192, 512, False, False),
+    (Q4_1, 64, 8192, 513, False, True), (Q8_0, 64, 8192, 128, False, False), (Q8_0, 64, 8192, 256, False, True),
+    (Q4_0, 33, 640, 4096, False, False), (Q4_0, 33, 640, 4224, False, True), (Q8_0, 40, 256, 128, False, True),
+    (MLX8, 160, 1792, 12288, False, False), (MLX8, 64, 640, 512, False, False), (MLX8, 192, 4096, 4096, False, True),
+    # prefill
+    (Q4_1, 300, 64, 4096, False, True), (Q4_1, 1024, 64, 4096, False, False), (Q4_1, 128, 128, 512, True, False),
+    (Q4_1, 130, 128, 512, True, True), (Q4_0, 512, 256, 300, False, True), (Q8_0, 300, 64, 512, False, False),
+    (Q8_0, 1024, 192, 4096, False, False), (Q8_0, 1024, 576, 4096, False, True), (MLX8, 1024, 1024, 4096, False, False),
+    (MLX8, 512, 1024, 4096, False, True), (MLX8, 300, 4096, 2048, False, False), (MLX8, 257, 4096, 768, False, True), (MLX4, 1100, 8256, 256, False, False),
+    (MLX4, 1100, 8256, 257, False, True), (Q5_K, 300, 256, 64, False, True)], ids=str)
+def test_rule(ctx, orc, monkeypatch, case):
+    """Both sides of the lines between this kernel and the batched-decode
+    kernels and the exact GEMM, each against the oracle."""
+    import torch
+
+    monkeypatch.delenv("RLXQ_BS")
+    scheme, m, k, n, ybf, want = case
+    announce(f"block-scaled rule {NAMES[scheme]} {case[1:]}")
+    kern = _check(ctx, orc, scheme, m, k, n, y_dtype=torch.bfloat16 if ybf else None, bs_only=False)
+    assert kern.startswith(f"rlxq_bs_{NAMES[scheme]}_rt") == want, kern
+    if not want:
+        assert kern.startswith("rlxq_gemm_" if ybf or m > 256 else "rlxq_skinny"), kern
