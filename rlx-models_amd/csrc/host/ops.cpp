@@ -338,7 +338,8 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
 //   12288, two rows 17.8 10.8, four 18.8 13.1; Q4_K at 8192, two rows 8.7
 //   7.9), and three or four rows (MLX 7.7 6.8 | 9.5 9.2 | 23.7 17.7, Q4_K 8.3
 //   6.9 | 10.4 9.3 | 24.7 18.3), Q4_1 only with many weight rows (7.1 6.8 |
-//   8.6 9.1 | 22.5 18.4).
+//   8.6 9.1 | 22.5 18.4) and MLX past K = 2048 or with many (2048->2048 4.7
+//   5.3).
 // RLXQ_GEMV_MF=0 turns it off, =1 takes it wherever it applies (tuning); the
 // other kernels' tuning variables pick those.
 bool mf_applies(int scheme, int group, bool xbf, int64_t m, int64_t k, int64_t n, int64_t rb) {
@@ -355,6 +356,7 @@ bool mf_applies(int scheme, int group, bool xbf, int64_t m, int64_t k, int64_t n
   if (m == 1) return false;
   // (the register kernel's unit chunks are 4096 of K for Q4_K, else 2048)
   if (k > (scheme == RLXQ_GGUF_Q4_K ? 4096 : m == 2 ? 8192 : 4096)) return true;
+  if (scheme == RLXQ_MLX_AFFINE4 && k == 2048 && n < 8192) return false;
   return m > 2 && (scheme != RLXQ_GGUF_Q4_1 || n >= 16384);
 }
 

@@ -105,6 +105,15 @@ def test_large_elements_on_zero_weights(ctx, orc, monkeypatch, scheme, bf16):
         assert "_mf" in kern, kern
 
 
+def test_mlx_short_rows_stay_on_the_register_kernel(ctx, orc):
+    """Three and four bf16 rows of MLX 4-bit at K = 2048: the register kernel,
+    past it (and with many weight rows) this one."""
+    for m, k, n, want in ((3, 2048, 64, False), (4, 2048, 2048, False), (4, 2304, 64, True), (3, 2048, 8192, True)):
+        announce(f"matrix-core decode rule mlx4 m={m} k={k} n={n}")
+        kern = _check(ctx, orc, MLX4, m, k, n, True)
+        assert ("_mf" in kern) == want, (m, k, n, kern)
+
+
 def test_a_row_that_is_not_finite_stays_alone(ctx, orc):
     """An infinity or NaN in one row leaves the others' bits as they were."""
     import torch
