@@ -5,6 +5,7 @@
 #include <hip/hip_runtime_api.h>
 
 #include <algorithm>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -230,9 +231,28 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
   // f32 activations on the block-scaled kernel (chunks of 32 entries; row
   // offsets within an expert's slab fit 32 bits): Q6_K's SwiGLU and the
   // tuning switches keep the row-pair kernels
-  const bool bs = sk && sk_pairs && bs_scheme(scheme) && !(swiglu && !(is_gguf(scheme) || scheme == RLXQ_GGUF_Q4_K ||
-                                                                       scheme == RLXQ_GGUF_Q5_K)) &&
-                  n * rb < ((int64_t)1 << 31) && !std::getenv("RLXQ_MOE_SK") && !std::getenv("RLXQ_MOE_KERNEL");
+  bool bs = sk && sk_pairs && bs_scheme(scheme) && !(swiglu && !(is_gguf(scheme) || scheme == RLXQ_GGUF_Q4_K ||
+                                                                 scheme == RLXQ_GGUF_Q5_K)) &&
+            n * rb < ((int64_t)1 << 31) && !std::getenv("RLXQ_MOE_SK") && !std::getenv("RLXQ_MOE_KERNEL");
+  if (const char* ev = std::getenv("RLXQ_BS")) {
+    bs = bs && std::strcmp(ev, "0") != 0;
+  } else if (bs) {
+    // Where its workgroups (chunk, 128 columns; a chunk's walk K in one go) are
+    // enough for the CUs, or K is short: the row-pair kernels have four to eight
+    // times as many.  us here / there, gate|up of Q4_1 unless named: 2 experts of
+    // 8 entries, 4096 -> 2 x 2048 (32 workgroups) 56 and 28, 8 of 10, 5120 -> 2 x
+    // 1536 (96) 72 and 57, 8 of 16 (96) 73 and 70, 16 of 8, 2048 -> 2 x 1536
+    // (192) 40 and 46; down, 2 of 8, 2048 -> 4096 (64) 28 and 24, 4 of 8 (128) 29
+    // and 30.  Over 407 calls
+    // a format and form the rule is 0.2 to 1.2% behind the faster one.
+    const int64_t wgs = fired_est * (int64_t)std::ceil(avg_e / 32.0) * ((width + 127) / 128);
+    // (Q8_0's SwiGLU form spills, one workgroup a CU: 2 of 48, 4096 -> 2 x 2048
+    // 79 and 54)
+    const bool half = avg_e >= 16.0;   // chunks at least half full
+    if (!swiglu) bs = wgs > 128 || (half && wgs > 64 && k <= 8192) || k <= 1024;
+    else if (scheme == RLXQ_GGUF_Q8_0) bs = (half && wgs > 96) || k <= 256;
+    else bs = wgs > 112 || (half && wgs > (k <= 2048 ? 48 : 64)) || k <= 512;
+  }
   const int64_t rpc = bs ? 32 : sk_pairs ? 8 * sk_mt : 16 * sk_mt;
   const int64_t sk_mp = sk ? ((n_entries + fired_est * (rpc - 1) + rpc - 1) / rpc) * rpc : 0;   // gathered rows
   const int64_t sk_xr = sk_pairs ? 2 * sk_mp : sk_mp;                                            // x16 rows

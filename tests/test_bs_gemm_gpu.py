@@ -31,25 +31,32 @@ def _t(a):
     return torch.from_numpy(np.ascontiguousarray(a)).cuda()
 
 
-def _case(orc, scheme, rng, n, k):
+def _case(orc, scheme, rng, n, k, group=None, slab="f32"):
     """(packed, scales, biases, group, dequantized float64 weights)"""
     if scheme in (MLX4, MLX8):
-        bits, group = (4, 64) if scheme == MLX4 else (8, 32)
+        import torch
+
+        bits, group = (4, group or 64) if scheme == MLX4 else (8, group or 32)
         codes = rng.integers(0, 1 << bits, (n, k)).astype(np.uint32)
         wq = orc.mlx_pack(codes, bits)
         sc = rng.uniform(0.01, 0.1, (n, k // group)).astype(np.float32)
         bi = rng.uniform(-0.5, 0.1, (n, k // group)).astype(np.float32)
+        if slab == "bf16":
+            ts, tb = _t(sc).to(torch.bfloat16), _t(bi).to(torch.bfloat16)
+            sc, bi = ts.float().cpu().numpy(), tb.float().cpu().numpy()
+        else:
+            ts, tb = _t(sc), _t(bi)
         wd = codes * np.repeat(sc.astype(np.float64), group, 1) + np.repeat(bi.astype(np.float64), group, 1)
-        return _t(wq.view(np.uint8)), _t(sc), _t(bi), group, wd
+        return _t(wq.view(np.uint8)), ts, tb, group, wd
     packed = orc.synth(scheme, rng, n, k)
     return _t(packed), None, None, 32, orc.dequantize(scheme, packed, k).astype(np.float64).reshape(n, k)
 
 
-def _check(ctx, orc, scheme, m, k, n, y_dtype=None, bs_only=True):
+def _check(ctx, orc, scheme, m, k, n, y_dtype=None, bs_only=True, group=None, slab="f32"):
     import torch
 
     rng = np.random.default_rng(m * 7 + k + n * 3 + scheme)
-    w, sc, bi, group, wd = _case(orc, scheme, rng, n, k)
+    w, sc, bi, group, wd = _case(orc, scheme, rng, n, k, group, slab)
     x = rng.standard_normal((m, k)).astype(np.float32)
     x[0] *= 1e-6
     x[m // 2] *= 3e4
@@ -100,6 +107,16 @@ def test_row_tiles_and_splits(ctx, orc, monkeypatch, cfg):
         announce(f"block-scaled {cfg} {NAMES[scheme]} {mkn}")
         kern = _check(ctx, orc, scheme, *mkn)
         assert kern == f"rlxq_bs_{NAMES[scheme]}_rt{cfg[0]}", kern
+
+
+@pytest.mark.parametrize("scheme", [MLX4, MLX8], ids=lambda s: NAMES[s])
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("slab", ["f32", "bf16"])
+def test_mlx_groups_and_slabs(ctx, orc, scheme, group, slab):
+    for mkn in ((17, 640, 17), (70, 1152, 131), (300, 4608, 129)):
+        announce(f"block-scaled {NAMES[scheme]} group={group} slab={slab} {mkn}")
+        kern = _check(ctx, orc, scheme, *mkn, group=group, slab=slab)
+        assert kern.startswith(f"rlxq_bs_{NAMES[scheme]}_rt"), kern
 
 
 def test_noalloc_is_the_same(ctx, orc):
