@@ -38,6 +38,21 @@ double bs_unit_factor(int scheme) {
     default: return 1.0;
   }
 }
+constexpr int kNh = 2;   // parts of an f32 row: f16 hi and lo
+
+// Scratch of one pass over `rows` rows: fragments, row factors, block sums,
+// K-split partial sums.
+struct BsBytes {
+  size_t x, s, sum, part;
+  BsBytes(int64_t rows, int RT, int64_t n, int64_t nu, int64_t splits) {
+    const int64_t t = (rows + 32 * RT - 1) / (32 * RT) * RT;   // 32-row tiles
+    x = round256((size_t)(16 * nu * t * kNh) * 1024);
+    s = round256((size_t)t * 128);
+    sum = round256((size_t)(nu * t) * 1024);
+    part = splits > 1 ? round256((size_t)(splits * rows * n) * 4) : 0;
+  }
+  size_t all() const { return x + s + sum + part; }
+};
 }  // namespace
 
 bool bs_scheme(int scheme) {
@@ -130,8 +145,84 @@ int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream) {
   return launch(ctx, fn, dim3((unsigned)(rows / per)), dim3(1024), 0, stream, args, name);
 }
 
+namespace {
+// One pass: preparation, matmul, reduction.
+int bs_pass(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m, int64_t k,
+            int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, int RT, int64_t splits, int64_t uslice,
+            const char* name) {
+  const int64_t nu = (k + 255) / 256, tiles_m = (m + 32 * RT - 1) / (32 * RT), tiles_n = (n + 127) / 128;
+  const int64_t rtiles = tiles_m * RT;
+  const BsBytes b(m, RT, n, nu, splits);
+  void* ws = nullptr;
+  int rc;
+  if ((rc = workspace(ctx, b.all(), &ws, stream))) return rc;
+  char* wsb = static_cast<char*>(ws);
+
+  rlxq_bs_prep_args p;
+  std::memset(&p, 0, sizeof p);
+  p.x = x;
+  p.x16 = reinterpret_cast<uint8_t*>(wsb);
+  p.inv_s = reinterpret_cast<float*>(wsb + b.x);
+  p.ssum = reinterpret_cast<uint32_t*>(wsb + b.x + b.s);
+  p.M = m;
+  p.K = k;
+  p.rtiles = (int32_t)rtiles;
+  p.nh = kNh;
+  p.kb8 = (int32_t)(8 * nu);
+  p.order = bs_order(scheme);
+  p.x_bf16 = x_dtype == RLXQ_BF16;
+  p.rdiv = 1;
+  if ((rc = bs_prep(ctx, p, stream))) return rc;
+  hipFunction_t fn;
+
+  rlxq_bs_args a;
+  std::memset(&a, 0, sizeof a);
+  a.x16 = p.x16;
+  a.inv_s = p.inv_s;
+  a.ssum = p.ssum;
+  a.w = static_cast<const uint8_t*>(w);
+  a.scales = sb.scales;
+  a.biases = sb.biases;
+  a.part = splits > 1 ? reinterpret_cast<float*>(wsb + b.x + b.s + b.sum) : nullptr;
+  a.y = y;
+  a.M = m;
+  a.N = n;
+  a.K = k;
+  a.rb = rb;
+  a.y_ld = n;
+  a.group = sb.group;
+  a.rtiles = (int32_t)rtiles;
+  a.uslice = (int32_t)uslice;
+  a.splits = (int32_t)splits;
+  a.tiles_n = (int32_t)tiles_n;
+  a.tiles_m = (int32_t)tiles_m;
+  a.y_bf16 = y_dtype == RLXQ_BF16;
+  a.sb_bf16 = sb.sb_bf16;
+  if ((rc = get_fn(ctx, name, &fn))) return rc;
+  void* args[] = {&a};
+  const size_t lds = bs_lds_bytes(scheme, RT);
+  if ((rc = launch(ctx, fn, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(256), lds, stream, args, name)))
+    return rc;
+  if (splits > 1) {
+    rlxq_skinny_args r;
+    std::memset(&r, 0, sizeof r);
+    r.part = a.part;
+    r.y = y;
+    r.M = m;
+    r.N = n;
+    r.y_ld = n;
+    r.splits = (int32_t)splits;
+    r.y_bf16 = a.y_bf16;
+    rc = splits_reduce(ctx, r, stream);
+    if (!rc) ctx->last_kernel = name;
+  }
+  return rc;
+}
+}  // namespace
+
 int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
-                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, bool prefill) {
+                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, bool prefill,
+                size_t counted) {
   const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
   const int64_t nu = (k + 255) / 256;   // 256-element units
   // 64-row tiles past 32 rows (197 rows of Q4_K, 4096->24576: 131 us in four
@@ -139,7 +230,6 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   // columns.  RLXQ_BS="RT,splits" (tuning) sets the 32-row tiles per
   // workgroup (1 or 2; 0: the form with 64-bit row offsets) and, unless 0,
   // the K splits.
-  const int64_t r32 = (m + 31) / 32;
   // (32 weight rows past 4 GB: the form with 64-bit row offsets)
   bool wide = rb >= ((int64_t)1 << 27);
   int RT = m > 32 ? 2 : 1;
@@ -156,7 +246,6 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   if (prefill)
     if (const char* e = std::getenv("RLXQ_GEMM_SPLITS")) want = std::max(1, std::atoi(e));
   const int64_t tiles_m = (m + 32 * RT - 1) / (32 * RT), tiles_n = (n + 127) / 128;
-  const int64_t rtiles = tiles_m * RT;
   int64_t splits = 1;
   if (want > 0) {
     splits = std::min<int64_t>(want, nu);
@@ -184,81 +273,38 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   }
   const int64_t uslice = (nu + splits - 1) / splits;
   splits = (nu + uslice - 1) / uslice;
-  if (tiles_m * tiles_n * splits > 0x7fffffff || rtiles > 0x3ffffff)
+  if (tiles_m * tiles_n * splits > 0x7fffffff || tiles_m * RT > 0x3ffffff)
     return fail(ctx, RLXQ_E_SHAPE, "dequant_matmul: block-scaled grid");
 
-  const int nh = 2;
-  const size_t x_bytes = round256((size_t)(16 * nu * rtiles * nh) * 1024), s_bytes = round256((size_t)rtiles * 128);
-  const size_t sum_bytes = round256((size_t)(nu * rtiles) * 1024);
-  const size_t part_bytes = splits > 1 ? round256((size_t)(splits * m * n) * 4) : 0;
-  void* ws = nullptr;
-  int rc;
-  // (what counts against the no-allocation limit: the f16 hi and lo rows)
-  const size_t need = x_bytes + s_bytes + sum_bytes + part_bytes, core = (size_t)(r32 * 32 * k) * 4;
-  if ((rc = workspace(ctx, need, &ws, stream, need > core ? need - core : 0))) return rc;
-  char* wsb = static_cast<char*>(ws);
-
-  rlxq_bs_prep_args p;
-  std::memset(&p, 0, sizeof p);
-  p.x = x;
-  p.x16 = reinterpret_cast<uint8_t*>(wsb);
-  p.inv_s = reinterpret_cast<float*>(wsb + x_bytes);
-  p.ssum = reinterpret_cast<uint32_t*>(wsb + x_bytes + s_bytes);
-  p.M = m;
-  p.K = k;
-  p.rtiles = (int32_t)rtiles;
-  p.nh = nh;
-  p.kb8 = (int32_t)(8 * nu);
-  p.order = bs_order(scheme);
-  p.x_bf16 = x_dtype == RLXQ_BF16;
-  p.rdiv = 1;
-  if ((rc = bs_prep(ctx, p, stream))) return rc;
-  hipFunction_t fn;
-
-  rlxq_bs_args a;
-  std::memset(&a, 0, sizeof a);
-  a.x16 = p.x16;
-  a.inv_s = p.inv_s;
-  a.ssum = p.ssum;
-  a.w = static_cast<const uint8_t*>(w);
-  a.scales = sb.scales;
-  a.biases = sb.biases;
-  a.part = splits > 1 ? reinterpret_cast<float*>(wsb + x_bytes + s_bytes + sum_bytes) : nullptr;
-  a.y = y;
-  a.M = m;
-  a.N = n;
-  a.K = k;
-  a.rb = rb;
-  a.y_ld = n;
-  a.group = sb.group;
-  a.rtiles = (int32_t)rtiles;
-  a.uslice = (int32_t)uslice;
-  a.splits = (int32_t)splits;
-  a.tiles_n = (int32_t)tiles_n;
-  a.tiles_m = (int32_t)tiles_m;
-  a.y_bf16 = y_dtype == RLXQ_BF16;
-  a.sb_bf16 = sb.sb_bf16;
+  // Rows per pass: all of them, or as many whole tiles as the array of the
+  // no-allocation entry point holds (rows do not depend on each other and the
+  // K splits stay those of the whole call: the same bits).  Which calls that
+  // entry point takes is decided by `counted`, what the batched-decode kernels
+  // or the exact GEMM need for them; fragments in whole 256-element units are
+  // four times that at K = 64, and partial sums of other splits.
+  int64_t pass = m;
+  if (ctx->fixed_active) {
+    if (counted > ctx->fixed_bytes) return scratch_refused(ctx, counted);
+    if (BsBytes(m, RT, n, nu, splits).all() > ctx->fixed_bytes) {
+      if (BsBytes(32 * RT, RT, n, nu, splits).all() > ctx->fixed_bytes) RT = 1;
+      int64_t lo = 0, hi = (m + 32 * RT - 1) / (32 * RT);   // tiles that fit, and that do not
+      while (hi - lo > 1) {
+        const int64_t mid = (lo + hi) / 2;
+        (BsBytes(mid * 32 * RT, RT, n, nu, splits).all() <= ctx->fixed_bytes ? lo : hi) = mid;
+      }
+      // (at prefill one does: 32 rows take half of what 64, the fewest, count)
+      if (lo > 0) pass = lo * 32 * RT;
+      else if (!prefill) return skinny_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb);
+    }
+  }
   char name[64];
   if (wide) std::snprintf(name, sizeof name, "rlxq_bs_%s_wide", scheme_name(scheme));
   else std::snprintf(name, sizeof name, "rlxq_bs_%s_rt%d", scheme_name(scheme), RT);
-  if ((rc = get_fn(ctx, name, &fn))) return rc;
-  void* args[] = {&a};
-  const size_t lds = bs_lds_bytes(scheme, RT);
-  if ((rc = launch(ctx, fn, dim3((unsigned)(tiles_m * tiles_n * splits)), dim3(256), lds, stream, args, name)))
-    return rc;
-  if (splits > 1) {
-    rlxq_skinny_args r;
-    std::memset(&r, 0, sizeof r);
-    r.part = a.part;
-    r.y = y;
-    r.M = m;
-    r.N = n;
-    r.y_ld = n;
-    r.splits = (int32_t)splits;
-    r.y_bf16 = a.y_bf16;
-    rc = splits_reduce(ctx, r, stream);
-    if (!rc) ctx->last_kernel = name;
-  }
+  int rc = RLXQ_OK;
+  for (int64_t r0 = 0; r0 < m && !rc; r0 += pass)
+    rc = bs_pass(ctx, scheme, static_cast<const char*>(x) + r0 * k * (x_dtype == RLXQ_BF16 ? 2 : 4), x_dtype, w, rb,
+                 std::min(pass, m - r0), k, n, static_cast<char*>(y) + r0 * n * (y_dtype == RLXQ_BF16 ? 2 : 4), y_dtype,
+                 stream, sb, RT, splits, uslice, name);
   return rc;
 }
 

@@ -3,8 +3,7 @@
 // serving loops, harnesses that forbid hipMalloc).
 //
 // Its scratch (prepared activations, split-K partial sums) is one file-scope
-// device array, `scratch`, of RLXQ_NOALLOC_SCRATCH_BYTES (the limit a call is
-// held to) and kNoallocSlack for padding and partial sums.  Each GPU holds its
+// device array, `scratch`, of RLXQ_NOALLOC_SCRATCH_BYTES.  Each GPU holds its
 // own copy, at its own address, until the process ends.  In host code the
 // array's name is only a host-side handle: its device address on a device is
 // taken once, with that device current, by hipGetSymbolAddress (from
@@ -26,7 +25,7 @@
 
 namespace {
 
-static __device__ __align__(256) unsigned char scratch[RLXQ_NOALLOC_SCRATCH_BYTES + rlxq::kNoallocSlack];
+static __device__ __align__(256) unsigned char scratch[RLXQ_NOALLOC_SCRATCH_BYTES];
 
 constexpr int kMaxDevices = 64;
 std::mutex g_mu;

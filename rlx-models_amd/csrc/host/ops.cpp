@@ -249,7 +249,9 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
     sb.biases = biases;
     sb.group = is_mlx(scheme) ? group : 32;
     sb.sb_bf16 = sb_code(sb_dtype);
-    return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, true);
+    const size_t counted = prep_x16_bytes(m, k, false, 0, 2) +
+                           (splits > 1 ? (((size_t)(splits * m * n) * 4 + 255) & ~(size_t)255) : 0);
+    return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, true, counted);
   }
   char name[64];
   std::snprintf(name, sizeof name, "rlxq_gemm_%s_t%d%s", scheme_name(scheme), tile, vs.c_str());
@@ -423,8 +425,13 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
       sb.group = is_mlx(scheme) ? group : 32;
       sb.sb_bf16 = sb_code(sb_dtype);
       if (use_bs && !std::getenv("RLXQ_SKINNY_XR") && !std::getenv("RLXQ_SKINNY_NS") &&
-          !std::getenv("RLXQ_SKINNY_XL"))
-        return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, false);
+          !std::getenv("RLXQ_SKINNY_XL")) {
+        size_t counted = 0;
+        if (ctx->fixed_active &&
+            (rc = skinny_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, &counted)))
+          return rc;
+        return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, false, counted);
+      }
       return skinny_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb);
     }
   }

@@ -154,12 +154,15 @@ int launch(rlxq_ctx* ctx, hipFunction_t fn, dim3 grid, dim3 block, size_t lds, v
   return RLXQ_OK;
 }
 
-int workspace(rlxq_ctx* ctx, size_t bytes, void** out, void* stream, size_t slack) {
+int scratch_refused(rlxq_ctx* ctx, size_t bytes) {
+  return fail(ctx, RLXQ_E_SCRATCH,
+              "this call needs " + std::to_string(bytes) + " B of scratch; the no-allocation entry point holds " +
+                  std::to_string(ctx->fixed_bytes) + " B");
+}
+
+int workspace(rlxq_ctx* ctx, size_t bytes, void** out, void* stream) {
   if (ctx->fixed_active) {
-    if (bytes > ctx->fixed_bytes + std::min(slack, kNoallocSlack))
-      return fail(ctx, RLXQ_E_SCRATCH,
-                  "this call needs " + std::to_string(bytes) + " B of scratch; the no-allocation entry point holds " +
-                      std::to_string(ctx->fixed_bytes) + " B");
+    if (bytes > ctx->fixed_bytes) return scratch_refused(ctx, bytes);
     *out = ctx->fixed_p;
     return RLXQ_OK;
   }

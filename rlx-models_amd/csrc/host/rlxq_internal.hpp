@@ -88,17 +88,12 @@ int blocks_per_cu(rlxq_ctx* ctx, const std::string& name, hipFunction_t fn, int 
 int launch(rlxq_ctx* ctx, hipFunction_t fn, dim3 grid, dim3 block, size_t lds, void* stream,
            void** args, const char* what);
 
-// Bytes the no-allocation array holds past RLXQ_NOALLOC_SCRATCH_BYTES: block
-// sums, padding rows and split-K partial sums of the block-scaled matmul,
-// which do not count against the published limit (24 MiB of partial sums and,
-// at the limit's 64 MiB of activations, at most 3 of block sums and 22 of
-// padding).
-constexpr size_t kNoallocSlack = (size_t)52 << 20;
-
 // Ensures at least `bytes` of context scratch for `stream`; returns its
-// device pointer.  `slack` of them do not count against the no-allocation
-// entry point's limit.
-int workspace(rlxq_ctx* ctx, size_t bytes, void** out, void* stream, size_t slack = 0);
+// device pointer.
+int workspace(rlxq_ctx* ctx, size_t bytes, void** out, void* stream);
+// RLXQ_E_SCRATCH with its message: a call of the no-allocation entry point
+// that needs `bytes`.
+int scratch_refused(rlxq_ctx* ctx, size_t bytes);
 // Frees the stream's retired buffers whose completion event has passed
 // (reclaim), or all of them (free, after the stream has been synchronised).
 void reclaim_retired(rlxq_ctx::Scratch& w);
@@ -149,6 +144,7 @@ int splits_reduce(rlxq_ctx* ctx, rlxq_skinny_args& a, void* stream);
 // lo (f32 activations keep ~22 significant bits), with a factor each: rows
 // 2r, 2r + 1 (split 1), or 64-row blocks of 32 hi then 32 lo rows (split 2,
 // row-major; m rounded up to 32, the extra rows zero).
+size_t prep_x16_bytes(int64_t m, int64_t k, bool frag_major, int64_t mp, int split);
 int prep_x16(rlxq_ctx* ctx, const void* x, int x_dtype, int64_t m, int64_t k, int order, size_t extra,
              rlxq_x16_args& xa, char** rest, void* stream, bool frag_major = false, int64_t mp = 0,
              bool out_bf16 = false, int split = 0, int post_exp = 0);
@@ -156,17 +152,21 @@ int prep_x16(rlxq_ctx* ctx, const void* x, int x_dtype, int64_t m, int64_t k, in
 // -8 for MLX affine (their f16 weights are prescaled by 2^8), else 0.
 int sk_post_exp(int scheme);
 int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
-                    int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb = SkinnySb());
+                    int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb = SkinnySb(),
+                    size_t* need = nullptr);   // (need: nothing is launched, *need = its bytes of scratch)
 // Block-scaled MFMA matmul (f32 activations): its formats, and the call.
 // prefill: a call of the exact GEMM's (more than 256 rows, or bf16 output),
 // whose tuning variables it obeys.
+// counted: the bytes of scratch that decide whether the no-allocation entry
+// point takes the call.
 bool bs_scheme(int scheme);
 bool bs_applies(int scheme, int64_t m, int64_t k, int64_t n, bool prefill);
 int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream);
 int64_t bs_lds_row(int scheme);   // bytes of a weight row's unit in LDS
 int bs_order(int scheme);         // code order of its prepared activations
 int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
-                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, bool prefill);
+                int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, bool prefill,
+                size_t counted);
 int i8b_dispatch(rlxq_ctx* ctx, int group, const void* x, int x_dtype, const void* w, const void* scales,
                  const void* zp, int sb_dtype, int64_t m, int64_t k, int64_t n, void* y, int y_dtype,
                  void* stream);

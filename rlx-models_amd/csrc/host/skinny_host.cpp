@@ -19,8 +19,6 @@ namespace {
 size_t round256(size_t b) { return (b + 255) & ~(size_t)255; }
 }  // namespace
 
-// x -> prepared f16 activations and row scales in the workspace (x16 at
-// the start, inv_s after it; `extra` more bytes follow for the caller).
 int splits_reduce(rlxq_ctx* ctx, rlxq_skinny_args& a, void* stream) {
   hipFunction_t fn;
   int rc;
@@ -30,6 +28,16 @@ int splits_reduce(rlxq_ctx* ctx, rlxq_skinny_args& a, void* stream) {
   return launch(ctx, fn, dim3((unsigned)((threads + 255) / 256)), dim3(256), 0, stream, rargs, "rlxq_skinny_reduce");
 }
 
+// Bytes of scratch that prep_x16 takes beside `extra`.
+size_t prep_x16_bytes(int64_t m, int64_t k, bool frag_major, int64_t mp, int split) {
+  const int64_t rows = split == 2 ? (m + 31) / 32 * 64 : (split ? 2 * m : m);
+  if (!frag_major || mp < rows) mp = rows;
+  return round256((size_t)(mp * k) * 2) + round256((size_t)rows * 4) +
+         (frag_major ? round256((size_t)(mp * (k / 32)) * 4) : 0);
+}
+
+// x -> prepared f16 activations and row scales in the workspace (x16 at
+// the start, inv_s after it; `extra` more bytes follow for the caller).
 int prep_x16(rlxq_ctx* ctx, const void* x, int x_dtype, int64_t m, int64_t k, int order, size_t extra,
              rlxq_x16_args& xa, char** rest, void* stream, bool frag_major, int64_t mp, bool out_bf16, int split,
              int post_exp) {
@@ -91,7 +99,7 @@ int64_t xl_chunk_bytes(int scheme) {
 // grid holds about two workgroups per CU (RLXQ_SKINNY_WGS scales that).
 int skinny_xr_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
                        int64_t k, int64_t n, void* y, int y_dtype, void* stream, int MT, int NT, int D,
-                       const SkinnySb& sb, int SC = 0) {
+                       const SkinnySb& sb, size_t* need, int SC = 0) {
   // f32 activations: hi and lo rows (2m x16 rows), added in the epilogue
   const bool split = x_dtype == RLXQ_F32;
   const int64_t mr = split ? 2 * m : m;
@@ -113,10 +121,14 @@ int skinny_xr_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, co
   splits = (k + kslice - 1) / kslice;
   if (tiles_n * mch * splits > 0x7fffffff) return fail(ctx, RLXQ_E_SHAPE, "dequant_matmul: batched-decode grid");
   const size_t part_bytes = splits > 1 ? round256((size_t)(splits * m * n) * 4) : 0;
+  const int64_t mp = mch * 16 * MT;
+  if (need) {
+    *need = prep_x16_bytes(m, k, true, mp, split ? 1 : 0) + part_bytes;
+    return RLXQ_OK;
+  }
   rlxq_x16_args xa;
   char* rest = nullptr;
   int rc;
-  const int64_t mp = mch * 16 * MT;
   if ((rc = prep_x16(ctx, x, x_dtype, m, k, sk_order(scheme), part_bytes, xa, &rest, stream, true, mp,
                      scheme == RLXQ_MLX_MXFP4, split ? 1 : 0, sk_post_exp(scheme))))
     return rc;
@@ -171,7 +183,7 @@ int skinny_xr_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, co
 // splits as for the register-streamed kernel.
 int skinny_ns_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
                        int64_t k, int64_t n, void* y, int y_dtype, void* stream, int MT, int NT, int D,
-                       const SkinnySb& sb) {
+                       const SkinnySb& sb, size_t* need) {
   // f32 activations: hi and lo rows (2m x16 rows), added in the epilogue
   const bool split = x_dtype == RLXQ_F32;
   const int64_t mr = split ? 2 * m : m;
@@ -186,10 +198,14 @@ int skinny_ns_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, co
   splits = (k + kslice - 1) / kslice;
   if (tiles_n * mch * splits > 0x7fffffff) return fail(ctx, RLXQ_E_SHAPE, "dequant_matmul: batched-decode grid");
   const size_t part_bytes = splits > 1 ? round256((size_t)(splits * m * n) * 4) : 0;
+  const int64_t mp = mch * 16 * MT;
+  if (need) {
+    *need = prep_x16_bytes(m, k, true, mp, split ? 1 : 0) + part_bytes;
+    return RLXQ_OK;
+  }
   rlxq_x16_args xa;
   char* rest = nullptr;
   int rc;
-  const int64_t mp = mch * 16 * MT;
   if ((rc = prep_x16(ctx, x, x_dtype, m, k, sk_order(scheme), part_bytes, xa, &rest, stream, true, mp,
                      scheme == RLXQ_MLX_MXFP4, split ? 1 : 0, sk_post_exp(scheme))))
     return rc;
@@ -265,7 +281,7 @@ bool skinny_applies(int scheme, int group, int sb_dtype, int64_t m, int64_t k) {
 // at most 32 and at most one split per K step; their partial sums (f32,
 // [splits, M, N]) are added in split order.
 int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m_out,
-                    int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb) {
+                    int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, size_t* need) {
   const bool mlx = scheme == RLXQ_MLX_AFFINE4 || scheme == RLXQ_MLX_AFFINE8 || scheme == RLXQ_MLX_MXFP4;
   // f32 activations run as hi and lo x16 rows (the register-streamed and
   // N-split kernels add each pair): the tilings below are chosen on those
@@ -273,10 +289,10 @@ int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const
   const bool f32x = x_dtype == RLXQ_F32;
   const int64_t m = f32x ? 2 * m_out : m_out;
   auto run_xr = [&](int MT, int NT, int D) {
-    return skinny_xr_dispatch(ctx, scheme, x, x_dtype, w, rb, m_out, k, n, y, y_dtype, stream, MT, NT, D, sb);
+    return skinny_xr_dispatch(ctx, scheme, x, x_dtype, w, rb, m_out, k, n, y, y_dtype, stream, MT, NT, D, sb, need);
   };
   auto run_ns = [&](int MT, int NT, int D) {
-    return skinny_ns_dispatch(ctx, scheme, x, x_dtype, w, rb, m_out, k, n, y, y_dtype, stream, MT, NT, D, sb);
+    return skinny_ns_dispatch(ctx, scheme, x, x_dtype, w, rb, m_out, k, n, y, y_dtype, stream, MT, NT, D, sb, need);
   };
   // The LDS-staged kernels (Q4_1, Q4_0, Q8_0, Q4_K, Q5_K; K whole 2-chunk
   // steps), MT 1, NT 2, 2-chunk steps, ring depth 1 (three waves per SIMD):
@@ -299,7 +315,8 @@ int skinny_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const
       else if (e[0] == '0') xl = false;
     }
     if (xl && (k / 128) % lsc == 0)
-      return skinny_xr_dispatch(ctx, scheme, x, x_dtype, w, rb, m_out, k, n, y, y_dtype, stream, lmt, lnt, ld, sb, lsc);
+      return skinny_xr_dispatch(ctx, scheme, x, x_dtype, w, rb, m_out, k, n, y, y_dtype, stream, lmt, lnt, ld, sb, need,
+                                lsc);
   }
   // The register-streamed kernels (no LDS stage).  RLXQ_SKINNY_XR="MT,NT,D"
   // picks a compiled one (every combination for Q4_1, the defaults for the

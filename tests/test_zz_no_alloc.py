@@ -82,3 +82,71 @@ def test_noalloc_rejects_oversized_scratch(ctx, orc):
     assert e.value.status == rlxq.E_SCRATCH
     torch.cuda.synchronize()
     assert float(y.abs().max()) == 0.0
+
+
+def _bytes_q4_1(gen, n, k):
+    """Q4_1 rows of finite scales (every byte below 60)."""
+    import torch
+
+    return torch.randint(0, 60, (n, k // 32 * 20), device="cuda", dtype=torch.uint8, generator=gen)
+
+
+@pytest.mark.parametrize("k,m", [(64, 254176), (128, 129024), (320, 52096)], ids=str)
+def test_noalloc_f32_prefill_up_to_the_limit(ctx, orc, monkeypatch, k, m):
+    """f32 rows at prefill count as the exact GEMM lays them out (a hi and a lo
+    f16 row and a factor each): m rows are the most that fit, and one more is
+    refused.  The block-scaled matmul, whose fragments take whole 256-element
+    units, does them in passes: the same bits."""
+    import torch
+    import rlxq
+
+    monkeypatch.setenv("RLXQ_BS", "1")
+    n = 64
+    need = lambda rows: (rows + 31) // 32 * 64 * (2 * k + 4)   # (both parts whole 256 bytes here)
+    assert need(m) <= 64 << 20 < need(m + 1)
+    announce(f"noalloc f32 prefill limit k={k} m={m}")
+    gen = torch.Generator(device="cuda").manual_seed(k)
+    w = _bytes_q4_1(gen, n, k).view(-1)
+    x = torch.randn((m + 1, k), device="cuda", generator=gen)
+    want = ctx.dequant_matmul(x[:m], w, rlxq.GGUF_Q4_1, n)
+    kern = ctx.last_kernel
+    y = torch.full((m + 1, n), float("nan"), device="cuda")
+    ctx.dequant_matmul_noalloc(x[:m], w, rlxq.GGUF_Q4_1, n, y=y[:m])
+    torch.cuda.synchronize()
+    assert ctx.last_kernel == kern == "rlxq_bs_q4_1_rt2"
+    assert torch.equal(y[:m], want) and bool(torch.isnan(y[m]).all())
+    rows = np.array([0, 1, m // 2, m - 1])
+    wd = orc.dequantize(orc.Q4_1, w.view(n, -1).cpu().numpy(), k).astype(np.float64)
+    ref = x[torch.from_numpy(rows).cuda()].cpu().numpy().astype(np.float64) @ wd.T
+    assert np.max(np.abs(y[torch.from_numpy(rows).cuda()].cpu().numpy() - ref)) <= 2e-5 * np.max(np.abs(ref))
+    with pytest.raises(rlxq.RlxqError) as e:
+        ctx.dequant_matmul_noalloc(x, w, rlxq.GGUF_Q4_1, n, y=y)
+    assert e.value.status == rlxq.E_SCRATCH
+
+
+def test_noalloc_f32_batched_near_the_limit(ctx, monkeypatch):
+    """f32 rows of a batch count as the batched-decode kernels lay them out.
+    Partial sums of more splits than theirs: passes over the rows, or where one
+    tile of rows does not fit, those kernels."""
+    import torch
+    import rlxq
+
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    for bs, m, k, n, same in (("2,32", 256, 57344, 256, True), ("1,32", 32, 458752, 4096, False)):
+        monkeypatch.setenv("RLXQ_BS", bs)
+        announce(f"noalloc f32 batched near the limit {(m, k, n)}")
+        w = _bytes_q4_1(gen, n, k).view(-1)
+        x = torch.randn((m, k), device="cuda", generator=gen)
+        want = ctx.dequant_matmul(x, w, rlxq.GGUF_Q4_1, n)
+        assert ctx.last_kernel == f"rlxq_bs_q4_1_rt{bs[0]}"
+        y = torch.full((m, n), float("nan"), device="cuda")
+        ctx.dequant_matmul_noalloc(x, w, rlxq.GGUF_Q4_1, n, y=y)
+        torch.cuda.synchronize()
+        if same:
+            assert ctx.last_kernel == f"rlxq_bs_q4_1_rt{bs[0]}"
+            assert torch.equal(y, want)
+        else:
+            assert ctx.last_kernel.startswith("rlxq_skinny"), ctx.last_kernel
+            assert float((y - want).abs().max()) <= 2e-5 * float(want.abs().max())
+        del w, x, y, want
+        torch.cuda.empty_cache()
