@@ -989,7 +989,7 @@ RLXQ_SKINNYNS_INST(q6_k, SCH_Q6_K, 4, 1, 2)
 // place the entries.  (A routing table and a layout from it, each with its
 // scans of ten barriers, took 7.0 + 7.8 us for 2048 entries.)
 extern "C" __global__ __launch_bounds__(1024) void rlxq_moe_layout_k(rlxq_moe_layout_args a) {
-  __shared__ int32_t cnt[1024], cur[1024], wsum[16];
+  __shared__ int32_t cnt[1024], cur[1024], fc[1024], wsum[16];
   const int t = threadIdx.x, lane = t & 63, wv = t >> 6;
   const int E = a.t.E, R = a.rows_per_chunk;
   auto expert_of = [&](int64_t i) -> int {
@@ -1015,18 +1015,36 @@ extern "C" __global__ __launch_bounds__(1024) void rlxq_moe_layout_k(rlxq_moe_la
     const int o = __shfl_up(inc, d, 64);
     if (lane >= d) inc += o;
   }
-  if (lane == 63) wsum[wv] = inc;
+  // (the top bit: an expert of the wave has many chunks)
+  const int many = __ballot(ch > 8) ? (int)0x80000000 : 0;
+  if (lane == 63) wsum[wv] = inc | many;
   __syncthreads();
-  int base = 0, total = 0;
+  int base = 0, total = 0, any = 0;
 #pragma unroll
   for (int w = 0; w < 16; w++) {
-    base += w < wv ? wsum[w] : 0;
-    total += wsum[w];
+    base += w < wv ? wsum[w] & 0x7fffffff : 0;
+    total += wsum[w] & 0x7fffffff;
+    any |= wsum[w];
   }
   const int first = base + inc - ch;   // the expert's first chunk
   cur[t] = first * R;
   if (t == 0) a.cmap[0] = total;
-  for (int q = 0; q < ch; q++) a.cmap[1 + first + q] = t;
+  if (any < 0) {
+    // a crowded expert: every chunk by a thread of its own, which looks its
+    // expert up (the last one whose first chunk is at most it: those without
+    // entries share the next one's).  16384 of 32768 entries on one expert took
+    // 46 us with a thread storing each expert's chunks, 33 so.
+    fc[t] = first;
+    __syncthreads();
+    for (int q = t; q < total; q += 1024) {
+      int e = 0;
+#pragma unroll
+      for (int d = 512; d > 0; d >>= 1) e += fc[e + d] <= q ? d : 0;
+      a.cmap[1 + q] = e;
+    }
+  } else {
+    for (int q = 0; q < ch; q++) a.cmap[1 + first + q] = t;
+  }
   // padding rows: past the expert's entries, and past the last chunk
   for (int p = c; p < ch * R; p++) a.emap[(int64_t)first * R + p] = -1;
   for (int64_t p = (int64_t)total * R + t; p < a.Mp; p += 1024) a.emap[p] = -1;
