@@ -10,7 +10,10 @@ activations bf16 N(0,1), outputs f32.  Inputs are resident in HBM before the
 timed region.  `value` is algorithmic bytes (N*K*0.625 + K*2 + N*4 per GEMV)
 moved per second over K timed steps.
 
-Extra keys of the same JSON line:
+Extra keys of the same JSON line (batched_decode, prefill_detail and schemes
+give each entry's microseconds only, so that the line stays short enough to be
+kept whole: `--section batched|prefill|schemes` prints one of them with
+kernels, rates and both timings):
   roofline        the dominant kernel of the step (largest total time):
                   algorithmic bytes per launch / average launch duration, the
                   durations from HIP events on the launch stream around runs
@@ -482,7 +485,7 @@ def prefill_headline(detail: dict) -> dict:
             f32[f"{sname}_kernel"] = a["kernel"]
     return {"TFLOPs": round(tf, 1), "unit": "TFLOP/s", "frac_bf16_peak": round(tf / BF16_PEAK_TFLOPS, 4),
             "f32_contract": dict(f32, workload="the same two shapes with F32 x and F32 y (the reference "
-                                               "operator's operand types): exact f16 hi + lo weights, x as "
+                                               "operator's operand types): block-scaled MFMA matmul, x as "
                                                "hi + lo f16 rows"),
             "workload": "Q4_1 group-32 dequant-GEMM, bf16 x and y, f32 accumulate, M=4096: Qwen3-8B gate_up "
                         "4096->24576 + down 12288->4096",
@@ -777,7 +780,7 @@ def moe_section(ctx, gen, sptr, stream, scheme: str = "q4_1", tokens: int = 16, 
     their own expert banks and logits alternate (755 MB of banks).  `tokens`
     = 256: the same layer at a prefill size (the grouped MFMA kernels).
     `xdt` = "f32": hidden rows and the intermediate in f32 (the reference's
-    operand types; hi/lo row pairs on the grouped MFMA kernels)."""
+    operand types; the grouped block-scaled kernel)."""
     import torch
     import rlxq
 
@@ -818,8 +821,8 @@ def moe_section(ctx, gen, sptr, stream, scheme: str = "q4_1", tokens: int = 16, 
         out["launches_per_layer"] = ("route, gate|up + SwiGLU (routing in the workgroups), down and combine in one "
                                      "token-major launch")
     else:
-        out["launches_per_layer"] = ("route, then per grouped call: routing table, gathered-row layout, f16 rows, "
-                                     "grouped MFMA kernel (+ combine kernel for down)")
+        out["launches_per_layer"] = ("route, then per grouped call: gathered-row layout, f16 rows, grouped MFMA "
+                                     "kernel (+ combine kernel for down)")
         out["TFLOPs"] = round(2.0 * T * TOPK * (2 * I * H + H * I) / us / 1e6, 1)
     return out
 
@@ -889,6 +892,11 @@ def q8_section(ctx, gen, sptr, stream) -> dict:
         out[label] = {"kernel": kern, "us": round(us, 3), "GBps": round(b / us / 1e3, 1),
                       "us_eager": t["us_eager"], "us_graph": t["us_graph"]}
     return out
+
+
+def microseconds(section: dict) -> dict:
+    """A section's entries reduced to their us (entries without one stay)."""
+    return {k: (v["us"] if "us" in v else microseconds(v)) if isinstance(v, dict) else v for k, v in section.items()}
 
 
 def main() -> int:
@@ -1052,13 +1060,13 @@ def main() -> int:
                                    "traffic": measured_traffic(out["prefill"]["kernel"]),
                                    "traffic_note": "HBM bytes per launch (mean of the gate_up and down launches) "
                                                    "from the committed FETCH_SIZE / WRITE_SIZE counters"}
-        out["prefill_detail"] = detail
-        out["batched_decode"] = batched_section(ctx, gen, sptr, stream)
+        out["prefill_detail"] = microseconds(detail)
+        out["batched_decode"] = microseconds(batched_section(ctx, gen, sptr, stream))
         out["moe"] = moe_section(ctx, gen, sptr, stream)
         out["moe_q4_k"] = moe_section(ctx, gen, sptr, stream, "q4_k")
         out["moe_prefill"] = moe_section(ctx, gen, sptr, stream, "q4_1", 256)
         out["moe_prefill_f32"] = moe_section(ctx, gen, sptr, stream, "q4_1", 256, "f32")
-        out["schemes"] = schemes_section(ctx, gen, sptr, stream)
+        out["schemes"] = microseconds(schemes_section(ctx, gen, sptr, stream))
         out["q8_gemv"] = q8_section(ctx, gen, sptr, stream)
         out["gguf_upload"] = gguf_section(ctx, gen, sptr, stream)
     if not a.no_cpu:
