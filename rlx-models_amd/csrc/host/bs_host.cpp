@@ -38,15 +38,13 @@ double bs_unit_factor(int scheme) {
     default: return 1.0;
   }
 }
-constexpr int kNh = 2;   // parts of an f32 row: f16 hi and lo
-
 // Scratch of one pass over `rows` rows: fragments, row factors, block sums,
 // K-split partial sums.
 struct BsBytes {
   size_t x, s, sum, part;
   BsBytes(int64_t rows, int RT, int64_t n, int64_t nu, int64_t splits) {
     const int64_t t = (rows + 32 * RT - 1) / (32 * RT) * RT;   // 32-row tiles
-    x = round256((size_t)(16 * nu * t * kNh) * 1024);
+    x = round256((size_t)(32 * nu * t) * 1024);   // (f16 hi and lo)
     s = round256((size_t)t * 128);
     sum = round256((size_t)(nu * t) * 1024);
     part = splits > 1 ? round256((size_t)(splits * rows * n) * 4) : 0;
@@ -147,7 +145,7 @@ int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream) {
 
 namespace {
 // One pass: preparation, matmul, reduction.
-int bs_pass(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m, int64_t k,
+int bs_pass(rlxq_ctx* ctx, int scheme, const float* x, const void* w, int64_t rb, int64_t m, int64_t k,
             int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, int RT, int64_t splits, int64_t uslice,
             const char* name) {
   const int64_t nu = (k + 255) / 256, tiles_m = (m + 32 * RT - 1) / (32 * RT), tiles_n = (n + 127) / 128;
@@ -167,10 +165,8 @@ int bs_pass(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w
   p.M = m;
   p.K = k;
   p.rtiles = (int32_t)rtiles;
-  p.nh = kNh;
   p.kb8 = (int32_t)(8 * nu);
   p.order = bs_order(scheme);
-  p.x_bf16 = x_dtype == RLXQ_BF16;
   p.rdiv = 1;
   if ((rc = bs_prep(ctx, p, stream))) return rc;
   hipFunction_t fn;
@@ -220,7 +216,7 @@ int bs_pass(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w
 }
 }  // namespace
 
-int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
+int bs_dispatch(rlxq_ctx* ctx, int scheme, const float* x, const void* w, int64_t rb, int64_t m,
                 int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, bool prefill,
                 size_t counted) {
   const int64_t cus = ctx->cu_count > 0 ? ctx->cu_count : 256;
@@ -294,7 +290,7 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
       }
       // (at prefill one does: 32 rows take half of what 64, the fewest, count)
       if (lo > 0) pass = lo * 32 * RT;
-      else if (!prefill) return skinny_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb);
+      else if (!prefill) return skinny_dispatch(ctx, scheme, x, RLXQ_F32, w, rb, m, k, n, y, y_dtype, stream, sb);
     }
   }
   char name[64];
@@ -302,8 +298,7 @@ int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const voi
   else std::snprintf(name, sizeof name, "rlxq_bs_%s_rt%d", scheme_name(scheme), RT);
   int rc = RLXQ_OK;
   for (int64_t r0 = 0; r0 < m && !rc; r0 += pass)
-    rc = bs_pass(ctx, scheme, static_cast<const char*>(x) + r0 * k * (x_dtype == RLXQ_BF16 ? 2 : 4), x_dtype, w, rb,
-                 std::min(pass, m - r0), k, n, static_cast<char*>(y) + r0 * n * (y_dtype == RLXQ_BF16 ? 2 : 4), y_dtype,
+    rc = bs_pass(ctx, scheme, x + r0 * k, w, rb, std::min(pass, m - r0), k, n, static_cast<char*>(y) + r0 * n * (y_dtype == RLXQ_BF16 ? 2 : 4), y_dtype,
                  stream, sb, RT, splits, uslice, name);
   return rc;
 }

@@ -210,7 +210,7 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
     void* xargs[] = {&ga};
     return launch(ctx, fx, dim3((unsigned)grid), dim3(64 * top_k), (size_t)top_k * tc * 4, stream, xargs, name);
   }
-  const size_t table_bytes = fused ? 0 : ((size_t)(2 + 2 * num_experts + n_entries) * 4 + 255) & ~size_t(255);
+  const size_t table_bytes = fused || sk ? 0 : ((size_t)(2 + 2 * num_experts + n_entries) * 4 + 255) & ~size_t(255);
   const size_t tmp_bytes = combine ? (((size_t)n_entries * width * 4 + 255) & ~size_t(255)) : 0;
   // grouped MFMA path: chunks of RPC gathered rows, each expert's entries
   // padded to whole chunks
@@ -264,7 +264,7 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
   const size_t total_ws = table_bytes + tmp_bytes + cmap_bytes + emap_bytes + x16_bytes + is_bytes + sum_bytes;
   void* ws = nullptr;
   if (total_ws && (rc = workspace(ctx, total_ws, &ws, stream))) return rc;
-  int32_t* table = fused ? nullptr : static_cast<int32_t*>(ws);
+  int32_t* table = fused || sk ? nullptr : static_cast<int32_t*>(ws);
   float* tmp = combine ? reinterpret_cast<float*>(static_cast<char*>(ws) + table_bytes) : nullptr;
   char* skb = static_cast<char*>(ws) + table_bytes + tmp_bytes;
 
@@ -302,7 +302,7 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
       // kernel over (chunk, 128 columns)
       rlxq_bs_prep_args bp;
       std::memset(&bp, 0, sizeof bp);
-      bp.x = x;
+      bp.x = static_cast<const float*>(x);
       bp.x16 = reinterpret_cast<uint8_t*>(skb + cmap_bytes + emap_bytes);
       bp.inv_s = reinterpret_cast<float*>(skb + cmap_bytes + emap_bytes + x16_bytes);
       bp.ssum = reinterpret_cast<uint32_t*>(skb + cmap_bytes + emap_bytes + x16_bytes + is_bytes);
@@ -310,7 +310,6 @@ int grouped_run(rlxq_ctx* ctx, const char* what, int scheme, int group, const vo
       bp.cmap = pa.cmap;
       bp.K = k;
       bp.rtiles = (int32_t)(sk_mp / 32);
-      bp.nh = 2;
       bp.kb8 = (int32_t)(bs_nu * 8);
       bp.order = bs_order(scheme);
       bp.rdiv = x_div;

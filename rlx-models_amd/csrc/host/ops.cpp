@@ -251,7 +251,7 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
     sb.sb_bf16 = sb_code(sb_dtype);
     const size_t counted = prep_x16_bytes(m, k, false, 0, 2) +
                            (splits > 1 ? (((size_t)(splits * m * n) * 4 + 255) & ~(size_t)255) : 0);
-    return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, true, counted);
+    return bs_dispatch(ctx, scheme, static_cast<const float*>(x), w, rb, m, k, n, y, y_dtype, stream, sb, true, counted);
   }
   char name[64];
   std::snprintf(name, sizeof name, "rlxq_gemm_%s_t%d%s", scheme_name(scheme), tile, vs.c_str());
@@ -430,7 +430,7 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
         if (ctx->fixed_active &&
             (rc = skinny_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, &counted)))
           return rc;
-        return bs_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb, false, counted);
+        return bs_dispatch(ctx, scheme, static_cast<const float*>(x), w, rb, m, k, n, y, y_dtype, stream, sb, false, counted);
       }
       return skinny_dispatch(ctx, scheme, x, x_dtype, w, rb, m, k, n, y, y_dtype, stream, sb);
     }

@@ -164,7 +164,7 @@ bool bs_applies(int scheme, int64_t m, int64_t k, int64_t n, bool prefill);
 int bs_prep(rlxq_ctx* ctx, const rlxq_bs_prep_args& p, void* stream);
 int64_t bs_lds_row(int scheme);   // bytes of a weight row's unit in LDS
 int bs_order(int scheme);         // code order of its prepared activations
-int bs_dispatch(rlxq_ctx* ctx, int scheme, const void* x, int x_dtype, const void* w, int64_t rb, int64_t m,
+int bs_dispatch(rlxq_ctx* ctx, int scheme, const float* x, const void* w, int64_t rb, int64_t m,
                 int64_t k, int64_t n, void* y, int y_dtype, void* stream, const SkinnySb& sb, bool prefill,
                 size_t counted);
 int i8b_dispatch(rlxq_ctx* ctx, int group, const void* x, int x_dtype, const void* w, const void* scales,

@@ -4,27 +4,27 @@
 #define RLXQ_BS_ARGS_H
 #include <stdint.h>
 
-/* Activation preparation: x [M, K] (f32 or bf16) -> f16 MFMA fragments, each
- * row scaled by a power of two (inv_s[m] = 1 / scale).  nh parts per row: the
- * rounded row (hi) and, with nh = 2, what the rounding left over (lo).
+/* Activation preparation: f32 x [M, K] -> f16 MFMA fragments, each row scaled
+ * by a power of two (inv_s[m] = 1 / scale) in two parts: the rounded row (hi)
+ * and what the rounding left over (lo).
  * Fragment (block b of 32 elements, tile t of 32 rows, half m of the block,
- * part p) is 1 KB at (((b * rtiles + t) * 2 + m) * nh + p) * 1024: lane
+ * part p) is 1 KB at (((b * rtiles + t) * 2 + m) * 2 + p) * 1024: lane
  * 32 h + j holds positions 16m + 8h .. + 7 (code order) of row 32 t + j.
  * Blocks run to kb8 (whole units of eight), rows to 32 rtiles; what lies
  * past K and M is zero.
  * ssum: the rows' block sums as f16 hi | lo << 16, for the min / bias term:
  * block 8 C + 4 h + q of row 32 t + j at dword
- * ((C * rtiles + t) * 64 + 32 h + j) * 4 + q.  NULL: not wanted.           */
+ * ((C * rtiles + t) * 64 + 32 h + j) * 4 + q.                              */
 typedef struct rlxq_bs_prep_args {
-  const void* x;
+  const float* x;
   uint8_t* x16;
   float* inv_s;           /* [32 rtiles]                                   */
-  uint32_t* ssum;         /* [kb8 / 8][rtiles][64][4] or NULL             */
+  uint32_t* ssum;         /* [kb8 / 8][rtiles][64][4]                     */
   const int32_t* rmap;    /* row r is x row rmap[r] / rdiv, unused where
                              rmap[r] < 0; NULL: x row r                  */
   const int32_t* cmap;    /* with rmap: cmap[0] 32-row tiles are in use  */
   int64_t M, K;
-  int32_t rtiles, nh, kb8, order, x_bf16, rdiv;
+  int32_t rtiles, kb8, order, rdiv;
 } rlxq_bs_prep_args;
 
 typedef struct rlxq_bs_args {

@@ -243,12 +243,13 @@ RLXQ_DEV float bs_scale(const BsRaw<SCH>& q, const BsRow<SCH>& r) {
 
 // The contraction of 32 RT activation rows (32-row tiles rt0 ..) with the
 // wave's 32 TN weight rows (row r of them at w + roff(r)) over units [u0, u1).
-// lds: three activation slots of RT NH 4 KB, then the four waves' weight
+// lds: three activation slots of 8 RT KB, then the four waves' weight
 // regions of 32 TN LROW bytes.  Off: type of the byte offsets between the
 // wave's weight rows (32 bits while 32 rows lie within 4 GB).
-template <int SCH, int RT, int TN, int NH, class Off, class RowOff>
+template <int SCH, int RT, int TN, class Off, class RowOff>
 RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16, const uint32_t* ssum, int rtiles,
                       int rt0, int u0, int u1, f32x16_t (&acc)[RT][TN], uint8_t* lds) {
+  constexpr int NH = 2;                           // f16 hi and lo of an activation row
   constexpr int XB = RT * NH * 2;                 // fragments (1 KB) per block
   constexpr int SLOT = 2 * XB * 1024, NX = 2 * XB * 64 / 256;   // NX pieces per thread and step
   constexpr int SEG = bs_seg<SCH>(), PPR = SEG / 16, LROW = bs_lrow<SCH>(), R = 32 * TN;
@@ -455,9 +456,9 @@ RLXQ_DEV void bs_core(const rlxq_gemm_args& ga, RowOff roff, const uint8_t* x16,
       if constexpr (rt == 0 && pr + 2 < 8 * TN) bs_fetch<SCH, (pr + 2) / TN>(rp[(pr + 2) % TN], h, row[(pr + 2) % TN], raw[q]);
       const f16x8_t(&xf)[2][NH] = xa[b & 1][rt];
       T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][0], op[q][0][0], zero, 0, 0, 0);
-      if constexpr (NH == 2) T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][1], op[q][0][0], T[z], 0, 0, 0);
+      T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][1], op[q][0][0], T[z], 0, 0, 0);
       T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][0], op[q][1][0], T[z], 0, 0, 0);
-      if constexpr (NH == 2) T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][1], op[q][1][0], T[z], 0, 0, 0);
+      T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][1], op[q][1][0], T[z], 0, 0, 0);
       if constexpr (bs_nop<SCH>() == 2) {   // (the lo x lo products, ~2^-22 of a term, are skipped)
         T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[0][0], op[q][0][1], T[z], 0, 0, 0);
         T[z] = __builtin_amdgcn_mfma_f32_32x32x16_f16(xf[1][0], op[q][1][1], T[z], 0, 0, 0);
@@ -544,7 +545,7 @@ struct BsDenseRows {
 };
 
 // Dense form: workgroup = (32 RT rows, 128 TN weight rows, K split).
-template <int SCH, int RT, int TN, int NH, class Off>
+template <int SCH, int RT, int TN, class Off>
 RLXQ_DEV void bs_body(const rlxq_bs_args& a) {
   extern __shared__ __align__(16) uint8_t bs_lds[];
   const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -575,7 +576,7 @@ RLXQ_DEV void bs_body(const rlxq_bs_args& a) {
   ga.biases = a.biases;
   const BsDenseRows roff{n0, a.N, a.rb, bs_mlx<SCH>() ? a.K / a.group : 0};
   f32x16_t acc[RT][TN];
-  bs_core<SCH, RT, TN, NH, Off>(ga, roff, a.x16, a.ssum, a.rtiles, mc * RT, u0, u1, acc, bs_lds);
+  bs_core<SCH, RT, TN, Off>(ga, roff, a.x16, a.ssum, a.rtiles, mc * RT, u0, u1, acc, bs_lds);
   // C[i][j] of a 32 x 32 tile sits in lane j + 32 ((i / 4) % 2), register
   // 4 (i / 8) + i % 4.  The row factors come as vector loads and the bounds
   // and the destination are decided once per workgroup (a load and a branch
@@ -662,7 +663,7 @@ RLXQ_DEV void bs_moe_body(const rlxq_moe_sk_args& a) {
   ga.biases = a.biases;
   const BsMoeRows roff{n0, width, a.rb, bs_mlx<SCH>() ? a.K / a.group : 0, (int64_t)e * a.N};
   f32x16_t acc[1][TN];
-  bs_core<SCH, 1, TN, 2, uint32_t>(ga, roff, reinterpret_cast<const uint8_t*>(a.x16), reinterpret_cast<const uint32_t*>(a.ssum),
+  bs_core<SCH, 1, TN, uint32_t>(ga, roff, reinterpret_cast<const uint8_t*>(a.x16), reinterpret_cast<const uint32_t*>(a.ssum),
                          (int)(a.Mp / 32), chunk, 0, (int)((a.K + 255) / 256), acc, bs_lds);
   typedef int32_t i32x4_t __attribute__((ext_vector_type(4)));
   const int64_t m0 = (int64_t)chunk * 32 + 4 * h, c = n0 + j;
@@ -722,22 +723,8 @@ RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
     // 4i .. 4i + 3, 16 + 4i ..), MLX nibbles (8i, 8i + 2, .., 8i + 1, ..)
     const int64_t e0 = src * a.K + (int64_t)b * 32 + (ORD == 1 ? 4 * i : 8 * i);
     const int64_t e1 = e0 + (ORD == 1 ? 16 : 4);
-    float n[8];
-    if (a.x_bf16) {
-      const uint16_t* x = reinterpret_cast<const uint16_t*>(a.x);
-      const uint2 u0 = *reinterpret_cast<const uint2*>(x + e0), u1 = *reinterpret_cast<const uint2*>(x + e1);
-      const uint32_t w[4] = {u0.x, u0.y, u1.x, u1.y};
-#pragma unroll
-      for (int e = 0; e < 4; e++) {
-        n[2 * e] = bf16_bits_to_f32(w[e] & 0xffffu);
-        n[2 * e + 1] = bf16_bits_to_f32(w[e] >> 16);
-      }
-    } else {
-      const float* x = reinterpret_cast<const float*>(a.x);
-      const float4 f0 = *reinterpret_cast<const float4*>(x + e0), f1 = *reinterpret_cast<const float4*>(x + e1);
-      n[0] = f0.x; n[1] = f0.y; n[2] = f0.z; n[3] = f0.w;
-      n[4] = f1.x; n[5] = f1.y; n[6] = f1.z; n[7] = f1.w;
-    }
+    const float4 f0 = *reinterpret_cast<const float4*>(a.x + e0), f1 = *reinterpret_cast<const float4*>(a.x + e1);
+    const float n[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
 #pragma unroll
     for (int e = 0; e < 8; e++) v[e] = n[ORD == 2 ? (e < 4 ? 2 * e : 2 * (e - 4) + 1) : e];
   };
@@ -790,19 +777,17 @@ RLXQ_DEV void bs_prep_body(const rlxq_bs_prep_args& a) {
       const float r0 = w0 - f16_bits_to_f32(h0), r1 = w1 - f16_bits_to_f32(h1);
       const uint32_t l0 = f32_to_f16_bits(r0), l1 = f32_to_f16_bits(r1);
       lo[e] = l0 | (l1 << 16);
-      sum += a.nh == 2 ? w0 : f16_bits_to_f32(h0);
-      sum += a.nh == 2 ? w1 : f16_bits_to_f32(h1);
+      sum += w0;
+      sum += w1;
     }
     // piece i: half i / 2 of the block, lane 32 (i % 2) + j
-    uint4* dst = reinterpret_cast<uint4*>(a.x16) + ((((int64_t)b * a.rtiles + rt) * 2 + (i >> 1)) * a.nh) * 64 + 32 * (i & 1) + j;
+    uint4* dst = reinterpret_cast<uint4*>(a.x16) + ((((int64_t)b * a.rtiles + rt) * 2 + (i >> 1)) * 2) * 64 + 32 * (i & 1) + j;
     dst[0] = make_uint4(hi[0], hi[1], hi[2], hi[3]);
-    if (a.nh == 2) dst[64] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
-    if (a.ssum) {
-      // the block's four pieces are four neighbouring lanes
-      sum += __shfl_xor(sum, 1, 64);
-      sum += __shfl_xor(sum, 2, 64);
-      if (i == 0) a.ssum[(((int64_t)(b >> 3) * a.rtiles + rt) * 64 + 32 * ((b >> 2) & 1) + j) * 4 + (b & 3)] = f16_split(sum);
-    }
+    dst[64] = make_uint4(lo[0], lo[1], lo[2], lo[3]);
+    // the block's four pieces are four neighbouring lanes
+    sum += __shfl_xor(sum, 1, 64);
+    sum += __shfl_xor(sum, 2, 64);
+    if (i == 0) a.ssum[(((int64_t)(b >> 3) * a.rtiles + rt) * 64 + 32 * ((b >> 2) & 1) + j) * 4 + (b & 3)] = f16_split(sum);
   };
 #pragma unroll
   for (int q = 0; q < NP; q++)
@@ -833,7 +818,7 @@ RLXQ_BS_PREP(rlxq_bs_prep8, 8)
 // form, with SwiGLU.
 #define RLXQ_BS_INST(NAME, SCH, RT, OFF)                                                       \
   extern "C" __global__ __launch_bounds__(256, 2) void NAME(rlxq_bs_args a) {                  \
-    rlxq::bs_body<SCH, RT, 1, 2, OFF>(a);                                                      \
+    rlxq::bs_body<SCH, RT, 1, OFF>(a);                                                      \
   }
 #define RLXQ_BS_SCHEME(SNAME, SCH)                                                             \
   RLXQ_BS_INST(rlxq_bs_##SNAME##_rt1, SCH, 1, uint32_t)                                         \
