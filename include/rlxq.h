@@ -181,7 +181,7 @@ int rlxq_dequant_matmul(rlxq_ctx* ctx, int scheme, int group_size,
  * batched decode and split-K need is a static device array of
  * RLXQ_NOALLOC_SCRATCH_BYTES per GPU, held until the process ends.  A call
  * that would need more returns RLXQ_E_SCRATCH before any launch (f32 rows on
- * the block-scaled matmul count as the kernels that it replaced laid them out,
+ * the block-scaled matmul count as the kernels that it stands beside lay them out,
  * and go through the array in as many passes as they take).  Every call
  * on one GPU shares that GPU's array: calls that overlap on one GPU (other
  * streams, contexts or threads) race and must be serialised by the caller. */

@@ -77,7 +77,7 @@ size_t bs_lds_bytes(int scheme, int RT) {
 // 256-element units, and start up faster.  T: its tiles (32 rows up to 32, 64
 // past them, by 128 columns), two of which share a CU (Q8_0 and MLX 8 bit: one).
 // us here / there, Q4_1 unless named; over 20800 batched and 6100 prefill
-// shapes (K 64 to 16384, N 64 to 24576) the rule is 0.1 to 0.5% behind the
+// shapes (K 64 to 16384, N 64 to 24576) the rule is 0.1 to 0.6% behind the
 // faster of the two, this kernel alone 0.5 to 5%, prefill of Q8_0 and MLX 8 bit
 // 4 and 12%.  RLXQ_BS=0 turns it off, any other value on (bs_dispatch).
 bool bs_applies(int scheme, int64_t m, int64_t k, int64_t n, bool prefill) {

@@ -161,12 +161,14 @@ int check_weights(rlxq_ctx* ctx, const char* what, int scheme, int group, const 
 // Schemes with the exact f32-output variant of the prefill GEMM (each
 // weight's f32 value as f16 hi + lo, f16 MFMA on prepared activations):
 // every format but MXFP4, whose E8M0-scaled codes are exact in bf16 and take
-// the bf16 kernels.
+// the bf16 kernels.  (Q4_K, Q5_K, Q6_K: for bf16 rows; their f32 rows run on the
+// block-scaled matmul.)
 bool has_exact_gemm(int scheme) { return scheme != RLXQ_MLX_MXFP4; }
 
 // Prefill dequant-GEMM launch (tilings and split-K below).  f32 output or
 // f32 activations take the exact variant; f32 activations are prepared as a
-// hi and a lo f16 row per row (the epilogue adds the pair).
+// hi and a lo f16 row per row (the epilogue adds the pair), or take the
+// block-scaled matmul (bs_applies).
 int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dtype, const void* w,
                   const void* scales, const void* biases, int sb_dtype, int64_t rb, int64_t m, int64_t k, int64_t n,
                   void* y, int y_dtype, void* stream) {
@@ -324,24 +326,24 @@ int gemm_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
 // One to four rows on the matrix cores (mfgemv.hip): whole 256-element units
 // of Q4_1, Q4_K, Q8_0, Q6_K (rows of whole dwords) and MLX 4-bit (group a
 // power of two), at least eight units (one per wave).  Where it is the faster
-// kernel (us, the other one's first; 4096 -> 4096 | 4096 -> 6144 | 4096 ->
+// kernel (us, the other one's first; 2048 -> 2048 | 4096 -> 6144 | 4096 ->
 // 24576 | 12288 -> 4096):
-//   Q8_0: always (one f32 row 8.6 6.5 | 13.9 9.0 | 31.9 21.6 | 19.6 13.0,
-//   one bf16 row 7.0 6.3 | 12.0 8.9 | 25.5 21.4 | 15.7 12.7).
-//   Q6_K: f32 rows and from two bf16 rows always (one f32 row 6.9 6.9 | 10.5
-//   9.4 | 26.0 23.3 | 15.2 13.8, two 42.5 24.3 at 24576); one bf16 row with
-//   many weight rows or a long K (6.7 7.0 | 9.2 9.5 | 24.2 23.0 | 13.8 13.8,
-//   14336 -> 6144 27.4 24.4).
-//   4-bit codes, f32: from two rows (Q4_K, two rows 39.9 18.0 at 24576, 18.9
-//   12.2 at 12288); one row past the K the register kernel is good at (12288
-//   -> 4096, Q4_K 11.9 10.8, MLX 11.8 10.4, Q4_1 10.3 10.3; 8192 -> 2048,
+//   Q8_0: always (one f32 row 5.7 4.5 | 14.7 9.4 | 32.4 22.0 | 20.2 13.4,
+//   one bf16 row 5.5 4.2 | 12.5 9.0 | 25.9 21.6 | 16.3 13.2).
+//   Q6_K: f32 rows and from two bf16 rows always (one f32 row 6.5 4.7 | 10.5
+//   10.3 | 27.5 24.7 | 15.7 14.9, two 43.7 25.8 at 24576; three and four at
+//   8192 -> 8192 are the exceptions, 36.2 37.5 and 37.6 37.7); one bf16 row
+//   with many weight rows or a long K (9.7 9.7 | 25.3 24.0 | 14.1 14.2).
+//   4-bit codes, f32: from two rows (Q4_K, two rows 40.4 18.0 at 24576, 20.0
+//   12.7 at 12288); one row past the K the register kernel is good at (12288
+//   -> 4096, Q4_K 12.5 11.4, MLX 11.8 10.8, Q4_1 10.3 10.3; 8192 -> 2048,
 //   Q4_K 7.8 7.4, MLX 5.8 7.5, Q4_1 6.4 6.7).
 //   4-bit codes, bf16: where the register kernel does not hold K (Q4_1 at
-//   12288, two rows 17.8 10.8, four 18.8 13.1; Q4_K at 8192, two rows 8.7
-//   7.9), and three or four rows (MLX 7.7 6.8 | 9.5 9.2 | 23.7 17.7, Q4_K 8.3
-//   6.9 | 10.4 9.3 | 24.7 18.3), Q4_1 only with many weight rows (7.1 6.8 |
-//   8.6 9.1 | 22.5 18.4) and MLX past K = 2048 or with many (2048->2048 4.7
-//   5.3).
+//   12288, two rows 18.4 11.3, four 19.2 13.3; Q4_K at 8192, two rows 15.3
+//   13.5), and three or four rows (four: MLX 9.8 8.8 | 23.3 18.1, Q4_K 6.0 4.9
+//   | 10.7 8.8 | 24.9 18.7), Q4_1 only with many weight rows (4096 -> 6144 8.6
+//   9.1, -> 24576 22.2 18.3) and MLX past K = 2048 or with many (2048 -> 2048
+//   4.7 4.8).
 // RLXQ_GEMV_MF=0 turns it off, =1 takes it wherever it applies (tuning); the
 // other kernels' tuning variables pick those.
 bool mf_applies(int scheme, int group, bool xbf, int64_t m, int64_t k, int64_t n, int64_t rb) {
@@ -383,7 +385,8 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
   // bf16 GEMM (weights rounded to bf16, the 2e-2 prefill bar).  f32 output
   // past 256 rows, or f32 activations (the reference's operand type) from 64
   // rows with bf16 output: the exact variant (f16 hi + lo weights; f32
-  // activations as hi + lo rows).  MXFP4 with E8M0 scales and bf16
+  // activations as hi + lo rows) or, f32 activations where bs_applies has it,
+  // the block-scaled matmul.  MXFP4 with E8M0 scales and bf16
   // activations is exact on the bf16 GEMM for f32 output too; MXFP4 with f32
   // activations or bf16 scales stays on the GEMV for f32 output.
   // RLXQ_PREFILL=gemv|gemm forces one of them where both apply (tests).
@@ -392,7 +395,7 @@ int gemv_dispatch(rlxq_ctx* ctx, int scheme, int group, const void* x, int x_dty
     const bool gemm_ok = k % 64 == 0 && (xbf || has_exact_gemm(scheme));
     bool use_gemm;
     if (xbf && y_dtype == RLXQ_BF16) use_gemm = m >= 64;
-    else if (y_dtype == RLXQ_BF16) use_gemm = m >= 64;                 // f32 x: exact variant
+    else if (y_dtype == RLXQ_BF16) use_gemm = m >= 64;                 // f32 x: exact variant or block-scaled
     else use_gemm = m > 256 && (has_exact_gemm(scheme) || mx_exact_bf16);
     use_gemm = use_gemm && gemm_ok;
     if (const char* e = std::getenv("RLXQ_PREFILL")) {

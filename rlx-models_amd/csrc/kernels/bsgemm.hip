@@ -1,6 +1,7 @@
 // Block-scaled MFMA matmul for f32 activations over packed weights:
-// y[m, n] = sum_k x[m, k] * dequant(W)[n, k], from a few rows to prefill sizes.
-// Replaces the backend kernel of Op::DequantMatMul on the reference's operand
+// y[m, n] = sum_k x[m, k] * dequant(W)[n, k], from 17 rows to prefill sizes, and
+// the expert ops' gathered rows.
+// Serves Op::DequantMatMul and Op::DequantGroupedMatMul on the reference's operand
 // types (F32 x and y, crates/rlx-models-core/src/standard_decoder.rs:727-738,
 // 12421-12433).
 //

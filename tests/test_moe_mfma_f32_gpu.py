@@ -6,7 +6,9 @@ K-quant (Q5_K, Q3_K, Q2_K, Q8_K beside Q4_K and Q6_K).
 F32 activations run as a hi and a lo f16 row per gathered row (hi = f16(s*x),
 lo = f16(s*x - hi), ~22 significant bits): a chunk of 16 MT x16 rows holds
 8 MT entries, and the epilogue adds each pair's sums (a lane's registers 0 + 1
-and 2 + 3) before the row scale, the SwiGLU and the store.  Bars: max|got -
+and 2 + 3) before the row scale, the SwiGLU and the store.  (Where no kernel is
+asked for, large calls of some formats take the block-scaled kernel:
+test_bs_grouped_gpu.py.)  Bars: max|got -
 want| / max|want| <= 1e-3 against the float64 oracle on the f32 activations
 themselves; 2e-5 where the weights are exact in f16 (Q4_1 with d = 2^-6,
 m = 0), which bf16 or f16 activations alone miss by an order of magnitude,
