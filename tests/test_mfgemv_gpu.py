@@ -21,11 +21,11 @@ pytestmark = pytest.mark.gpu
 SCHEMES = [Q8_0, Q4_1, MLX4, Q4_K, Q6_K]
 
 
-def _check(ctx, orc, scheme, m, k, n, bf16, y_dtype=None, change=None):
+def _check(ctx, orc, scheme, m, k, n, bf16, y_dtype=None, change=None, group=None, slab="f32"):
     import torch
 
     rng = np.random.default_rng(m * 11 + k + n * 5 + scheme)
-    w, sc, bi, group, wd = _case(orc, scheme, rng, n, k)
+    w, sc, bi, group, wd = _case(orc, scheme, rng, n, k, group, slab)
     x = rng.standard_normal((m, k)).astype(np.float32)
     x[0] *= 1e-6
     x[m // 2] *= 3e4
@@ -102,6 +102,18 @@ def test_large_elements_on_zero_weights(ctx, orc, monkeypatch, scheme, bf16):
     for m in (1, 2, 4):
         announce(f"matrix-core decode, large elements on zero weights {NAMES[scheme]} m={m} bf16={bf16}")
         kern = _check(ctx, orc, scheme, m, k, n, bf16, change=change)
+        assert "_mf" in kern, kern
+
+
+@pytest.mark.parametrize("group", [32, 64, 128])
+@pytest.mark.parametrize("slab", ["f32", "bf16"])
+@pytest.mark.parametrize("bf16", [False, True], ids=["f32", "bf16"])
+def test_mlx_groups_and_slabs(ctx, orc, monkeypatch, group, slab, bf16):
+    """A lane's two blocks under one scale and bias or two, from either slab."""
+    monkeypatch.setenv("RLXQ_GEMV_MF", "1")
+    for m, k, n in ((1, 2048, 17), (2, 4608, 61), (4, 4608, 17)):
+        announce(f"matrix-core decode mlx4 group={group} slab={slab} m={m} k={k} n={n} bf16={bf16}")
+        kern = _check(ctx, orc, MLX4, m, k, n, bf16, group=group, slab=slab)
         assert "_mf" in kern, kern
 
 
